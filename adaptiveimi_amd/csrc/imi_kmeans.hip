@@ -12,16 +12,15 @@
 // k up to kIvfMaxK, kmeans++ with seed 42.
 //
 // Work layout: every kernel covers all H*P (head, subspace) segments at once.
-// E-step (k <= 128): distances are screened on the matrix cores (bf16 MFMA
-// with the centroids split into hi + lo bf16 parts, under a proven rounding
-// bound) and only the centroids that can still win get the exact reference
-// distance; k > 128 uses the exact distance to every centroid.  Both emit
-// the block histogram of labels and each token's stable rank inside its
-// block, so the M-step's member lists come from one scan + one scatter.  The
-// M-step sums each cluster sequentially in ascending token order (the
-// reference's order with one thread per subspace run): one workgroup per
-// cluster, one wave running the chains while three waves stream the member
-// rows through register rings and an LDS hand-off.
+// E-step: distances are screened on the matrix cores (bf16 MFMA with the
+// centroids split into hi + lo bf16 parts, under a proven rounding bound) and
+// only the centroids that can still win get the exact reference distance.
+// The member lists come from a stable counting sort per superblock of tokens;
+// the M-step finds its members through every superblock's label offsets and
+// sums each cluster sequentially in ascending token order (the reference's
+// order with one thread per subspace run): one workgroup per cluster, one wave
+// running the chains while three waves stream the member rows through
+// register rings and an LDS hand-off.
 #include <limits>
 #include <random>
 #include <vector>
@@ -40,37 +39,58 @@ struct KmParams {
     float* cent;       // [seg][kmax][DP]
     int32_t* labels;   // [seg][T]
     float* mind;       // [seg][T] or null
-    int32_t* hist;     // [seg][kmax][nblk] or null
-    int32_t* rank;     // [seg][T]
-    float* ipart;      // [seg][nblk]
-    int32_t* sorted;   // [seg][T]
-    int32_t* off;      // [seg][kmax + 1]
-    int32_t* empties;  // [seg][kmax]
-    float* prev;       // [seg]
+    float* wpart;      // [seg][4 nblk] inertia per 64 tokens, or null
+    int32_t* sorted;   // [seg][T] member lists, superblock by superblock
+    // [seg][nsb][kmax + 1] each superblock's first place of every label, then
+    // its token count
+    int32_t* loff;
+    int32_t* empties;  // [seg][kmax] ordinal of an empty cluster, -1 otherwise
+    float* prev;       // [seg][2] inertia of the last tested iteration
     int32_t* done;     // [seg] or null
     int32_t* iters;    // [seg] or null
     void* ppstats;     // kmeans++ block statistics [seg][T / kPpRows] (init_mode 2)
-    int nblk;
+    int nblk;          // 256-token blocks
     int max_iters;
     float tol;
     int es_min;
     float es_rel;
     int exact;         // the E-step's distances are read (min distances or the early-stop inertia)
-    // Block member lists (no km_scan / km_scatter pass): the E-step writes each
-    // block's tokens in label order to `rank` ([seg][T], position blk * 256 +
-    // the token's place in its block) and the block's row of label offsets to
-    // loff ([seg][nblk][kmax + 1]: first place of each label, then the
-    // block's token count); the M-step finds its members from its label's
-    // pair of offsets in every row.  Null: the scanned member lists.
-    int32_t* loff;
+    int sbt;           // tokens per superblock of the member lists
+    int nsb;           // superblocks per segment (at most kMaxSuper)
+    float* ppmd;       // kmeans++: the second minima buffer [seg][T] (init_mode 2)
 };
+
+// The same distance with both rows read eight dims at a time (few registers).
+template <int DP>
+__device__ __forceinline__ float l2_lanes8_rolled(const uint16_t* x, const float* cr) {
+    float acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+#pragma unroll 2
+    for (int i = 0; i < DP; i += 8) {
+        const float4 c0 = *reinterpret_cast<const float4*>(cr + i);
+        const float4 c1 = *reinterpret_cast<const float4*>(cr + i + 4);
+        const uint4 v = *reinterpret_cast<const uint4*>(x + i);
+        const float cv[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float d = (j & 1 ? bf16_hi(w[j / 2]) : bf16_lo(w[j / 2])) - cv[j];
+            acc[j] = __builtin_fmaf(d, d, acc[j]);
+        }
+    }
+    float t = acc[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) t = t + acc[j];
+    return t;
+}
 
 struct Draws {
     int32_t v[256];  // uniform draws for the empty clusters of one iteration
 };
 
 constexpr int kDraws = 256;      // empty-cluster draws one launch carries
-constexpr int kLocalMaxBlk = 512;   // blocks (T <= 131072) of the block member lists
+constexpr int kMaxSuper = 512;   // superblocks of the member lists
 constexpr int kIvfMaxK = 4096;   // IVF clusters per head
 
 __host__ __device__ inline int bits_for(int n) {
@@ -88,37 +108,10 @@ __global__ __launch_bounds__(64) void km_init_first_kernel(KmParams a) {
             bf16_to_f32(a.keys[h * a.hs + static_cast<int64_t>(c) * a.ts + p * a.DP + d]);
 }
 
-// Reference distance between the register-resident subvector x and centroid
-// row cr (LDS): lane j accumulates dims j, j+8, ... with fused multiply-add,
-// then the eight lane sums are added left to right.
-template <int DP>
-__device__ __forceinline__ float l2_lanes8(const float (&x)[DP], const float* cr) {
-    float acc[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < DP; i += 8) {
-        const float4 c0 = *reinterpret_cast<const float4*>(cr + i);
-        const float4 c1 = *reinterpret_cast<const float4*>(cr + i + 4);
-        float d;
-        d = x[i + 0] - c0.x; acc[0] = __builtin_fmaf(d, d, acc[0]);
-        d = x[i + 1] - c0.y; acc[1] = __builtin_fmaf(d, d, acc[1]);
-        d = x[i + 2] - c0.z; acc[2] = __builtin_fmaf(d, d, acc[2]);
-        d = x[i + 3] - c0.w; acc[3] = __builtin_fmaf(d, d, acc[3]);
-        d = x[i + 4] - c1.x; acc[4] = __builtin_fmaf(d, d, acc[4]);
-        d = x[i + 5] - c1.y; acc[5] = __builtin_fmaf(d, d, acc[5]);
-        d = x[i + 6] - c1.z; acc[6] = __builtin_fmaf(d, d, acc[6]);
-        d = x[i + 7] - c1.w; acc[7] = __builtin_fmaf(d, d, acc[7]);
-    }
-    float t = acc[0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) t = t + acc[j];
-    return t;
-}
-
-// The same distance with the row still in its bf16 load registers (each
-// 16-byte part holds dims i .. i+7 of lanes 0..7): no float copy of the row,
-// for kernels that keep many rows in flight.
+// Reference distance between a row in its bf16 load registers (each 16-byte
+// part holds dims i .. i+7 of lanes 0..7) and the fp32 row cr: lane j
+// accumulates dims j, j+8, ... with fused multiply-add, then the eight lane
+// sums are added left to right.
 template <int DP, typename V>
 __device__ __forceinline__ float l2_lanes8_bf16(const V (&v)[DP / 8], const float* cr) {
     float acc[8];
@@ -144,160 +137,54 @@ __device__ __forceinline__ float l2_lanes8_bf16(const V (&v)[DP / 8], const floa
     return t;
 }
 
-// E-step over one block of 256 tokens of one segment.
-template <int DP>
-__global__ __launch_bounds__(256) void km_assign_kernel(KmParams a) {
-    extern __shared__ float smem[];
-    const int seg = blockIdx.y, blk = blockIdx.x;
-    if (a.done && a.done[seg]) return;
-    const int h = seg / a.P, p = seg % a.P;
-    const int k = a.k[p];
-    const int tid = threadIdx.x;
-    float* cs = smem;                                   // [k][DP]
-    int* wcnt = reinterpret_cast<int*>(smem + a.kmax * DP);  // [4][kmax]
-    float* red = reinterpret_cast<float*>(wcnt + 4 * a.kmax);  // [4]
-
-    const float* cg = a.cent + static_cast<int64_t>(seg) * a.kmax * DP;
-    for (int i = tid; i < k * DP; i += 256) cs[i] = cg[i];
-
-    const int t = blk * 256 + tid;
-    const bool valid = t < a.T;
-    float x[DP];
-    if (valid) {
-        const uint4* src = reinterpret_cast<const uint4*>(a.keys + h * a.hs + static_cast<int64_t>(t) * a.ts + p * DP);
-#pragma unroll
-        for (int i = 0; i < DP / 8; ++i) {
-            const uint4 v = src[i];
-            x[8 * i + 0] = bf16_lo(v.x); x[8 * i + 1] = bf16_hi(v.x);
-            x[8 * i + 2] = bf16_lo(v.y); x[8 * i + 3] = bf16_hi(v.y);
-            x[8 * i + 4] = bf16_lo(v.z); x[8 * i + 5] = bf16_hi(v.z);
-            x[8 * i + 6] = bf16_lo(v.w); x[8 * i + 7] = bf16_hi(v.w);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < DP; ++i) x[i] = 0.0f;
-    }
-    __syncthreads();
-
-    float best = 3.402823466e38f;  // FLT_MAX
-    int arg = 0;
-    for (int c = 0; c < k; ++c) {
-        const float dist = l2_lanes8<DP>(x, cs + c * DP);
-        if (dist < best) {
-            best = dist;
-            arg = c;
-        }
-    }
-    if (valid) {
-        a.labels[static_cast<int64_t>(seg) * a.T + t] = arg;
-        if (a.mind) a.mind[static_cast<int64_t>(seg) * a.T + t] = best;
-    }
-    if (a.hist == nullptr) return;
-
-    // inertia partial of this block (fixed reduction order)
-    float part = wave_sum(valid ? best : 0.0f);
-    if (lane_id() == 0) red[tid >> 6] = part;
-    const int r = block_digit_rank(arg, valid, k, bits_for(k), wcnt,
-                                   a.hist + static_cast<int64_t>(seg) * a.kmax * a.nblk, a.nblk, blk);
-    if (valid) a.rank[static_cast<int64_t>(seg) * a.T + t] = r;
-    if (tid == 0) a.ipart[static_cast<int64_t>(seg) * a.nblk + blk] = ((red[0] + red[1]) + red[2]) + red[3];
-}
-
-// E-step of the IVF index (Dp = 128, k up to kIvfMaxK): the centroids pass
-// through LDS in tiles of kTileC rows; the exact reference distance to every
-// centroid, c ascending, strict '<'.  Outputs as km_assign_kernel.
-constexpr int kTileC = 64;
-
-template <int DP>
-size_t tiled_lds_bytes(int kmax) {
-    return static_cast<size_t>(kTileC) * DP * sizeof(float) + 4 * static_cast<size_t>(kmax) * sizeof(int) + 64;
-}
-
-template <int DP>
-__global__ __launch_bounds__(256) void km_assign_tiled_kernel(KmParams a) {
-    extern __shared__ float smem[];
-    const int seg = blockIdx.y, blk = blockIdx.x;
-    if (a.done && a.done[seg]) return;
-    const int h = seg / a.P, p = seg % a.P;
-    const int k = a.k[p];
-    const int tid = threadIdx.x;
-    float* cs = smem;                                              // [kTileC][DP]
-    int* wcnt = reinterpret_cast<int*>(smem + kTileC * DP);        // [4][kmax]
-    float* red = reinterpret_cast<float*>(wcnt + 4 * a.kmax);      // [4]
-    const float4* cg = reinterpret_cast<const float4*>(a.cent + static_cast<int64_t>(seg) * a.kmax * DP);
-
-    const int t = blk * 256 + tid;
-    const bool valid = t < a.T;
-    float x[DP];
-    {
-        // past the end: row T - 1 again (a valid row; its label is not stored)
-        const uint4* src = reinterpret_cast<const uint4*>(a.keys + h * a.hs +
-                                                          static_cast<int64_t>(valid ? t : a.T - 1) * a.ts + p * DP);
-#pragma unroll
-        for (int i = 0; i < DP / 8; ++i) {
-            const uint4 v = src[i];
-            x[8 * i + 0] = bf16_lo(v.x); x[8 * i + 1] = bf16_hi(v.x);
-            x[8 * i + 2] = bf16_lo(v.y); x[8 * i + 3] = bf16_hi(v.y);
-            x[8 * i + 4] = bf16_lo(v.z); x[8 * i + 5] = bf16_hi(v.z);
-            x[8 * i + 6] = bf16_lo(v.w); x[8 * i + 7] = bf16_hi(v.w);
-        }
-    }
-    float best = 3.402823466e38f;  // FLT_MAX
-    int arg = 0;
-    for (int c0 = 0; c0 < k; c0 += kTileC) {
-        const int nc = min(kTileC, k - c0);
-        __syncthreads();   // the previous tile is read
-        for (int i = tid; i < nc * (DP / 4); i += 256)
-            reinterpret_cast<float4*>(cs)[i] = cg[static_cast<int64_t>(c0) * (DP / 4) + i];
-        __syncthreads();
-#pragma unroll 1
-        for (int c = 0; c < nc; ++c) {
-            const float dist = l2_lanes8<DP>(x, cs + c * DP);
-            if (dist < best) {
-                best = dist;
-                arg = c0 + c;
-            }
-        }
-    }
-    if (valid) {
-        a.labels[static_cast<int64_t>(seg) * a.T + t] = arg;
-        if (a.mind) a.mind[static_cast<int64_t>(seg) * a.T + t] = best;
-    }
-    if (a.hist == nullptr) return;
-    float part = wave_sum(valid ? best : 0.0f);
-    if (lane_id() == 0) red[tid >> 6] = part;
-    const int r = block_digit_rank(arg, valid, k, bits_for(k), wcnt,
-                                   a.hist + static_cast<int64_t>(seg) * a.kmax * a.nblk, a.nblk, blk);
-    if (valid) a.rank[static_cast<int64_t>(seg) * a.T + t] = r;
-    if (tid == 0) a.ipart[static_cast<int64_t>(seg) * a.nblk + blk] = ((red[0] + red[1]) + red[2]) + red[3];
-}
-
-// E-step with matrix-core screening (k <= 128).  For token x and centroid
-// c the distance is approximated as D~ = |x|^2 + |c|^2 - 2 x.c, with x.c on
-// v_mfma_f32_16x16x32_bf16: x is bf16 already and c enters as two bf16
-// parts (hi = bf16(c), lo = bf16(c - hi), |c - hi - lo| <= 2^-16 |c|).
-// Rounding analysis (unit roundoff u = 2^-24, at most ~256 accumulations
-// per dot product, reference distance = 8 FMA chains + 7 adds):
-//   |D~ - D_ref| <= 2^-14.6 (|x|^2 + |c|^2) <= E = 2^-12 (|x|^2 + max|c|^2)
-// (4x margin, plus 1e-30 for flushed subnormal products).  Any centroid
-// that can win under the reference order satisfies D~(c) <= min D~ + 2E, so
-// only those candidates get the exact reference distance (l2_lanes8, c
-// ascending, strict '<'); usually there is one.  Non-finite or huge values
-// (|x|^2 + max|c|^2 > 1e37) make every centroid a candidate, which is the
-// plain exact E-step.  Outputs (labels, min distances, block ranks, label
-// histogram, inertia partials) are those of km_assign_kernel.
+// ------------------------------------------------------------------ E-step
+// Matrix-core screening for any k.  For token x and centroid c the value
+//   f(c) = x.c - |c|^2 / 2 = (|x|^2 - D(x, c)) / 2
+// orders the centroids like the distance (largest f first).  x.c runs on
+// v_mfma_f32_16x16x32_bf16: x is bf16 already and c enters as two bf16 parts
+// (hi = bf16(c), lo = bf16(c - hi), |c - hi - lo| <= 2^-16 |c|); the
+// accumulators start at -|c|^2 / 2.  Rounding analysis with mag = |x|^2 +
+// max|c|^2, every partial sum of f bounded by |x||c| + |c|^2 / 2 <= mag: at
+// most 256 accumulations of at most 2^-23 each (2^-15, also if the matrix
+// core truncates), the split of c (2^-18 |x||c|) and the norm's chain
+// (2^-17 |c|^2) stay below 2^-14.6 mag, and the reference's own distance (8 FMA
+// chains + 7 adds) adds less than 2^-18.  So the reference's winner satisfies
+// f >= max f - 2^-13.5 mag - 1e-30 (the last term for flushed subnormals).
+//
+// Each lane keeps the three largest f of its token (a max and two med3 per
+// value), each value carrying its centroid's number in its lowest bits, which
+// moves a value by less than 2^(bits - 23) mag; for IVF the number inside its
+// chunk of 64, the chunk beside it.  With E = (2^-13 + 2^(bits - 22)) mag + 1e-30:
+//   second < best - E   the best is the reference's label;
+//   third < best - E    best and second get the exact reference distance
+//                       (l2 in 8 lanes, strict '<' over ascending c);
+//   otherwise, for non-finite or huge magnitudes (mag > 1e37), and for equal
+//   best and second values (their chunks cannot be told apart), every
+//   centroid does.
+// With k-means centroids over the benchmark's keys 0.5-1 % of the tokens take
+// the second form and 0.01 % the third (k = 32..1018).  Outputs (labels, min
+// distances, inertia partials) are those of the exhaustive loop.
+//
+// A wave owns 64 tokens (four 16-token tiles) and shares nothing with the
+// other waves but the packed centroids, so the loop over its token blocks has
+// no barrier and the waves' loads, matrix work and re-checks overlap; each
+// block's tokens are loaded while the one before is re-checked.  The
+// centroids are packed into LDS in the matrix-core operand layout by the
+// workgroup: all of them at once for subspaces (4 DP bytes each), in double-
+// buffered chunks of 64 for IVF (STREAM).
+//
+// Bound by: reading the keys up to k = 64 (64 x 64, 128k tokens, 8 heads: 268
+// MB in 59 us, 4.5 TB/s; a barrier-synchronised form with the label ranks in
+// it took 85 us), the three VALU operations and the and-or per value beside
+// the matrix work beyond (k = 181, 512k tokens: 515 us; 4.65 ms as fp32
+// distances to every centroid; IVF, k = 1018, 16k tokens, 8 heads: 106 us,
+// 1.02 ms as such).
 typedef __attribute__((ext_vector_type(8))) __bf16 km_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float km_f32x4_t;
 typedef __attribute__((ext_vector_type(4))) unsigned int km_u32x4_t;
 typedef __attribute__((ext_vector_type(2))) unsigned int km_u32x2_t;
 typedef __attribute__((ext_vector_type(4))) short km_s16x4_t;
 typedef __attribute__((address_space(3))) km_s16x4_t km_lds_s16x4_t;
-
-constexpr int kScreenMaxK = 128;
-constexpr int kScreenQueue = 64;   // queued exact passes per 256-token block
-
-__device__ __forceinline__ uint32_t xor16_u(uint32_t v) { return __float_as_uint(xor16(__uint_as_float(v))); }
-__device__ __forceinline__ uint32_t xor32_u(uint32_t v) { return __float_as_uint(xor32(__uint_as_float(v))); }
 
 // Intra-wave LDS hand-off (compiler ordering only; a wave's LDS instructions
 // execute in order).
@@ -307,14 +194,12 @@ __device__ __forceinline__ void km_wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int DP>
-size_t screen_lds_bytes(int kmax) {
-    constexpr int KH = DP / 32;
-    const size_t nct = (kmax + 15) / 16;
-    return static_cast<size_t>(kmax) * (DP + 4) * 4 + nct * KH * 2 * 64 * 16 + nct * 16 * 4 + 256 * 2 * 8 +
-           kScreenQueue * 8 + 4 * static_cast<size_t>(kmax) * 4 + 16 + (kScreenQueue + 1) * 4 +
-           (kScreenQueue + 1) * 4;
-}
+constexpr float kFltMax = 3.402823466e38f;
+constexpr int kChunkTiles = 4;   // 16-centroid tiles per streamed chunk
+
+// Distances the E-step has to produce: none (labels only), exact ones with
+// the fp32 centroid rows in LDS, or with the rows in global memory.
+enum KmExact { kLabelsOnly = 0, kExactLds = 1, kExactGlobal = 2 };
 
 // Row shift left by K inside a row of 16 lanes: lane i gets lane i + K's value.
 template <int K>
@@ -322,368 +207,467 @@ __device__ __forceinline__ float dpp_row_shl(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + K, 0xF, 0xF, false));
 }
 
-// KT > 0: every segment has k = 16 KT centroids (whole tiles, no per-tile
-// tests); KT = 0: any k <= MAXK.
-template <int DP, int MAXK, int KT, bool EXACT>
-__global__ __launch_bounds__(256, 4) void km_assign_screen_kernel(KmParams a, int chunks) {
+// Two fp32 values rounded to bf16 (nearest even), packed (v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    typedef __attribute__((ext_vector_type(2))) float f2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, b2));
+}
+
+// max without the operand canonicalisation fmaxf costs (one more VALU
+// operation per screened value); no operand is a signalling NaN that matters:
+// NaN magnitudes send the token through every centroid.
+__device__ __forceinline__ float max_raw(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// One lane's share of a 16-centroid tile: dims 32 kh + 8 (lane / 16) .. + 7 of
+// centroid 16 ct + lane % 16 as hi and lo bf16 operands; sq += the dims' squares.
+__device__ __forceinline__ void pack_centroid(const float4 v0, const float4 v1, km_u32x4_t& hi, km_u32x4_t& lo,
+                                              float& sq) {
+    const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t h = pack_bf16(v[2 * i], v[2 * i + 1]);
+        hi[i] = h;
+        lo[i] = pack_bf16(v[2 * i] - bf16_lo(h), v[2 * i + 1] - bf16_hi(h));
+        sq = __builtin_fmaf(v[2 * i], v[2 * i], sq);
+        sq = __builtin_fmaf(v[2 * i + 1], v[2 * i + 1], sq);
+    }
+}
+
+// The three largest values of a token (best >= second >= third).
+struct Top3 {
+    float b, s, t;
+    __device__ __forceinline__ void add(float v) {
+        t = __builtin_amdgcn_fmed3f(s, t, v);
+        s = __builtin_amdgcn_fmed3f(b, s, v);
+        b = max_raw(b, v);
+    }
+    __device__ __forceinline__ void merge(const Top3& o) {
+        add(o.b);
+        add(o.s);
+        add(o.t);
+    }
+};
+
+// permlane swaps of two values: after swap32 the lanes below 32 hold x of both
+// halves (x, y) and the others y of both halves; swap16 does so for the even
+// and odd rows of 16 lanes.
+__device__ __forceinline__ void swap32(float& x, float& y) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(r[0]);
+    y = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& x, float& y) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(r[0]);
+    y = __uint_as_float(r[1]);
+}
+// Three largest values with the centroids of the first two (STREAM: a value
+// carries only its number in the chunk).
+struct Top3Ids {
+    Top3 v;
+    int ib, is;
+};
+
+// Halves (or rows) exchange their tiles: the lanes that keep x's tile get y's
+// lanes' part of it, the others x's lanes' part of y's tile.
+template <bool HALF, bool IDS>
+__device__ __forceinline__ Top3Ids swap_merge(Top3Ids x, Top3Ids y) {
+    auto swap = [](float& p, float& q) {
+        if (HALF)
+            swap32(p, q);
+        else
+            swap16(p, q);
+    };
+    swap(x.v.b, y.v.b);
+    swap(x.v.s, y.v.s);
+    swap(x.v.t, y.v.t);
+    if (IDS) {
+        float xi = __int_as_float(x.ib), yi = __int_as_float(y.ib), xj = __int_as_float(x.is), yj = __int_as_float(y.is);
+        swap(xi, yi);
+        swap(xj, yj);
+        x.ib = __float_as_int(xi);
+        x.is = __float_as_int(xj);
+        y.ib = __float_as_int(yi);
+        y.is = __float_as_int(yj);
+        const bool xb = x.v.b >= y.v.b;
+        const bool keep = xb ? x.v.s >= y.v.b : y.v.s >= x.v.b;   // the winner's second stays second
+        const int ib = xb ? x.ib : y.ib;
+        x.is = xb ? (keep ? x.is : y.ib) : (keep ? y.is : x.ib);
+        x.ib = ib;
+    }
+    x.v.merge(y.v);
+    return x;
+}
+
+template <int DP>
+struct ScreenLds {
+    static constexpr int KH = DP / 32;
+    static size_t packed(int tiles) { return static_cast<size_t>(tiles) * (KH * 2 * 64 * 16 + 64); }
+    static size_t rows(int kmax) { return static_cast<size_t>(kmax) * (DP + 4) * sizeof(float); }
+};
+
+template <int DP, int NW, bool STREAM, int EXACT>
+__global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXACT ? 3 : 4)) void km_screen_kernel(KmParams a, int chunks) {
     constexpr int KH = DP / 32;   // 32-dim K steps per subvector
-    constexpr int NCT = KT > 0 ? KT : MAXK / 16;   // centroid tiles held per lane
-    extern __shared__ float smem[];
+    constexpr int CS = DP + 4;    // padded fp32 row
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int seg = blockIdx.y;
     if (a.done && a.done[seg]) return;
     const int h = seg / a.P, p = seg % a.P;
-    const int k = KT > 0 ? 16 * KT : a.k[p];
-    const int nct = KT > 0 ? KT : (k + 15) >> 4;
-    const int nct_max = (a.kmax + 15) >> 4;
+    const int k = a.k[p];
+    const int nct = (k + 15) >> 4;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    constexpr int CS = DP + 4;
-    float* cs = smem;                                                        // [kmax][DP + 4]
-    km_u32x4_t* apk = reinterpret_cast<km_u32x4_t*>(cs + a.kmax * CS);      // [nct][KH][hi,lo][64 lanes]
-    float* ccs = reinterpret_cast<float*>(apk + nct_max * KH * 2 * 64);     // [nct * 16]
-    uint64_t* cmask = reinterpret_cast<uint64_t*>(ccs + nct_max * 16);      // [256][2] candidate bits
-    uint64_t* qbest = cmask + 256 * 2;                                      // [kScreenQueue] (distance, centroid)
-    int* wcnt = reinterpret_cast<int*>(qbest + kScreenQueue);               // [4][kmax]
-    float* red = reinterpret_cast<float*>(wcnt + 4 * a.kmax);               // [4]
-    int* qtok = reinterpret_cast<int*>(red + 4);                            // [kScreenQueue] queued tokens
-    int* qcnt = qtok + kScreenQueue;                                        // queue length
-    int* qoff = qcnt + 1;                                                   // [kScreenQueue + 1] first pair
-    // the block rank's label offsets reuse the queue's slots, which are read
-    // before its first barrier ([kmax] <= 2 * kScreenQueue ints, [4])
-    int* lofs = reinterpret_cast<int*>(qbest);
-    int* lwsum = qoff;
-
+    const int grp = lane >> 4;
+    // packed tiles [tile][KH][hi, lo][64 lanes], then -|c|^2 / 2 [tile][16]
+    const int tiles = STREAM ? 2 * kChunkTiles : nct;
+    km_u32x4_t* apk = reinterpret_cast<km_u32x4_t*>(smem_raw);
+    float* cch = reinterpret_cast<float*>(apk + tiles * KH * 2 * 64);
+    float* cs = cch + tiles * 16;   // [k][CS] (kExactLds)
     const float* cg = a.cent + static_cast<int64_t>(seg) * a.kmax * DP;
-    {
-        // centroid rows -> LDS (padded rows), every float4 load issued first
-        constexpr int PER = MAXK * DP / 4 / 256;
-        float4 v[PER];
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int i4 = tid + u * 256;
-            v[u] = i4 * 4 < k * DP ? reinterpret_cast<const float4*>(cg)[i4] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        }
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int i = (tid + u * 256) * 4;
-            if (i < k * DP) *reinterpret_cast<float4*>(cs + (i / DP) * CS + i % DP) = v[u];
-        }
-    }
-    if (tid == 0) *qcnt = 0;
-    __syncthreads();
-    // A operands: lane l of tile ct holds centroid 16ct + l%16, dims
-    // 32kh + 8(l/16) .. +7 (v_mfma_f32_16x16x32_bf16 A layout)
-    for (int e = tid; e < nct * KH * 2 * 64; e += 256) {
-        const int l = e & 63, part = (e >> 6) & 1, t2 = e >> 7;
-        const int kh = t2 % KH, ct = t2 / KH;
-        const int c = ct * 16 + (l & 15);
-        const int d0 = kh * 32 + 8 * (l >> 4);
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        if (c < k) {
-#pragma unroll
-            for (int i = 0; i < 8; i += 2) {
-                const float v0 = cs[c * CS + d0 + i], v1 = cs[c * CS + d0 + i + 1];
-                uint16_t b0 = f32_to_bf16(v0), b1 = f32_to_bf16(v1);
-                if (part) {
-                    b0 = f32_to_bf16(v0 - bf16_to_f32(b0));
-                    b1 = f32_to_bf16(v1 - bf16_to_f32(b1));
-                }
-                w[i / 2] = static_cast<uint32_t>(b0) | (static_cast<uint32_t>(b1) << 16);
-            }
-        }
-        apk[e] = km_u32x4_t{w[0], w[1], w[2], w[3]};
-    }
-    for (int c = tid; c < nct * 16; c += 256) {
-        float sq = INFINITY;   // padding rows of A are zero: their e(c) is +inf
-        if (c < k) {
-            sq = 0.0f;
-#pragma unroll
-            for (int d = 0; d < DP; ++d) sq = __builtin_fmaf(cs[c * CS + d], cs[c * CS + d], sq);
-        }
-        ccs[c] = sq;
-    }
-    __syncthreads();
-    float ccmax = 0.0f;
-    for (int c = lane; c < k; c += 64) ccmax = fmaxf(ccmax, ccs[c]);
-    ccmax = wave_max(ccmax);
-    const int nwords = (nct + 1) >> 1;          // 32-bit candidate words in use
-    // |c|^2 of the lane's accumulator rows (centroid 16 ct + 4 (lane / 16) + r)
-    // in registers for up to 4 tiles, else read from LDS per use
-    constexpr bool CCREG = NCT <= 4;
-    float ccv[CCREG ? NCT : 1][4];
-#pragma unroll
-    for (int ct = 0; ct < (CCREG ? NCT : 1); ++ct)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ccv[ct][r] = ct < nct ? -0.5f * ccs[ct * 16 + 4 * (lane >> 4) + r] : -INFINITY;
-
     const uint16_t* kb = a.keys + h * a.hs + p * DP;
-    // 256-token blocks blockIdx.x * chunks .. +chunks-1 (the prologue above is
-    // shared by all of them)
-#pragma unroll 1
-    for (int ci = 0; ci < chunks; ++ci) {
-    const int blk = blockIdx.x * chunks + ci;
-    if (blk >= a.nblk) break;
-    if (ci > 0) __syncthreads();   // the previous block's LDS reads are done
-    // the MFMA operands of the wave's four 16-token tiles are loaded up front
-    // (lane l: token l%16, dims 32kh + 8(l/16) .. +7)
-    const int tw0 = blk * 256 + wave * 64;
-    const int t = blk * 256 + tid;
-    const bool valid = t < a.T;
-    // (tokens past T re-read token T - 1: the loads need no branches, and
-    // those lanes' results are never stored)
-    km_u32x4_t bqa[4][KH];
+    // bits of the centroid number a value carries (of its number in the chunk)
+    const int nbits = STREAM ? bits_for(16 * kChunkTiles) : bits_for(nct * 16);
+    const uint32_t idx_mask = ~((1u << nbits) - 1u);
+    const float e_rel = 0x1p-13f + ldexpf(1.0f, nbits - 22);
+    // the lane's rows of a 16-token tile
+    const uint16_t* lane_rows = kb + static_cast<int64_t>(lane & 15) * a.ts + 8 * grp;
+    float ccmax = 0.0f;   // of the lane's own centroids until the reduction
+
+    // tile ct -> slot: one wave packs it; padding centroids are zero rows
+    // whose f stays at -3e38
+    auto load_tile = [&](int ct, float4 (&v)[2 * KH]) {
+        const int c = min(16 * ct + (lane & 15), k - 1);
+        const float4* row = reinterpret_cast<const float4*>(cg + static_cast<int64_t>(c) * DP);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int tt = min(tw0 + 16 * j + (lane & 15), a.T - 1);
-#pragma unroll
-        for (int kh = 0; kh < KH; ++kh)
-            bqa[j][kh] = *reinterpret_cast<const km_u32x4_t*>(kb + static_cast<int64_t>(tt) * a.ts + kh * 32 +
-                                                              8 * (lane >> 4));
-    }
-    // the thread's own token row for the exact pass, loaded now as well
-    km_u32x4_t xr[EXACT ? DP / 8 : 1];
-    if constexpr (EXACT) {
-        const int tc = min(t, a.T - 1);
-#pragma unroll
-        for (int i = 0; i < DP / 8; ++i)
-            xr[i] = *reinterpret_cast<const km_u32x4_t*>(kb + static_cast<int64_t>(tc) * a.ts + 8 * i);
-    }
-    // screening: token tile j = tokens 16j .. 16j+15 of this wave's 64.
-    // f(c) = x.c - |c|^2 / 2 = -e(c) / 2 with e(c) = |c|^2 - 2 x.c, which
-    // orders the centroids like D~ = |x|^2 + e(c) (largest f first): the
-    // matrix cores start each tile's accumulator at -|c|^2 / 2 (halving is
-    // exact but for subnormals, which the absolute term of the bound covers).
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const km_u32x4_t* bq = bqa[j];
-        // |x|^2 from the diagonal of x x^T (the same registers serve as A and
-        // B): token t's entry sits in lane 16(t/4) + t, register t % 4
-        float xs;
-        {
-            km_f32x4_t dg = km_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kh = 0; kh < KH; ++kh)
-                dg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, bq[kh]),
-                                                             __builtin_bit_cast(km_bf16x8_t, bq[kh]), dg, 0, 0, 0);
-            const int tl = lane & 15, rr = tl & 3;
-            const float own = rr == 0 ? dg[0] : rr == 1 ? dg[1] : rr == 2 ? dg[2] : dg[3];
-            xs = __shfl(own, 16 * (tl >> 2) + tl);
+        for (int kh = 0; kh < KH; ++kh) {
+            v[2 * kh] = row[8 * kh + 2 * grp];
+            v[2 * kh + 1] = row[8 * kh + 2 * grp + 1];
         }
-        float ev[NCT][4];
-        float emax = -INFINITY;
+    };
+    auto store_tile = [&](int ct, int slot, float4 (&v)[2 * KH]) {
+        const bool real = 16 * ct + (lane & 15) < k;
+        float sq = 0.0f;
 #pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-            if (KT > 0 || ct < nct) {
-                km_f32x4_t acc;
+        for (int kh = 0; kh < KH; ++kh) {
+            km_u32x4_t hi, lo;
+            pack_centroid(v[2 * kh], v[2 * kh + 1], hi, lo, sq);
+            const km_u32x4_t zero = km_u32x4_t{0u, 0u, 0u, 0u};
+            apk[((slot * KH + kh) * 2 + 0) * 64 + lane] = real ? hi : zero;
+            apk[((slot * KH + kh) * 2 + 1) * 64 + lane] = real ? lo : zero;
+        }
+        sq += xor16(sq);
+        sq += xor32(sq);
+        if (real) ccmax = sq > ccmax || sq != sq ? sq : ccmax;   // a NaN norm stays
+        if (lane < 16) cch[slot * 16 + lane] = real ? -0.5f * sq : -3e38f;
+    };
+    auto reduce_ccmax = [&](float* sh) {
+        // (fmax would drop a NaN: an infinite bound stands for it)
+        float m = ccmax == ccmax ? ccmax : INFINITY;
+        m = wave_max(m);
+        if (lane == 0) sh[wave] = m;
+        __syncthreads();
+        m = sh[0];
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    acc[r] = CCREG ? ccv[CCREG ? ct : 0][r] : -0.5f * ccs[ct * 16 + 4 * (lane >> 4) + r];
+        for (int w = 1; w < NW; ++w) m = fmaxf(m, sh[w]);
+        return m;
+    };
+    const int nblk = (a.T + 64 * NW - 1) / (64 * NW);
+    const int blk0 = blockIdx.x * chunks, blk1 = min(blk0 + chunks, nblk);
+    // B operands of the wave's four 16-token tiles of block blk (lane l: token
+    // l % 16, dims 32 kh + 8 (l / 16) .. + 7); tokens past T re-read token T - 1
+    km_u32x4_t bq[4][KH];
+    auto load_tokens = [&](int blk) {
+        const int t0 = __builtin_amdgcn_readfirstlane((blk * NW + wave) * 64);
+        const uint16_t* src[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) src[j] = lane_rows + static_cast<int64_t>(t0 + 16 * j) * a.ts;
+        if (t0 + 64 > a.T) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                src[j] = kb + static_cast<int64_t>(min(t0 + 16 * j + (lane & 15), a.T - 1)) * a.ts + 8 * grp;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int kh = 0; kh < KH; ++kh) bq[j][kh] = *reinterpret_cast<const km_u32x4_t*>(src[j] + kh * 32);
+    };
+    // the first block's tokens come while the centroids are packed, each
+    // later block's while the one before is re-checked and stored
+    load_tokens(blk0);
+    __shared__ float s_cc[NW];
+    if constexpr (!STREAM) {
+        for (int ct = wave; ct < nct; ct += NW) {
+            float4 v[2 * KH];
+            load_tile(ct, v);
+            store_tile(ct, ct, v);
+        }
+        if constexpr (EXACT == kExactLds) {
+            for (int i = tid; i < k * (DP / 4); i += 64 * NW)
+                *reinterpret_cast<float4*>(cs + (i / (DP / 4)) * CS + 4 * (i % (DP / 4))) =
+                    reinterpret_cast<const float4*>(cg)[i];
+        }
+        ccmax = reduce_ccmax(s_cc);
+    }
+
+#pragma unroll 1
+    for (int blk = blk0; blk < blk1; ++blk) {
+        const int t0 = __builtin_amdgcn_readfirstlane((blk * NW + wave) * 64);
+        if (!STREAM && t0 >= a.T) break;   // (streaming waves keep to the barriers)
+        const int t = t0 + lane;
+        const bool valid = t < a.T;
+        Top3 top[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) top[j] = Top3{-INFINITY, -INFINITY, -INFINITY};
+        // centroid numbers of the lane's four accumulator rows (kept apart, so
+        // that the number enters a value with one and-or)
+        uint32_t num[4];
+        auto number_from = [&](uint32_t c) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) {
+                num[r] = c + 4 * grp + r;
+                asm("" : "+v"(num[r]));
+            }
+        };
+        number_from(0);
+        // the 16 centroids of packed slot `slot`
+        auto screen_tile = [&](int slot) {
+            km_u32x4_t ah[KH], al[KH];
+#pragma unroll
+            for (int kh = 0; kh < KH; ++kh) {
+                ah[kh] = apk[((slot * KH + kh) * 2 + 0) * 64 + lane];
+                al[kh] = apk[((slot * KH + kh) * 2 + 1) * 64 + lane];
+            }
+            const km_f32x4_t init = *reinterpret_cast<const km_f32x4_t*>(cch + slot * 16 + 4 * grp);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                km_f32x4_t acc = init;
 #pragma unroll
                 for (int kh = 0; kh < KH; ++kh) {
-                    const km_u32x4_t ah = apk[((ct * KH + kh) * 2 + 0) * 64 + lane];
-                    const km_u32x4_t al = apk[((ct * KH + kh) * 2 + 1) * 64 + lane];
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, ah),
-                                                                  __builtin_bit_cast(km_bf16x8_t, bq[kh]), acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, al),
-                                                                  __builtin_bit_cast(km_bf16x8_t, bq[kh]), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, ah[kh]),
+                                                                  __builtin_bit_cast(km_bf16x8_t, bq[j][kh]), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, al[kh]),
+                                                                  __builtin_bit_cast(km_bf16x8_t, bq[j][kh]), acc, 0, 0, 0);
                 }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    ev[ct][r] = acc[r];
-                    emax = fmaxf(emax, acc[r]);
+                for (int r = 0; r < 4; ++r)
+                    top[j].add(__uint_as_float((__float_as_uint(acc[r]) & idx_mask) | num[r]));
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) num[r] += 16;
+        };
+        int chb[4] = {0, 0, 0, 0}, chs[4] = {0, 0, 0, 0};   // chunks of best and second (STREAM)
+        if constexpr (STREAM) {
+            // chunk q in slots kChunkTiles (q % 2) ..: wave w packs its tile
+            // w of chunk q + 1 while chunk q is screened
+            static_assert(!STREAM || NW == kChunkTiles, "one tile per wave and chunk");
+            const int nch = (nct + kChunkTiles - 1) / kChunkTiles;
+            float4 v[2 * KH];
+            load_tile(wave, v);
+            __syncthreads();   // the previous block's reads are done
+            store_tile(wave, wave, v);
+            __syncthreads();
+#pragma unroll 1
+            for (int q = 0; q < nch; ++q) {
+                const int nxt = (q + 1) * kChunkTiles + wave;
+                if (q + 1 < nch) load_tile(nxt, v);
+                float pb[4], ps[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    pb[j] = top[j].b;
+                    ps[j] = top[j].s;
+                }
+                number_from(0);
+#pragma unroll 1
+                for (int i = 0; i < kChunkTiles; ++i) screen_tile((q & 1) * kChunkTiles + i);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (top[j].s != ps[j]) chs[j] = top[j].s == pb[j] ? chb[j] : q;
+                    if (top[j].b != pb[j]) chb[j] = q;
+                }
+                if (q + 1 < nch) store_tile(nxt, ((q + 1) & 1) * kChunkTiles + wave, v);
+                __syncthreads();
+            }
+            if (blk == blk0) ccmax = reduce_ccmax(s_cc);
+        } else {
+#pragma unroll 1
+            for (int ct = 0; ct < nct; ++ct) screen_tile(ct);
+        }
+        // |x|^2: each lane has its quarter of every tile's dims
+        float xs[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            xs[j] = 0.0f;
+#pragma unroll
+            for (int kh = 0; kh < KH; ++kh)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x0 = bf16_lo(bq[j][kh][i]), x1 = bf16_hi(bq[j][kh][i]);
+                    xs[j] = __builtin_fmaf(x0, x0, xs[j]);
+                    xs[j] = __builtin_fmaf(x1, x1, xs[j]);
+                }
+        }
+        // row g of the wave ends with tile g: halves exchange tiles (0, 2) and
+        // (1, 3), then rows
+        swap32(xs[0], xs[2]);
+        swap32(xs[1], xs[3]);
+        float x02 = xs[0] + xs[2], x13 = xs[1] + xs[3];
+        swap16(x02, x13);
+        const float mag = (x02 + x13) + ccmax;
+        Top3Ids own[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            own[j].v = top[j];
+            own[j].ib = 16 * kChunkTiles * chb[j] + static_cast<int>(__float_as_uint(top[j].b) & ~idx_mask);
+            own[j].is = 16 * kChunkTiles * chs[j] + static_cast<int>(__float_as_uint(top[j].s) & ~idx_mask);
+        }
+        const Top3Ids m02 = swap_merge<true, STREAM>(own[0], own[2]);
+        const Top3Ids m13 = swap_merge<true, STREAM>(own[1], own[3]);
+        const Top3Ids mi = swap_merge<false, STREAM>(m02, m13);
+        const Top3 m = mi.v;
+        const float lim = m.b - (e_rel * mag + 1e-30f);
+        const bool every = !(mag <= 1e37f) || !(m.t < lim) || m.s == m.b;
+        const bool pair = !every && !(m.s < lim);
+        const int c1 = STREAM ? mi.ib : static_cast<int>(__float_as_uint(m.b) & ~idx_mask);
+        const int c2 = STREAM ? mi.is : static_cast<int>(__float_as_uint(m.s) & ~idx_mask);
+        float best = kFltMax;
+        int arg = 0;
+        // every centroid: a few tokens spread over the lanes by centroid, or
+        // each token on its own lane
+        uint64_t full = __ballot(every && valid);
+        if (full) {
+            if (__popcll(full) > 8) {
+                if (every && valid) {
+                    const uint16_t* row = kb + static_cast<int64_t>(t) * a.ts;
+#pragma unroll 1
+                    for (int c = 0; c < k; ++c) {
+                        const float d = l2_lanes8_rolled<DP>(row, cg + static_cast<int64_t>(c) * DP);
+                        if (d < best) {
+                            best = d;
+                            arg = c;
+                        }
+                    }
+                    if (!(best < kFltMax)) arg = 0;
                 }
             } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) ev[ct][r] = -INFINITY;
-            }
-        }
-        emax = fmaxf(emax, xor16(emax));
-        emax = fmaxf(emax, xor32(emax));
-        // candidates: e(c) <= min e + 2E, i.e. f(c) >= max f - E; non-finite
-        // or huge magnitudes make every finite f a candidate (the exhaustive
-        // E-step)
-        const float mag = xs + ccmax;
-        const float lim0 = emax - (0x1p-12f * mag + 1e-30f);
-        const bool all = !(mag <= 1e37f) || !(lim0 > -INFINITY);
-        const float lim = all ? -3.402823466e38f : lim0;
-        uint32_t m[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) {
-            uint32_t nib = 0u;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) nib |= ev[ct][r] >= lim ? (1u << r) : 0u;
-            if (all) {
-                // every real centroid: past 1e37 the screen's products and
-                // norms can overflow to inf or NaN where a distance does not
-                const int c0 = 16 * ct + 4 * (lane >> 4);
-                nib = KT > 0 ? 0xFu : (c0 >= k ? 0u : (k - c0 >= 4 ? 0xFu : (1u << (k - c0)) - 1u));
-            }
-            m[ct >> 1] |= nib << ((ct & 1) * 16 + 4 * (lane >> 4));
-        }
-#pragma unroll
-        for (int w = 0; w < MAXK / 32; ++w) {
-            if (w < nwords) {
-                m[w] |= xor16_u(m[w]);
-                m[w] |= xor32_u(m[w]);
-            }
-        }
-        if (lane < 16) {
-            const int slot = wave * 64 + 16 * j + lane;
-            cmask[slot * 2 + 0] = static_cast<uint64_t>(m[0]) | (static_cast<uint64_t>(m[1]) << 32);
-            cmask[slot * 2 + 1] = static_cast<uint64_t>(m[2]) | (static_cast<uint64_t>(m[3]) << 32);
-        }
-    }
-    km_wave_lds_sync();
-
-    float best = 3.402823466e38f;  // FLT_MAX
-    int arg = 0;
-    if constexpr (EXACT) {
-        // exact reference distance to every candidate of the thread's token
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            uint64_t mm = cmask[tid * 2 + w];
-            while (mm) {
-                const int c = 64 * w + __builtin_ctzll(mm);
-                mm &= mm - 1;
-                const float dist = l2_lanes8_bf16<DP>(xr, cs + c * CS);
-                if (dist < best) {
-                    best = dist;
-                    arg = c;
-                }
-            }
-        }
-    } else {
-        // No distance is read: a lone candidate is the reference's label (the
-        // bound above).  Tokens with several candidates (a few percent, but
-        // in most waves) queue up; their (token, candidate) distances are
-        // spread over the block, 8 lanes per pair.
-        const uint64_t m0 = cmask[tid * 2], m1 = cmask[tid * 2 + 1];
-        arg = m0 ? __builtin_ctzll(m0) : (m1 ? 64 + __builtin_ctzll(m1) : 0);
-        const bool multi = valid && __popcll(m0) + __popcll(m1) > 1;
-        const uint64_t bal = __ballot(multi);
-        int slot = 0;
-        if (bal) {
-            int base = 0;
-            if (lane == 0) base = atomicAdd(qcnt, __popcll(bal));
-            slot = __shfl(base, 0) + __popcll(bal & lanemask_lt());
-        }
-        if (multi && slot < kScreenQueue) qtok[slot] = tid;
-        __syncthreads();
-        const int nq = min(*qcnt, kScreenQueue);
-        if (wave == 0) {
-            // the pairs of queued token i are [qoff[i], qoff[i + 1])
-            int n = 0;
-            if (lane < nq) {
-                const int tk = qtok[lane];
-                n = __popcll(cmask[tk * 2]) + __popcll(cmask[tk * 2 + 1]);
-                qbest[lane] = ~0ull;
-            }
-            const int incl = wave_incl_scan(n);
-            if (lane < kScreenQueue) qoff[lane] = incl - n;
-            if (lane == 63) qoff[kScreenQueue] = incl;
-        }
-        __syncthreads();
-        {
-            // Pair p on lanes 8 (p % 8) .. +7 of wave (p / 8) % 4: lane part j
-            // sums dims j, j + 8, .. in ascending order (the reference's
-            // lane j), the group adds the eight sums left to right on its
-            // first lane (row shifts inside the 16-lane row), and an LDS
-            // minimum over (distance bits, centroid) keeps the smallest
-            // distance below FLT_MAX and, among equal ones, the lowest
-            // centroid: the reference's strict < over ascending centroids.
-            const int npairs = qoff[kScreenQueue];
-            const int part = lane & 7;
+                while (full) {
+                    const int tk = __builtin_ctzll(full);
+                    full &= full - 1;
+                    const uint16_t* row = kb + static_cast<int64_t>(t0 + tk) * a.ts;
+                    unsigned long long key = ~0ull;
 #pragma unroll 1
-            for (int p0 = 0; p0 < npairs; p0 += 32) {
-                const int pr = p0 + wave * 8 + (lane >> 3);
+                    for (int c = lane; c < k; c += 64) {
+                        const float d = l2_lanes8_rolled<DP>(row, cg + static_cast<int64_t>(c) * DP);
+                        const unsigned long long kv =
+                            (static_cast<unsigned long long>(__float_as_uint(d)) << 32) | static_cast<uint32_t>(c);
+                        if (d < kFltMax && kv < key) key = kv;
+                    }
+#pragma unroll
+                    for (int o = 32; o > 0; o >>= 1) {
+                        const unsigned long long y = __shfl_xor(key, o);
+                        key = y < key ? y : key;
+                    }
+                    if (lane == tk) {
+                        arg = key == ~0ull ? 0 : static_cast<int>(static_cast<uint32_t>(key));
+                        best = key == ~0ull ? kFltMax : __uint_as_float(static_cast<uint32_t>(key >> 32));
+                    }
+                }
+            }
+        }
+        if constexpr (EXACT != kLabelsOnly) {
+            // the lane's own token row (in L2: its tiles were just read)
+            km_u32x4_t xr[DP / 8];
+            const uint16_t* src = kb + static_cast<int64_t>(min(t, a.T - 1)) * a.ts;
+#pragma unroll
+            for (int i = 0; i < DP / 8; ++i) xr[i] = *reinterpret_cast<const km_u32x4_t*>(src + 8 * i);
+            auto dist = [&](int c) {
+                return EXACT == kExactLds ? l2_lanes8_bf16<DP>(xr, cs + c * CS)
+                                          : l2_lanes8_bf16<DP>(xr, cg + static_cast<int64_t>(c) * DP);
+            };
+            if (!every) {
+                const int lo = pair ? min(c1, c2) : c1;
+                const float d = dist(lo);
+                if (d < best) {
+                    best = d;
+                    arg = lo;
+                }
+                if (pair) {
+                    const int hi = max(c1, c2);
+                    const float d2 = dist(hi);
+                    if (d2 < best) {
+                        best = d2;
+                        arg = hi;
+                    }
+                }
+            }
+        }
+        if (blk + 1 < blk1) load_tokens(blk + 1);
+        if constexpr (EXACT == kLabelsOnly) {
+            if (!every) arg = c1;
+            // Tokens with two candidates, four at a time: lanes 16 i .. + 7
+            // take the i-th token's lower candidate, + 8 .. + 15 the higher.
+            // Lane part j sums dims j, j + 8, .. in ascending order (the
+            // reference's lane j) and the first lane adds the eight sums left
+            // to right (row shifts).
+            uint64_t todo = __ballot(pair && valid);
+            while (todo) {
+                int s[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[i] = todo ? __builtin_ctzll(todo) : s[0];
+                    todo &= todo - 1;
+                }
+                const int tk = grp == 0 ? s[0] : grp == 1 ? s[1] : grp == 2 ? s[2] : s[3];
+                const int ca = __shfl(min(c1, c2), tk), cb = __shfl(max(c1, c2), tk);
+                const int c = lane & 8 ? cb : ca;
+                const int part = lane & 7;
+                const uint16_t* xrow = kb + static_cast<int64_t>(t0 + tk) * a.ts + part;
+                const float* crow = cg + static_cast<int64_t>(c) * DP + part;
+                uint16_t xv[DP / 8];
+                float cv[DP / 8];
+#pragma unroll
+                for (int i = 0; i < DP / 8; ++i) {
+                    xv[i] = xrow[8 * i];
+                    cv[i] = crow[8 * i];
+                }
                 float acc = 0.0f;
-                int qi = 0, c = 0;
-                if (pr < npairs) {
-                    for (int step = 32; step > 0; step >>= 1)
-                        if (qi + step < nq && qoff[qi + step] <= pr) qi += step;
-                    const int tk = qtok[qi];
-                    int r = pr - qoff[qi];
-                    const uint64_t w0 = cmask[tk * 2], w1 = cmask[tk * 2 + 1];
-                    const int n0 = __popcll(w0);
-                    uint64_t mm = r < n0 ? w0 : w1;
-                    const int cb = r < n0 ? 0 : 64;
-                    r = r < n0 ? r : r - n0;
-                    for (int i = 0; i < r; ++i) mm &= mm - 1;
-                    c = cb + __builtin_ctzll(mm);
-                    const uint16_t* xr = kb + static_cast<int64_t>(blk * 256 + tk) * a.ts + part;
-                    uint16_t xv[DP / 8];
 #pragma unroll
-                    for (int i = 0; i < DP / 8; ++i) xv[i] = xr[8 * i];
-                    const float* cr = cs + c * CS + part;
-#pragma unroll
-                    for (int i = 0; i < DP / 8; ++i) {
-                        const float d = bf16_to_f32(xv[i]) - cr[8 * i];
-                        acc = __builtin_fmaf(d, d, acc);
-                    }
+                for (int i = 0; i < DP / 8; ++i) {
+                    const float d = bf16_to_f32(xv[i]) - cv[i];
+                    acc = __builtin_fmaf(d, d, acc);
                 }
-                float t = acc;
-                t = t + dpp_row_shl<1>(acc);
-                t = t + dpp_row_shl<2>(acc);
-                t = t + dpp_row_shl<3>(acc);
-                t = t + dpp_row_shl<4>(acc);
-                t = t + dpp_row_shl<5>(acc);
-                t = t + dpp_row_shl<6>(acc);
-                t = t + dpp_row_shl<7>(acc);
-                if (pr < npairs && part == 0 && t < 3.402823466e38f)
-                    atomicMin(reinterpret_cast<unsigned long long*>(&qbest[qi]),
-                              (static_cast<unsigned long long>(__float_as_uint(t)) << 32) | static_cast<uint32_t>(c));
-            }
-        }
-        // past the queue's end a token runs its own exact pass (its row
-        // re-read: it is in L2)
-        auto exact_label = [&](int tk) {
-            km_u32x4_t xq[DP / 8];
+                float d = acc;
+                d = d + dpp_row_shl<1>(acc);
+                d = d + dpp_row_shl<2>(acc);
+                d = d + dpp_row_shl<3>(acc);
+                d = d + dpp_row_shl<4>(acc);
+                d = d + dpp_row_shl<5>(acc);
+                d = d + dpp_row_shl<6>(acc);
+                d = d + dpp_row_shl<7>(acc);
+                const float dh = dpp_row_shl<8>(d);   // the higher candidate's
+                int win = d < kFltMax ? ca : 0;
+                if (dh < (d < kFltMax ? d : kFltMax)) win = cb;
 #pragma unroll
-            for (int i = 0; i < DP / 8; ++i)
-                xq[i] = *reinterpret_cast<const km_u32x4_t*>(kb + static_cast<int64_t>(blk * 256 + tk) * a.ts + 8 * i);
-            float qb = 3.402823466e38f;
-            int qa = 0;
-#pragma unroll
-            for (int w = 0; w < 2; ++w) {
-                uint64_t mm = cmask[tk * 2 + w];
-                while (mm) {
-                    const int c = 64 * w + __builtin_ctzll(mm);
-                    mm &= mm - 1;
-                    const float dist = l2_lanes8_bf16<DP>(xq, cs + c * CS);
-                    if (dist < qb) {
-                        qb = dist;
-                        qa = c;
-                    }
+                for (int i = 0; i < 4; ++i) {
+                    const int w = __builtin_amdgcn_readlane(win, 16 * i);
+                    if (lane == s[i]) arg = w;
                 }
             }
-            return qa;
-        };
-        if (multi && slot >= kScreenQueue) arg = exact_label(tid);
-        __syncthreads();
-        if (multi && slot < kScreenQueue) {
-            const uint64_t b = qbest[slot];   // no distance below FLT_MAX: label 0, as the reference's loop
-            arg = b == ~0ull ? 0 : static_cast<int>(static_cast<uint32_t>(b));
         }
-        if (tid == 0) *qcnt = 0;   // read by every thread before the barrier above
-    }
-    if (valid) {
-        a.labels[static_cast<int64_t>(seg) * a.T + t] = arg;
-        if (EXACT && a.mind) a.mind[static_cast<int64_t>(seg) * a.T + t] = best;
-    }
-    if (a.hist == nullptr) continue;
-
-    float part = EXACT ? wave_sum(valid ? best : 0.0f) : 0.0f;
-    if (lane_id() == 0) red[tid >> 6] = part;
-    if (a.loff) {
-        // block member lists: the token at its place in the block's label order
-        const int pos = block_digit_pos(arg, valid, k, bits_for(k), wcnt, lofs, lwsum,
-                                        a.loff + (static_cast<int64_t>(seg) * a.nblk + blk) * (a.kmax + 1));
-        if (valid) a.rank[static_cast<int64_t>(seg) * a.T + blk * 256 + pos] = t;
-    } else {
-        const int r = block_digit_rank(arg, valid, k, bits_for(k), wcnt,
-                                       a.hist + static_cast<int64_t>(seg) * a.kmax * a.nblk, a.nblk, blk);
-        if (valid) a.rank[static_cast<int64_t>(seg) * a.T + t] = r;
-    }
-    if (tid == 0) a.ipart[static_cast<int64_t>(seg) * a.nblk + blk] = ((red[0] + red[1]) + red[2]) + red[3];
+        if (valid) {
+            a.labels[static_cast<int64_t>(seg) * a.T + t] = arg;
+            if (EXACT != kLabelsOnly && a.mind) a.mind[static_cast<int64_t>(seg) * a.T + t] = best;
+        }
+        if constexpr (EXACT != kLabelsOnly) {
+            if (a.wpart) {   // inertia partial of the wave's 64 tokens
+                const float part = wave_sum(valid ? best : 0.0f);
+                if (lane == 0 && (t0 >> 6) < 4 * a.nblk) a.wpart[static_cast<int64_t>(seg) * 4 * a.nblk + (t0 >> 6)] = part;
+            }
+        }
     }
 }
 
@@ -1041,163 +1025,147 @@ __global__ __launch_bounds__(256) void km_pp_pick_kernel(KmParams a, PpStep ps) 
     for (int d = tid; d < DP; d += 256) dst[d] = bf16_to_f32(xb[static_cast<int64_t>(sel) * a.ts + d]);
 }
 
-// Per segment: exclusive scan of the [label][block] counts, cluster offsets,
-// empty-cluster ordinals, inertia (fixed reduction order) and the early-stop
-// test of kmeans_core.cpp:244-262.  Up to 64 counts per thread (k * nblk <=
-// 65536, 16-byte aligned) stay in registers: one read, one write, and the
-// cluster offsets come from the threads that hold them; larger segments use
-// the two-pass block scan.
-constexpr int kScanRegInts = 64;
+// Early stop (kmeans_core.cpp:244-262) of one segment.  The inertia has a fixed
+// reduction order: the four wave partials of each 256-token block, contiguous
+// blocks per thread, lanes, then waves.  prev alternates between two slots,
+// so that several workgroups can run the test of one iteration.
+__device__ __forceinline__ float stop_block_partial(const KmParams& a, int seg, int b) {
+    const float* wp = a.wpart + static_cast<int64_t>(seg) * 4 * a.nblk;
+    const int nw = (a.T + 63) / 64;   // wave partials written
+    float v[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v[w] = 4 * b + w < nw ? wp[4 * b + w] : 0.0f;
+    return ((v[0] + v[1]) + v[2]) + v[3];
+}
 
-__global__ __launch_bounds__(1024) void km_scan_kernel(KmParams a, int it) {
-    __shared__ int sh[40];
-    __shared__ int soff[kIvfMaxK + 1];
+__device__ __forceinline__ bool stop_test(const KmParams& a, int seg, int it, float inertia, bool record) {
+    const float prev = a.prev[2 * seg + (it & 1)];
+    const float change = fabsf(prev - inertia);
+    const float rel = prev > 0.0f ? change / prev : 0.0f;
+    const bool min_ok = (it + 1) >= (a.es_min > 1 ? a.es_min : 1);
+    const bool stop = min_ok && (rel <= fmaxf(0.0f, a.es_rel) || change <= fmaxf(0.0f, a.tol));
+    if (record) {
+        if (a.iters) a.iters[seg] = it + 1;
+        if (stop)
+            a.done[seg] = 1;
+        else
+            a.prev[2 * seg + ((it + 1) & 1)] = inertia;
+    }
+    return stop;
+}
+
+__global__ __launch_bounds__(1024) void km_stop_kernel(KmParams a, int it) {
     __shared__ float sred[16];
-    __shared__ int stop;
-    const int seg = blockIdx.x;
-    if (a.done && a.done[seg]) return;
-    const int p = seg % a.P;
-    const int k = a.k[p];
-    const int tid = threadIdx.x, wave = tid >> 6;
-    int32_t* hist = a.hist + static_cast<int64_t>(seg) * a.kmax * a.nblk;
-    const int n = k * a.nblk;
-    const bool reg = n <= 1024 * kScanRegInts && (n & 3) == 0 && (reinterpret_cast<uintptr_t>(hist) & 15) == 0;
-    // this thread's counts: a contiguous run of `per` (multiple of 4) ints
-    int per = (n + 1023) / 1024;
-    per = (per + 3) & ~3;
-    const int lo = min(tid * per, n), hi = min(lo + per, n);
-    typedef int __attribute__((ext_vector_type(4))) i32x4;
-    i32x4 v[kScanRegInts / 4];
-    if (reg) {
-#pragma unroll
-        for (int u = 0; u < kScanRegInts / 4; ++u)
-            v[u] = lo + 4 * u < hi ? *reinterpret_cast<const i32x4*>(hist + lo + 4 * u) : i32x4{0, 0, 0, 0};
-    }
-    // inertia partials: contiguous chunk per thread, then waves in order
-    const float* ip = a.ipart + static_cast<int64_t>(seg) * a.nblk;
-    const int iper = (a.nblk + 1023) / 1024;
+    const int seg = blockIdx.x, tid = threadIdx.x;
+    if (a.done[seg]) return;
+    const int per = (a.nblk + 1023) / 1024;
     float part = 0.0f;
-    for (int b = tid * iper; b < (tid + 1) * iper && b < a.nblk; ++b) part += ip[b];
+    for (int b = tid * per; b < (tid + 1) * per && b < a.nblk; ++b) part += stop_block_partial(a, seg, b);
     part = wave_sum(part);
-    if ((tid & 63) == 0) sred[wave] = part;
-    int32_t* off = a.off + static_cast<int64_t>(seg) * (a.kmax + 1);
-    if (reg) {
-        int local = 0;
-#pragma unroll
-        for (int u = 0; u < kScanRegInts / 4; ++u) local += (v[u][0] + v[u][1]) + (v[u][2] + v[u][3]);
-        const int incl = wave_incl_scan(local);
-        if ((tid & 63) == 63) sh[wave] = incl;
-        __syncthreads();
-        if (tid < 64) {
-            const int x = tid < 16 ? sh[tid] : 0;
-            const int sc = wave_incl_scan(x);
-            if (tid < 16) sh[16 + tid] = sc - x;
-        }
-        __syncthreads();
-        const int run0 = sh[16 + wave] + incl - local;
-        // cluster offsets: the label boundaries c * nblk inside [lo, hi)
-        for (int c = (lo + a.nblk - 1) / a.nblk; c < k && c * a.nblk < hi; ++c) {
-            const int at = c * a.nblk - lo;
-            int sum = run0;
-#pragma unroll
-            for (int u = 0; u < kScanRegInts / 4; ++u)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) sum += 4 * u + e < at ? v[u][e] : 0;
-            off[c] = sum;
-            soff[c] = sum;
-        }
-        int run = run0;
-#pragma unroll
-        for (int u = 0; u < kScanRegInts / 4; ++u) {
-            if (lo + 4 * u < hi) {
-                i32x4 o;
-                o[0] = run;
-                run += v[u][0];
-                o[1] = run;
-                run += v[u][1];
-                o[2] = run;
-                run += v[u][2];
-                o[3] = run;
-                run += v[u][3];
-                *reinterpret_cast<i32x4*>(hist + lo + 4 * u) = o;
-            }
-        }
-    } else {
-        block_exclusive_scan_1024(hist, static_cast<int64_t>(n), sh);
-        for (int c = tid; c < k; c += 1024) {
-            const int o = hist[static_cast<int64_t>(c) * a.nblk];
-            off[c] = o;
-            soff[c] = o;
-        }
-    }
-    if (tid == 0) {
-        off[k] = a.T;
-        soff[k] = a.T;
-    }
+    if ((tid & 63) == 0) sred[tid >> 6] = part;
     __syncthreads();
-    // empty-cluster ordinals: exclusive count of empty clusters before c,
-    // 256 clusters at a time on the first four waves
-    for (int c0 = 0, carry = 0; c0 < k; c0 += 256) {
-        const int c = c0 + tid;
-        int empty = 0, eincl = 0;
-        if (wave < 4) {
-            empty = c < k && soff[c + 1] == soff[c] ? 1 : 0;
-            eincl = wave_incl_scan(empty);
-            if ((tid & 63) == 63) sh[32 + wave] = eincl;
-        }
-        __syncthreads();
-        if (wave < 4 && c < k) {
-            int before = carry;
-            for (int w = 0; w < wave; ++w) before += sh[32 + w];
-            a.empties[static_cast<int64_t>(seg) * a.kmax + c] = before + eincl - empty;
-        }
-        carry += (sh[32] + sh[33]) + (sh[34] + sh[35]);
-        __syncthreads();
-    }
     if (tid == 0) {
         float inertia = 0.0f;
         for (int w = 0; w < 16; ++w) inertia += sred[w];
-        if (a.iters) a.iters[seg] = it + 1;
-        const float prev = a.prev[seg];
-        const float change = fabsf(prev - inertia);
-        const float rel = prev > 0.0f ? change / prev : 0.0f;
-        const bool min_ok = (it + 1) >= (a.es_min > 1 ? a.es_min : 1);
-        stop = min_ok && (rel <= fmaxf(0.0f, a.es_rel) || change <= fmaxf(0.0f, a.tol));
-        if (!stop) a.prev[seg] = inertia;
+        stop_test(a, seg, it, inertia, true);
     }
-    __syncthreads();
-    if (tid == 0 && stop && a.done) a.done[seg] = 1;
 }
 
-// Member lists: token t of block b goes to the scanned [label][block] offset
-// plus its rank in the block.  Each thread takes one token of each of
-// kScatterBlocks consecutive blocks, so all its loads are in flight together.
-constexpr int kScatterBlocks = 4;
+// Member lists by superblocks of a.sbt tokens: each workgroup puts its
+// tokens in label order (ascending token inside a label) into its own slice
+// of `sorted` and writes the superblock's row of label offsets (loff[0 .. k]:
+// first place of each label, then the token count).  A stable counting sort:
+// label counts per wave (a wave owns consecutive tokens), one scan over
+// (label, wave), then every round of 64 tokens takes its places from the
+// wave's running offsets.  The ordered slice goes through LDS (coalesced
+// stores) up to kStagedTokens tokens.  11.6 us at 128k tokens, 16 segments;
+// superblocks of thousands of tokens keep the M-step's member search and its
+// column of label offsets short (62 us per M-step, 68 us with one row of
+// offsets per 256 tokens), and serve any T (a scan over per-block histograms
+// and a scatter took 340 us at 512k tokens, k = 181; this kernel 34 us).
+constexpr int kStagedTokens = 32768;
 
-__global__ __launch_bounds__(256) void km_scatter_kernel(KmParams a) {
-    const int seg = blockIdx.y;
+__host__ __device__ inline size_t members_lds_bytes(int waves, int kmax, int sbt) {
+    return (static_cast<size_t>(waves) * kmax + 32) * sizeof(int) + (sbt <= kStagedTokens ? 2 * static_cast<size_t>(sbt) : 0);
+}
+
+__global__ __launch_bounds__(1024) void km_members_kernel(KmParams a) {
+    extern __shared__ int smem_i[];
+    const int seg = blockIdx.y, sb = blockIdx.x;
     if (a.done && a.done[seg]) return;
-    const int64_t so = static_cast<int64_t>(seg) * a.T;
-    const int32_t* hist = a.hist + static_cast<int64_t>(seg) * a.kmax * a.nblk;
-    int lab[kScatterBlocks], rnk[kScatterBlocks];
+    const int k = a.k[seg % a.P], bits = bits_for(k);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int nthr = blockDim.x, nw = nthr >> 6;
+    int* cnt = smem_i;                          // [nw][k]
+    int* wsum = smem_i + nw * a.kmax;           // [16]
+    uint16_t* place = reinterpret_cast<uint16_t*>(wsum + 32);
+    const bool staged = a.sbt <= kStagedTokens;
+    const int base = sb * a.sbt;
+    const int m = min(a.sbt, a.T - base);
+    const int32_t* lab = a.labels + static_cast<int64_t>(seg) * a.T + base;
+    const int span = a.sbt / nw;                // tokens per wave (a multiple of 64)
+    const int w0 = wave * span, w1 = min(w0 + span, m);
+    for (int i = tid; i < nw * k; i += nthr) cnt[i] = 0;
+    __syncthreads();
+    int* mine = cnt + wave * k;
+    for (int i = w0; i < w1; i += 256) {
+        int l[4];
 #pragma unroll
-    for (int u = 0; u < kScatterBlocks; ++u) {
-        const int t = (blockIdx.x * kScatterBlocks + u) * 256 + threadIdx.x;
-        const bool in = t < a.T;
-        lab[u] = in ? a.labels[so + t] : 0;
-        rnk[u] = in ? a.rank[so + t] : 0;
-    }
-    int base[kScatterBlocks];
+        for (int u = 0; u < 4; ++u) l[u] = lab[min(i + 64 * u + lane, m - 1)];
 #pragma unroll
-    for (int u = 0; u < kScatterBlocks; ++u) {
-        const int blk = blockIdx.x * kScatterBlocks + u;
-        base[u] = blk < a.nblk ? hist[static_cast<int64_t>(lab[u]) * a.nblk + blk] : 0;
+        for (int u = 0; u < 4; ++u)
+            if (i + 64 * u + lane < w1) atomicAdd(&mine[l[u]], 1);
     }
+    __syncthreads();
+    // exclusive offsets over (label, wave): consecutive labels per thread
+    const int per = (k + nthr - 1) / nthr;
+    const int c0 = min(tid * per, k), c1 = min(c0 + per, k);
+    int local = 0;
+    for (int c = c0; c < c1; ++c)
+        for (int w = 0; w < nw; ++w) local += cnt[w * k + c];
+    const int incl = wave_incl_scan(local);
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int run = incl - local;
+    for (int w = 0; w < wave; ++w) run += wsum[w];
+    int32_t* row = a.loff + (static_cast<int64_t>(seg) * a.nsb + sb) * (a.kmax + 1);
+    for (int c = c0; c < c1; ++c) {
+        row[c] = run;
+        for (int w = 0; w < nw; ++w) {
+            const int n = cnt[w * k + c];
+            cnt[w * k + c] = run;
+            run += n;
+        }
+    }
+    if (tid == 0) row[k] = m;
+    __syncthreads();
+    int32_t* out = a.sorted + static_cast<int64_t>(seg) * a.T + base;
+    for (int i = w0; i < w1; i += 256) {
+        int l[4];
 #pragma unroll
-    for (int u = 0; u < kScatterBlocks; ++u) {
-        const int t = (blockIdx.x * kScatterBlocks + u) * 256 + threadIdx.x;
-        if (t < a.T) a.sorted[so + base[u] + rnk[u]] = t;
+        for (int u = 0; u < 4; ++u) l[u] = lab[min(i + 64 * u + lane, m - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (i + 64 * u >= w1) break;
+            const int tk = i + 64 * u + lane;
+            const bool in = tk < w1;
+            const uint64_t peers = match_peers(static_cast<uint32_t>(l[u]), bits, __ballot(in));
+            const int rank = __popcll(peers & lanemask_lt());
+            const int at = in ? mine[l[u]] : 0;
+            km_wave_lds_sync();
+            if (in) {
+                if (rank == 0) mine[l[u]] = at + __popcll(peers);
+                if (staged)
+                    place[at + rank] = static_cast<uint16_t>(tk);
+                else
+                    out[at + rank] = base + tk;
+            }
+            km_wave_lds_sync();
+        }
     }
+    if (!staged) return;
+    __syncthreads();
+    for (int i = tid; i < m; i += nthr) out[i] = base + place[i];
 }
 
 // M-step, one workgroup per cluster: wave 0 keeps the chains (lane d =
@@ -1209,8 +1177,16 @@ __global__ __launch_bounds__(256) void km_scatter_kernel(KmParams a) {
 // q+1 while wave 0 sums round q), one barrier per round.  Each loader keeps
 // NB local batches in flight in a register ring and loads the member ids 2 NB
 // local batches ahead.
-template <int DP>
-__global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws draws) {
+// SUPER: a power of two, at least the superblocks (the member search's steps).
+// SUPER = 0: no member lists; every workgroup scans the segment's labels
+// itself (a quarter per wave, the matching tokens to the wave's LDS slice, in
+// order), and runs the early-stop test of the iteration.  For the shortest
+// contexts the two launches this saves cost more than the scan: at 11k
+// tokens, k = 32, 4 heads, 11.8 us against 8.3 + 4.8 us (and 3.1 us for a stop
+// test) plus the launches between.
+template <int DP, int SUPER>
+__global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws draws, int it) {
+    constexpr bool SCAN = SUPER == 0;
     constexpr int PARTS = DP / 8;    // 16-byte parts per row
     constexpr int RPL = 64 / PARTS;  // rows per load instruction
     constexpr int LPB = PARTS;       // load instructions per 64-row batch
@@ -1222,11 +1198,15 @@ __global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws 
     constexpr int NB = 2;
     constexpr int HALVES = DP > 64 ? DP / 64 : 1;   // dims per chain lane
     __shared__ km_u32x4_t ring[2 * NL][64 * PARTS];
-    // block member lists: the label's exclusive prefix over the blocks, its
-    // first place in each block, the waves' member counts
-    __shared__ int s_pref[kLocalMaxBlk];
-    __shared__ int s_lof[kLocalMaxBlk];
+    // the label's exclusive prefix over the superblocks, its first place in
+    // each, the waves' member counts
+    __shared__ int s_pref[SCAN ? 1 : kMaxSuper];
+    __shared__ int s_lof[SCAN ? 1 : kMaxSuper];
     __shared__ int s_wt[4];
+    __shared__ int s_emp;
+    __shared__ int s_stop;
+    __shared__ uint8_t s_seen[SCAN ? kImiMaxK : 1];
+    extern __shared__ uint16_t s_list[];   // SCAN: [4][span]
     const int c = blockIdx.x, seg = blockIdx.y;
     const int h = seg / a.P, p = seg % a.P;
     if (c >= a.k[p]) return;
@@ -1234,81 +1214,125 @@ __global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint16_t* kbase = a.keys + h * a.hs + p * DP;
     float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + c) * DP;
-    const bool local = a.loff != nullptr;
-    int lo = 0, n = 0;
-    if (local) {
-        // this label's first place and count in every block (nblk <= 512:
-        // two blocks per thread, their offset pairs loaded together), then
-        // the prefix of the counts
-        const int32_t* rows = a.loff + static_cast<int64_t>(seg) * a.nblk * (a.kmax + 1) + c;
-        int cv[kLocalMaxBlk / 256], lv[kLocalMaxBlk / 256];
+    const int32_t* rows = a.loff + static_cast<int64_t>(seg) * a.nsb * (a.kmax + 1);
+    const int32_t* lab = a.labels + static_cast<int64_t>(seg) * a.T;
+    const int span = (a.T + 255) / 256 * 64;   // SCAN: tokens per wave
+    if (tid == 0) s_emp = 0;
+    if constexpr (SCAN) {
+        if (a.exact && wave == 0) {   // at most 64 blocks: one per lane
+            const float inertia = wave_sum(lane < a.nblk ? stop_block_partial(a, seg, lane) : 0.0f);
+            const bool stop = stop_test(a, seg, it, inertia, c == 0 && lane == 0);
+            if (lane == 0) s_stop = stop;
+        }
+        const int w0 = wave * span, w1 = min(w0 + span, a.T);
+        int run = 0;
+        // four consecutive labels per lane and load, eight loads in flight
+        typedef int __attribute__((ext_vector_type(4), aligned(4))) i32x4;
+        for (int i = w0; i < w1; i += 2048) {
+            i32x4 l[8];
 #pragma unroll
-        for (int u = 0; u < kLocalMaxBlk / 256; ++u) {
-            const int b = min(2 * tid + u, a.nblk - 1);
-            lv[u] = rows[static_cast<int64_t>(b) * (a.kmax + 1)];
-            cv[u] = rows[static_cast<int64_t>(b) * (a.kmax + 1) + 1];
+            for (int u = 0; u < 8; ++u) {
+                const int tk = i + 256 * u + 4 * lane;
+                if (tk + 4 <= a.T) {
+                    l[u] = *reinterpret_cast<const i32x4*>(lab + tk);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) l[u][e] = tk + e < a.T ? lab[tk + e] : -1;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (i + 256 * u >= w1) break;
+                const int tk = i + 256 * u + 4 * lane;
+                bool hit[4];
+                int cnt = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hit[e] = l[u][e] == c && tk + e < w1;
+                    cnt += hit[e];
+                }
+                const int incl = wave_incl_scan(cnt);
+                int at = w0 + run + incl - cnt;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (hit[e]) s_list[at++] = static_cast<uint16_t>(tk + e);
+                run += __builtin_amdgcn_readlane(incl, 63);
+            }
+        }
+        if (lane == 0) s_wt[wave] = run;
+        __syncthreads();
+        if (a.exact && s_stop) return;
+    } else {
+        // this label's first place and count in every superblock (two per
+        // thread, their offset pairs loaded together), then the prefix of the
+        // counts
+        int cv[kMaxSuper / 256], lv[kMaxSuper / 256];
+#pragma unroll
+        for (int u = 0; u < kMaxSuper / 256; ++u) {
+            const int32_t* r = rows + static_cast<int64_t>(min(2 * tid + u, a.nsb - 1)) * (a.kmax + 1) + c;
+            lv[u] = r[0];
+            cv[u] = r[1];
         }
 #pragma unroll
-        for (int u = 0; u < kLocalMaxBlk / 256; ++u) cv[u] = 2 * tid + u < a.nblk ? cv[u] - lv[u] : 0;
-        const int run = cv[0] + cv[1];
-        const int incl = wave_incl_scan(run);
+        for (int u = 0; u < kMaxSuper / 256; ++u) cv[u] = 2 * tid + u < a.nsb ? cv[u] - lv[u] : 0;
+        const int both = cv[0] + cv[1];
+        const int incl = wave_incl_scan(both);
         if (lane == 63) s_wt[wave] = incl;
         __syncthreads();
-        int before = incl - run;
+        int before = incl - both;
         for (int w = 0; w < wave; ++w) before += s_wt[w];
-        if (2 * tid < a.nblk) {
+        if (2 * tid < a.nsb) {
             s_pref[2 * tid] = before;
             s_lof[2 * tid] = lv[0];
         }
-        if (2 * tid + 1 < a.nblk) {
+        if (2 * tid + 1 < a.nsb) {
             s_pref[2 * tid + 1] = before + cv[0];
             s_lof[2 * tid + 1] = lv[1];
         }
         __syncthreads();
-        n = (s_wt[0] + s_wt[1]) + (s_wt[2] + s_wt[3]);
-    } else {
-        const int32_t* off = a.off + static_cast<int64_t>(seg) * (a.kmax + 1);
-        lo = off[c];
-        n = off[c + 1] - lo;
     }
+    const int n = (s_wt[0] + s_wt[1]) + (s_wt[2] + s_wt[3]);
     if (n == 0) {
-        int e;
-        if (local) {
-            // the empty ordinal: labels below c whose block counts are all zero
-            // (every thread sums one label's column, in parallel over labels)
-            __shared__ int s_emp;
-            if (tid == 0) s_emp = 0;
+        // the empty ordinal: labels below c with no member
+        if constexpr (SCAN) {
+            for (int c2 = tid; c2 < c; c2 += 256) s_seen[c2] = 0;
             __syncthreads();
-            for (int c2 = tid; c2 < c; c2 += 256) {
-                const int32_t* r2 = a.loff + static_cast<int64_t>(seg) * a.nblk * (a.kmax + 1) + c2;
-                int sum = 0;
-                for (int b = 0; b < a.nblk; ++b) sum += r2[static_cast<int64_t>(b) * (a.kmax + 1) + 1] - r2[static_cast<int64_t>(b) * (a.kmax + 1)];
-                if (sum == 0) atomicAdd(&s_emp, 1);
-            }
+            for (int i = tid; i < a.T; i += 256) s_seen[lab[i]] = 1;
             __syncthreads();
-            e = s_emp;
-        } else {
-            e = a.empties[static_cast<int64_t>(seg) * a.kmax + c];   // past this launch's draws: km_reseed_kernel
         }
+        for (int c2 = tid; c2 < c; c2 += 256) {
+            int any = SCAN ? s_seen[c2] : 0;
+            if (!SCAN)
+            for (int b = 0; b < a.nsb; ++b) {
+                const int32_t* r = rows + static_cast<int64_t>(b) * (a.kmax + 1) + c2;
+                any |= r[1] - r[0];
+            }
+            if (any == 0) atomicAdd(&s_emp, 1);
+        }
+        __syncthreads();
+        const int e = s_emp;
+        if (tid == 0) a.empties[static_cast<int64_t>(seg) * a.kmax + c] = e;   // past this launch's draws: km_reseed_kernel
         if (wave == 0 && e < kDraws) {
             const int tok = draws.v[e];
             for (int d = lane; d < DP; d += 64) dst[d] = bf16_to_f32(kbase[static_cast<int64_t>(tok) * a.ts + d]);
         }
         return;
     }
+    if (tid == 0) a.empties[static_cast<int64_t>(seg) * a.kmax + c] = -1;
     const int nb = (n + 63) >> 6;              // 64-row batches
     const int rounds = (nb + NL - 1) / NL;     // = local batches of loader 1
-    const int32_t* srt = a.sorted + static_cast<int64_t>(seg) * a.T + lo;
-    const int32_t* lst = a.rank + static_cast<int64_t>(seg) * a.T;
-    // member j: the block holding it (the last one whose prefix is <= j) and
-    // its place there
+    const int32_t* lst = a.sorted + static_cast<int64_t>(seg) * a.T;
+    // member j: the superblock holding it (the last one whose prefix is <= j)
+    // and its place there
+    const int p1 = s_wt[0], p2 = p1 + s_wt[1], p3 = p2 + s_wt[2];
     auto member = [&](int j) {
-        if (!local) return srt[j];
+        if constexpr (SCAN)
+            return static_cast<int>(s_list[j < p1 ? j : j < p2 ? span + j - p1 : j < p3 ? 2 * span + j - p2 : 3 * span + j - p3]);
         int b = 0;
 #pragma unroll
-        for (int step = kLocalMaxBlk / 2; step > 0; step >>= 1)
-            b = (b + step < a.nblk && s_pref[b + step] <= j) ? b + step : b;
-        return lst[b * 256 + s_lof[b] + (j - s_pref[b])];
+        for (int step = SUPER / 2; step > 0; step >>= 1)
+            b = (b + step < a.nsb && s_pref[b + step] <= j) ? b + step : b;
+        return lst[static_cast<int64_t>(b) * a.sbt + s_lof[b] + (j - s_pref[b])];
     };
     // rounds padded to whole ring cycles: the loaders' loop body is then free
     // of branches, so the compiler's wait before each slot write counts the
@@ -1461,8 +1485,6 @@ __global__ __launch_bounds__(64) void km_reseed_kernel(KmParams a, Draws draws, 
     const int h = seg / a.P, p = seg % a.P;
     if (c >= a.k[p]) return;
     if (a.done && a.done[seg]) return;
-    const int32_t* off = a.off + static_cast<int64_t>(seg) * (a.kmax + 1);
-    if (off[c + 1] != off[c]) return;
     const int e = a.empties[static_cast<int64_t>(seg) * a.kmax + c] - e0;
     if (e < 0 || e >= kDraws) return;
     const uint16_t* row = a.keys + h * a.hs + p * a.DP + static_cast<int64_t>(draws.v[e]) * a.ts;
@@ -1473,9 +1495,9 @@ __global__ __launch_bounds__(64) void km_reseed_kernel(KmParams a, Draws draws, 
 __global__ void km_reset_kernel(KmParams a) {
     const int seg = blockIdx.x * blockDim.x + threadIdx.x;
     if (seg >= a.H * a.P) return;
-    a.prev[seg] = 3.402823466e38f;
+    a.prev[2 * seg] = a.prev[2 * seg + 1] = 3.402823466e38f;
     if (a.done) a.done[seg] = 0;
-    if (a.iters) a.iters[seg] = a.loff ? a.max_iters : 0;   // no km_scan counts them without early stop
+    if (a.iters) a.iters[seg] = a.done ? 0 : a.max_iters;   // km_stop counts them with early stop
 }
 
 int validate(const imi_kmeans_args* a, int& kmax, int& dp) {
@@ -1510,88 +1532,115 @@ int validate(const imi_kmeans_args* a, int& kmax, int& dp) {
     return IMI_OK;
 }
 
+// Superblocks of the member lists: about two rounds of workgroups over the
+// device, 1024 .. 8192 tokens each (a segment's slice then sorts in LDS), and
+// at most kMaxSuper of them.
+void superblocks(int T, int segs, int& sbt, int& nsb) {
+    sbt = 1024;
+    while (sbt < 8192 && static_cast<int64_t>(sbt) * 2 * device_cus() < static_cast<int64_t>(T) * segs) sbt *= 2;
+    while ((static_cast<int64_t>(T) + sbt - 1) / sbt > kMaxSuper) sbt *= 2;
+    nsb = static_cast<int>((static_cast<int64_t>(T) + sbt - 1) / sbt);
+}
+
 size_t workspace_bytes(const imi_kmeans_args* a, int kmax, KmParams* out) {
     const int segs = a->kv_heads * a->parts;
     const int nblk = (a->n_tokens + 255) / 256;
     Carver cv(a->workspace);
     KmParams p{};
-    p.hist = cv.take<int32_t>(static_cast<size_t>(segs) * kmax * nblk);
-    p.rank = cv.take<int32_t>(static_cast<size_t>(segs) * a->n_tokens);
-    p.ipart = cv.take<float>(static_cast<size_t>(segs) * nblk);
+    superblocks(a->n_tokens, segs, p.sbt, p.nsb);
+    p.wpart = cv.take<float>(static_cast<size_t>(segs) * 4 * nblk);
     p.sorted = cv.take<int32_t>(static_cast<size_t>(segs) * a->n_tokens);
-    p.off = cv.take<int32_t>(static_cast<size_t>(segs) * (kmax + 1));
+    p.loff = cv.take<int32_t>(static_cast<size_t>(segs) * p.nsb * (kmax + 1));
     p.empties = cv.take<int32_t>(static_cast<size_t>(segs) * kmax);
-    p.prev = cv.take<float>(segs);
+    p.prev = cv.take<float>(2 * segs);
     p.done = cv.take<int32_t>(segs);
-    p.loff = cv.take<int32_t>(static_cast<size_t>(segs) * nblk * (kmax + 1));
     if (a->init_mode == 2) {
         const int nbp = (a->n_tokens + kPpRows - 1) / kPpRows;
-        PpBlock* st = cv.take<PpBlock>(static_cast<size_t>(2) * segs * nbp);   // two launches' worth
-        if (out) p.ppstats = st;
+        p.ppstats = cv.take<PpBlock>(static_cast<size_t>(2) * segs * nbp);   // two launches' worth
+        p.ppmd = cv.take<float>(static_cast<size_t>(segs) * a->n_tokens);
     }
     if (out) *out = p;
     return cv.used();
 }
 
-template <int DP, int MAXK, int KT, bool EXACT>
-int launch_screen(const KmParams& p, int segs, hipStream_t stream) {
-    const size_t lds = screen_lds_bytes<DP>(p.kmax);
-    const void* fn = reinterpret_cast<const void*>(&km_assign_screen_kernel<DP, MAXK, KT, EXACT>);
+template <int DP, int NW, bool STREAM, int EXACT>
+int launch_screen(const KmParams& p, int segs, size_t lds, hipStream_t stream) {
+    const void* fn = reinterpret_cast<const void*>(&km_screen_kernel<DP, NW, STREAM, EXACT>);
     if (lds > 64 * 1024)
         IMI_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
     // as many workgroups as fit on the device at once, each over `chunks`
-    // consecutive 256-token blocks
+    // consecutive blocks of 64 NW tokens
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, km_assign_screen_kernel<DP, MAXK, KT, EXACT>, 256,
-                                                     lds) != hipSuccess ||
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, km_screen_kernel<DP, NW, STREAM, EXACT>, 64 * NW, lds) !=
+            hipSuccess ||
         per_cu <= 0)
         per_cu = 1;
+    const int nblk = (p.T + 64 * NW - 1) / (64 * NW);
     const int64_t want = static_cast<int64_t>(per_cu) * device_cus();
-    const int chunks = static_cast<int>(std::max<int64_t>(1, (static_cast<int64_t>(p.nblk) * segs + want - 1) / want));
-    const int gx = (p.nblk + chunks - 1) / chunks;
-    hipLaunchKernelGGL((km_assign_screen_kernel<DP, MAXK, KT, EXACT>), dim3(gx, segs), dim3(256), lds, stream, p,
-                       chunks);
-    IMI_LAUNCH_CHECK("km_assign_screen_kernel");
+    const int chunks = static_cast<int>(std::max<int64_t>(1, (static_cast<int64_t>(nblk) * segs + want - 1) / want));
+    hipLaunchKernelGGL((km_screen_kernel<DP, NW, STREAM, EXACT>), dim3((nblk + chunks - 1) / chunks, segs),
+                       dim3(64 * NW), lds, stream, p, chunks);
+    IMI_LAUNCH_CHECK("km_screen_kernel");
     return IMI_OK;
 }
 
-// EXACT: the distances are read (min distances or the early-stop inertia)
-template <int DP, int MAXK, int KT>
-int run_screen(const KmParams& p, int segs, hipStream_t stream) {
-    return p.exact ? launch_screen<DP, MAXK, KT, true>(p, segs, stream)
-                   : launch_screen<DP, MAXK, KT, false>(p, segs, stream);
+// p.exact: the distances are read (min distances or the early-stop inertia);
+// their fp32 centroid rows stay in LDS beside the packed tiles up to 150 KB.
+// Four waves per workgroup while at least two workgroups' centroids fit in a
+// CU's LDS, eight beyond.
+template <int DP>
+int run_assign(const KmParams& p, int segs, hipStream_t stream) {
+    using L = ScreenLds<DP>;
+    if constexpr (DP == 128) {
+        const size_t lds = L::packed(2 * kChunkTiles);
+        return p.exact ? launch_screen<DP, 4, true, kExactGlobal>(p, segs, lds, stream)
+                       : launch_screen<DP, 4, true, kLabelsOnly>(p, segs, lds, stream);
+    } else {
+        const size_t lds = L::packed((p.kmax + 15) / 16);
+        if (!p.exact)
+            return lds <= 52 * 1024 ? launch_screen<DP, 4, false, kLabelsOnly>(p, segs, lds, stream)
+                                    : launch_screen<DP, 8, false, kLabelsOnly>(p, segs, lds, stream);
+        const size_t both = lds + L::rows(p.kmax);
+        if (both <= 150 * 1024)
+            return both <= 52 * 1024 ? launch_screen<DP, 4, false, kExactLds>(p, segs, both, stream)
+                                     : launch_screen<DP, 8, false, kExactLds>(p, segs, both, stream);
+        return launch_screen<DP, 8, false, kExactGlobal>(p, segs, lds, stream);
+    }
+}
+
+// Whether the M-step scans the labels itself (km_update_block_kernel, SUPER =
+// 0): up to 16384 tokens (16-bit list entries, at most 64 blocks for the stop
+// test) and 2^19 (token, cluster) pairs per segment, so that the workgroups of
+// a segment read at most 2 MB of labels from L2.
+bool scans_labels(const KmParams& p) {
+    return p.DP <= 64 && p.T <= 16384 && static_cast<int64_t>(p.T) * p.kmax <= (1 << 19);
 }
 
 template <int DP>
-int run_assign(const KmParams& p, int segs, hipStream_t stream) {
-    if constexpr (DP == 128) {
-        const size_t lds = tiled_lds_bytes<DP>(p.kmax);
-        if (lds > 64 * 1024)
-            IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_assign_tiled_kernel<DP>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        hipLaunchKernelGGL(km_assign_tiled_kernel<DP>, dim3(p.nblk, segs), dim3(256), lds, stream, p);
-        IMI_LAUNCH_CHECK("km_assign_tiled_kernel");
-        return IMI_OK;
-    } else if (p.kmax <= kScreenMaxK) {
-        bool same = true;   // every subspace has kmax centroids
-        for (int q = 0; q < p.P; ++q) same = same && p.k[q] == p.kmax;
-        if (same) {
-            switch (p.kmax) {
-                case 16: return run_screen<DP, 64, 1>(p, segs, stream);
-                case 32: return run_screen<DP, 64, 2>(p, segs, stream);
-                case 64: return run_screen<DP, 64, 4>(p, segs, stream);
-                case 128: return run_screen<DP, kScreenMaxK, 8>(p, segs, stream);
-                default: break;
-            }
-        }
-        return p.kmax <= 64 ? run_screen<DP, 64, 0>(p, segs, stream) : run_screen<DP, kScreenMaxK, 0>(p, segs, stream);
-    }
-    const size_t lds = static_cast<size_t>(p.kmax) * DP * sizeof(float) + 4 * p.kmax * sizeof(int) + 64;
-    if (lds > 64 * 1024) IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_assign_kernel<DP>),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           static_cast<int>(lds)));
-    hipLaunchKernelGGL(km_assign_kernel<DP>, dim3(p.nblk, segs), dim3(256), lds, stream, p);
-    IMI_LAUNCH_CHECK("km_assign_kernel");
+int run_update(const KmParams& p, int segs, const Draws& dr, int it, hipStream_t stream) {
+    const dim3 grid(p.kmax, segs);
+    if (DP <= 64 && scans_labels(p)) {
+        constexpr int W = DP <= 64 ? DP : 64;
+        const size_t lists = static_cast<size_t>((p.T + 255) / 256) * 512;   // beside the ring and its like
+        IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_update_block_kernel<W, 0>),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lists)));
+        hipLaunchKernelGGL((km_update_block_kernel<W, 0>), grid, dim3(256), lists, stream, p, dr, it);
+    } else if (p.nsb <= 32)
+        hipLaunchKernelGGL((km_update_block_kernel<DP, 32>), grid, dim3(256), 0, stream, p, dr, it);
+    else
+        hipLaunchKernelGGL((km_update_block_kernel<DP, kMaxSuper>), grid, dim3(256), 0, stream, p, dr, it);
+    IMI_LAUNCH_CHECK("km_update_block_kernel");
+    return IMI_OK;
+}
+
+int run_members(const KmParams& p, int segs, hipStream_t stream) {
+    const int waves = p.kmax <= kImiMaxK ? 16 : 4;   // label counts per wave in LDS
+    const size_t lds = members_lds_bytes(waves, p.kmax, p.sbt);
+    if (lds > 64 * 1024)
+        IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_members_kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    hipLaunchKernelGGL(km_members_kernel, dim3(p.nsb, segs), dim3(64 * waves), lds, stream, p);
+    IMI_LAUNCH_CHECK("km_members_kernel");
     return IMI_OK;
 }
 
@@ -1647,11 +1696,6 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
     const int segs = a->kv_heads * a->parts;
     const bool early_stop = a->early_stop_min_iter <= a->max_iters;
     if (!early_stop) p.done = nullptr;  // no test can fire: skip the flag reads
-    // Block member lists instead of km_scan + km_scatter: without early stop
-    // (nothing reads the inertia), with the screened E-step (subspaces of at
-    // most 64 dims, k <= 128) and at most kLocalMaxBlk blocks.
-    const bool local = !early_stop && dp <= 64 && kmax <= kScreenMaxK && p.nblk <= kLocalMaxBlk;
-    if (!local) p.loff = nullptr;
 
     hipLaunchKernelGGL(km_reset_kernel, dim3((segs + 63) / 64), dim3(64), 0, stream, p);
     IMI_LAUNCH_CHECK("km_reset_kernel");
@@ -1675,9 +1719,9 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
         const int nbp = (a->n_tokens + kPpRows - 1) / kPpRows;
         ps.nbp = nbp;
         PpBlock* st = static_cast<PpBlock*>(p.ppstats);
-        // minima and statistics alternate between two buffers (the member
-        // lists' `rank` and `sorted`, free until the first E-step)
-        float* md[2] = {reinterpret_cast<float*>(p.rank), reinterpret_cast<float*>(p.sorted)};
+        // minima and statistics alternate between two buffers (one of them
+        // the member lists' `sorted`, free until the first M-step)
+        float* md[2] = {p.ppmd, reinterpret_cast<float*>(p.sorted)};
         PpBlock* sts[2] = {st, st + static_cast<size_t>(segs) * nbp};
         const size_t lds = static_cast<size_t>(256) * (dp / 8 + 1) * 16;
         if (dp == 128)   // 68 KB of LDS per workgroup
@@ -1733,12 +1777,13 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
         rc = dp == 128 ? run_assign<128>(p, segs, stream)
                        : (dp == 64 ? run_assign<64>(p, segs, stream) : run_assign<32>(p, segs, stream));
         if (rc) return rc;
-        if (!local) {
-            hipLaunchKernelGGL(km_scan_kernel, dim3(segs), dim3(1024), 0, stream, p, it);
-            IMI_LAUNCH_CHECK("km_scan_kernel");
-            hipLaunchKernelGGL(km_scatter_kernel, dim3((p.nblk + kScatterBlocks - 1) / kScatterBlocks, segs),
-                               dim3(256), 0, stream, p);
-            IMI_LAUNCH_CHECK("km_scatter_kernel");
+        if (!scans_labels(p)) {
+            if (p.exact) {   // (before, no test can fire)
+                hipLaunchKernelGGL(km_stop_kernel, dim3(segs), dim3(1024), 0, stream, p, it);
+                IMI_LAUNCH_CHECK("km_stop_kernel");
+            }
+            rc = run_members(p, segs, stream);
+            if (rc) return rc;
         }
         // Empty-cluster draws of this iteration: std::mt19937(it + 12345) with
         // uniform_int_distribution<int32_t>(0, T-1), one per empty cluster in
@@ -1747,13 +1792,9 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
         std::mt19937 rng(static_cast<unsigned>(it + 12345));
         std::uniform_int_distribution<int32_t> dist(0, a->n_tokens - 1);
         for (int e = 0; e < std::min(kmax, kDraws); ++e) dr.v[e] = dist(rng);
-        if (dp == 128)
-            hipLaunchKernelGGL(km_update_block_kernel<128>, dim3(kmax, segs), dim3(256), 0, stream, p, dr);
-        else if (dp == 64)
-            hipLaunchKernelGGL(km_update_block_kernel<64>, dim3(kmax, segs), dim3(256), 0, stream, p, dr);
-        else
-            hipLaunchKernelGGL(km_update_block_kernel<32>, dim3(kmax, segs), dim3(256), 0, stream, p, dr);
-        IMI_LAUNCH_CHECK("km_update_block_kernel");
+        rc = dp == 128 ? run_update<128>(p, segs, dr, it, stream)
+                       : (dp == 64 ? run_update<64>(p, segs, dr, it, stream) : run_update<32>(p, segs, dr, it, stream));
+        if (rc) return rc;
         // the draws of empty ordinals kDraws and up (IVF, k > kDraws)
         for (int e0 = kDraws; e0 < kmax; e0 += kDraws) {
             for (int e = e0; e < std::min(kmax, e0 + kDraws); ++e) dr.v[e - e0] = dist(rng);

@@ -1,0 +1,92 @@
+"""The screened E-step and the superblock member lists at the sizes where they
+can go wrong: centroid counts around a 16-centroid tile, a streamed chunk and
+the largest k of each width; tokens with exactly two candidates, with more (a
+few per wave and whole waves), and token counts around a wave, a workgroup
+and a superblock.  Labels, distances and centroids equal the oracle's bit for
+bit (the results are defined exactly, so there is no tolerance)."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import gpu_available
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a HIP device")]
+
+DEV = "cuda:0"
+
+
+def _bits(t):
+    return t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.uint16)
+
+
+def _copies(rng, cent, form):
+    """Exact ties: each of a few centroids repeated once (two candidates), or
+    three times more (every centroid is searched, for a few tokens or, with
+    every centroid equal, for whole waves)."""
+    k = cent.shape[0]
+    if form == "equal":
+        cent[:] = cent[0]
+    elif form != "distinct" and k >= 8:
+        n = 1 if form == "pairs" else 3
+        at = rng.permutation(k)
+        for i in range(0, k // (n + 1) * (n + 1), (n + 1) * (1 if form == "pairs" else 8)):
+            cent[at[i + 1:i + 1 + n]] = cent[at[i]]
+    return cent
+
+
+@pytest.mark.parametrize("T,k,parts,form", [
+    (1, 1, 2, "distinct"), (63, 2, 2, "equal"), (257, 3, 4, "distinct"), (65, 15, 4, "pairs"), (300, 16, 2, "few"),
+    (511, 17, 2, "pairs"), (1000, 64, 4, "few"), (513, 65, 2, "equal"), (777, 129, 2, "pairs"), (1025, 181, 2, "few"),
+    (600, 208, 2, "distinct"), (600, 209, 2, "pairs"), (900, 257, 2, "few"), (700, 511, 2, "equal"),
+    (700, 512, 2, "pairs"), (65, 1, 1, "distinct"), (130, 5, 1, "equal"), (257, 63, 1, "pairs"), (600, 64, 1, "few"),
+    (600, 65, 1, "distinct"), (500, 1018, 1, "pairs"), (300, 4095, 1, "few"), (257, 4096, 1, "equal")])
+def test_estep_edges(oracle, T, k, parts, form):
+    from adaptiveimi_amd import ops, synthetic
+
+    print(f"[estep] T={T} k={k} parts={parts} {form}", flush=True)
+    H, Dp = 2, 128 // parts
+    keys, _ = synthetic.make_kv(H, T, seed=T + k)
+    rng = np.random.default_rng(T * 4099 + k)
+    kf = oracle.bf16_to_f32(_bits(keys))
+    cent = rng.standard_normal((H, parts, k, Dp)).astype(np.float32)
+    for h in range(H):
+        for p in range(parts):   # centroids near the keys, so that the screen has close calls
+            sub = kf[h][:, p * Dp:(p + 1) * Dp]
+            cent[h, p] = sub[rng.integers(0, T, k)] + 0.1 * cent[h, p]
+            _copies(rng, cent[h, p], form)
+    kd, cd = keys.to(DEV), torch.from_numpy(cent).to(DEV)
+    plain, _ = ops.kmeans_assign(kd, cd, [k] * parts, with_distance=False)
+    labels, mind = ops.kmeans_assign(kd, cd, [k] * parts)
+    for h in range(H):
+        for p in range(parts):
+            ref, rmind, _ = oracle.estep(np.ascontiguousarray(kf[h][:, p * Dp:(p + 1) * Dp]), cent[h, p])
+            assert np.array_equal(plain[h, p].cpu().numpy(), ref), (h, p)
+            assert np.array_equal(labels[h, p].cpu().numpy(), ref), (h, p)
+            assert np.array_equal(mind[h, p].cpu().numpy(), rmind), (h, p)
+
+
+@pytest.mark.parametrize("H,T,ks,stop", [
+    (1, 63, (3, 5), False), (1, 1023, (16, 7), False), (2, 1025, (33, 64), True), (2, 2049, (129, 40), False),
+    (1, 4097, (8, 8, 5, 3), True), (8, 36000, (64, 64), False), (8, 70001, (45, 20), True), (1, 2050, (300,), False),
+    (2, 1030, (700,), True), (1, 530000, (4, 3), False), (2, 16384, (32, 5), True), (2, 16385, (32, 5), True),
+    (2, 4096, (128, 60), False), (2, 4097, (128, 60), False), (1, 300, (200, 256), True), (2, 8000, (125,), True),
+    (2, 8001, (125,), False)])
+def test_lloyd_over_superblock_edges(oracle, H, T, ks, stop):
+    """Two Lloyd iterations (labels, member order and sums) around the
+    superblocks' sizes (one of 1024 tokens, several, 8192 tokens each, more of
+    them than the 32 the short member search covers), and around the largest
+    segment whose M-step scans the labels itself and the largest mean cluster
+    that one wave sums."""
+    from adaptiveimi_amd import ops, synthetic
+
+    print(f"[lloyd] H={H} T={T} ks={ks} stop={stop}", flush=True)
+    keys, _ = synthetic.make_kv(H, T, seed=T)
+    kw = dict(early_stop_min_iter=1, tol=0.0, early_stop_rel_tol=0.0) if stop else {}
+    cent, labels, iters = ops.kmeans(keys.to(DEV), list(ks), 2, **kw)
+    kf = oracle.bf16_to_f32(_bits(keys))
+    for h in ([0, H - 1] if H > 1 else [0]):
+        labs, cents, its = oracle.kmeans_head(kf[h], list(ks), 2, **kw)
+        for p, k in enumerate(ks):
+            assert int(iters[h, p]) == its[p], (h, p)
+            assert np.array_equal(labels[h, p].cpu().numpy(), labs[p]), (h, p)
+            assert np.array_equal(cent[h, p, :k].cpu().numpy(), cents[p]), (h, p)
