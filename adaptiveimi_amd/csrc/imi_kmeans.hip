@@ -48,7 +48,9 @@ struct KmParams {
     float* prev;       // [seg][2] inertia of the last tested iteration
     int32_t* done;     // [seg] or null
     int32_t* iters;    // [seg] or null
-    void* ppstats;     // kmeans++ block statistics [seg][T / kPpRows] (init_mode 2)
+    void* ppstats;     // kmeans++ block statistics, two launches' (init_mode 2)
+    uint8_t* ppq;      // kmeans++ 8-bit copy and its norms, scales, error bounds (or null)
+    float *ppqn, *ppqs, *ppqe;
     int nblk;          // 256-token blocks
     int max_iters;
     float tol;
@@ -673,7 +675,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 
 // ---------------------------------------------------------------- kmeans++
 // kmeans_plusplus_init_inplace (kmeans_core.cpp:138-186) for every (head,
-// subspace) segment at once, two launches per pick.  The random draws do not
+// subspace) segment at once, one launch per pick.  The random draws do not
 // depend on the data: the host replays std::mt19937_64(seed) for the first
 // index (uniform_int_distribution<int32_t>(0, T-1)) and for one
 // generate_canonical<double, 53> per pick, which is what
@@ -682,191 +684,213 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 // total, then the running sum that picks the first index with cumsum >=
 // target).  When every value is a multiple of the smallest value's ulp and
 // the total stays below 2^53 such units (the exponent spread is checked per
-// pick), no partial sum rounds, so the sequential doubles equal exact
-// integer prefix sums, which any blocking of the rows reproduces; otherwise
-// one thread replays the sequential loops.
-//   km_pp_step_kernel  (launch c >= 1; blocks of kPpRows rows x segments):
-//                      pick c - 1 (the first row, or found from launch
-//                      c - 1's block statistics and minima), written by the
-//                      segment's block 0; then each row's min distance to
-//                      the picks 0..c-1, and the block's exponent range and
-//                      its sum in units of its own smallest exponent
-//   km_pp_pick_kernel  (one workgroup per segment): the last pick
-// Every block finds the pick itself (a few KB of statistics and one block's
-// minima), so no launch separates a pick from the next distance pass; the
-// minima and statistics alternate between two buffers for that reason.
-constexpr int kPpRPT = 4;                 // consecutive rows per thread
-constexpr int kPpRows = 256 * kPpRPT;     // rows per distance block
+// pick), no partial sum rounds in double, whatever the order, so blocked
+// sums equal the sequential ones; otherwise one thread replays the loops.
+//
+// Launch c >= 1 finds pick c - 1 (the first row, or from launch c - 1's block
+// statistics and minima; every workgroup does, on its first wave, while its
+// other loads are in flight), then updates each row's min distance to the
+// picks and its block's statistics.  Minima and statistics alternate between
+// two buffers, so launch c never overwrites what its own picks read.
+//
+//   km_pp_exact_kernel   the distance of every row: small inputs, which are
+//                        bound by the chain of dependent loads of a pick (6.4
+//                        us at 11k tokens, 8 segments; 13.1 us with the whole
+//                        workgroup searching), and launch 1 of larger ones,
+//                        which also makes an 8-bit copy of the rows
+//   km_pp_screen_kernel  the later launches: only rows whose 8-bit copy
+//                        cannot rule the new pick out get the distance
+//   km_pp_pick_kernel    the last pick
+//
+// 8-bit copy: groups of 256 rows share one scale s_j per dim (largest
+// magnitude / 127); x^ = s q.  With e >= |x - x^| over the group,
+//   |x - c| >= |x^ - c| - e,
+// so a row keeps its minimum m when |x^ - c| >= sqrt(m) + e.  |x^ - c|^2 =
+// |x^|^2 + |c|^2 - 2 x^.c; x^.c = sum q_j (s_j c_j) runs on v_dot4_i32_i8
+// against s_j c_j rounded to 16 bits (two 8-bit parts, exact integer sums, the
+// rounding at most W / 2 per dim bounded apart).  fp32 rounding (at most 2^-17
+// relative in the two norms, 2^-22 elsewhere, 2^-19 in the reference's
+// distance) is covered by 2^-14 of the operands' magnitudes, subnormal
+// effects by 1e-30; NaN, infinities and norms past 1e37 get the distance.
+// The copy is half of the keys' bytes; over 63 picks of the benchmark's keys
+// the rows that change are 3.3 passes in total and those the copy cannot rule
+// out 3.9.
+constexpr int kPpScreenBytes = 16 << 20;   // key bytes from which the rows are copied to 8 bits
+constexpr int64_t kPpCopyBytes = int64_t{4} << 30;   // largest copy
 
-struct PpBlock {                 // per (segment, block)
-    unsigned long long units;    // sum of its values in units of 2^(emin - 150)
-    int emin, emax;              // exponent range of its non-zero values (emin = INT_MAX: none)
+struct PpBlock {    // per (segment, block)
+    double sum;     // of its min distances (exact when the exponent spread allows)
+    int emin, emax; // exponent range of its non-zero values (emin = INT_MAX: none)
 };
-
-
-// value m in units of 2^(emin_eff - 150) (m a multiple of that unit when the
-// segment passes the exactness test; shifts past 63 only occur when it fails)
-__device__ __forceinline__ unsigned long long pp_units(float m, int emin_eff) {
-    const uint32_t u = __float_as_uint(m);
-    const int e = static_cast<int>((u >> 23) & 0xFFu);
-    const unsigned long long mant = static_cast<unsigned long long>(u & 0x7FFFFFu) | (e > 0 ? (1ull << 23) : 0ull);
-    const int sh = (e > 0 ? e : 1) - emin_eff;
-    return (mant == 0 || sh < 0 || sh > 63) ? 0ull : mant << sh;
-}
 
 __device__ __forceinline__ int pp_exp(float m) {
     const int e = static_cast<int>((__float_as_uint(m) >> 23) & 0xFFu);
     return e > 0 ? e : 1;
 }
 
-__device__ __forceinline__ int wave_min_i(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+// Exponent range of one non-negative value, into (emin, emax).
+__device__ __forceinline__ void pp_range(float m, int& emin, int& emax) {
+    if (m > 0.0f || m != m) {
+        const int e = pp_exp(m);
+        emin = min(emin, e);
+        emax = max(emax, e);
+    }
+}
+
+template <int CTRL, int ROW_MASK = 0xF>
+__device__ __forceinline__ double dpp_f64(double v) {   // 0.0 where the source is outside
+    const long long u = __double_as_longlong(v);
+    const uint32_t lo = static_cast<uint32_t>(dpp_i<CTRL, ROW_MASK>(static_cast<int>(u)));
+    const uint32_t hi = static_cast<uint32_t>(dpp_i<CTRL, ROW_MASK>(static_cast<int>(u >> 32)));
+    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+
+// Inclusive prefix sum across the 64 lanes.
+__device__ __forceinline__ double wave_incl_scan_f64(double v) {
+    v += dpp_f64<0x111>(v);
+    v += dpp_f64<0x112>(v);
+    v += dpp_f64<0x114>(v);
+    v += dpp_f64<0x118>(v);
+    v += dpp_f64<0x142, 0xA>(v);
+    v += dpp_f64<0x143, 0xC>(v);
     return v;
 }
 
-__device__ __forceinline__ long long wave_incl_scan_ll(long long v) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const long long y = __shfl_up(v, o);
-        if (lane_id() >= o) v += y;
-    }
-    return v;
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+    const long long u = __double_as_longlong(v);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), lane));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), lane));
+    return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
 }
 
-// 256-thread exclusive scan of one long long per thread; the total to all
-__device__ __forceinline__ long long block_excl_scan_ll(long long v, long long* sh, long long& total) {
-    const long long incl = wave_incl_scan_ll(v);
-    const int w = threadIdx.x >> 6;
-    if (lane_id() == 63) sh[w] = incl;
-    __syncthreads();
-    long long base = 0;
-    total = 0;
+// emin / emax over the wave (every lane): exponents are 1 .. 255.
+__device__ __forceinline__ int wave_emin(int e) {
+    const uint32_t inv = wave_max_u32(e == 0x7FFFFFFF ? 0u : 256u - static_cast<uint32_t>(e));
+    return inv == 0 ? 0x7FFFFFFF : 256 - static_cast<int>(inv);
+}
+__device__ __forceinline__ int wave_emax(int e) { return static_cast<int>(wave_max_u32(static_cast<uint32_t>(e))); }
+
+// First entry i (ascending) whose inclusive prefix base + v_0 + .. + v_i
+// reaches target, over n entries held PER per lane (lane l: entries PER l ..);
+// n - 1 if none does.  before: the exclusive prefix of that entry.
+template <int PER>
+__device__ __forceinline__ int pp_first_reaching(const double (&v)[PER], double base, double target, int n,
+                                                 double& before) {
+    double own = v[0];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (j < w) base += sh[j];
-        total += sh[j];
+    for (int u = 1; u < PER; ++u) own += v[u];
+    const double incl = wave_incl_scan_f64(own) + base;
+    const uint64_t hit = __ballot(incl >= target);
+    const int l = hit ? __builtin_ctzll(hit) : 63;
+    // every lane walks its own entries; lane l's walk is the answer
+    double run = incl - own, at = run;
+    int i = -1;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (i < 0 && run + v[u] >= target) {
+            i = u;
+            at = run;
+        }
+        run += v[u];
     }
-    __syncthreads();
-    return base + incl - v;
+    before = readlane_f64(at, l);
+    const int u = __builtin_amdgcn_readlane(i, l);
+    return hit && u >= 0 ? min(PER * l + u, n - 1) : n - 1;
 }
 
-typedef unsigned int __attribute__((ext_vector_type(4))) pp_u32x4_t;
-
-struct PpShared {
-    int e[2][4];
-    long long sc[4];
-    int blk, sel;
-    long long base;
-};
-
-// Row of pick c >= 1 of one segment (all 256 threads; the row to every
-// thread) from the minima md and block statistics st the distance pass of
-// pick c wrote: the segment's exponent range and, when every partial sum is
-// exact in double, the block and then the row whose integer prefix sum
-// reaches the target; otherwise thread 0 replays the reference's sequential
-// double sums (kmeans_core.cpp:160-181).
-__device__ int pp_pick_row(const float* md, const PpBlock* st, int nbp, int T, double canon, PpShared& sh) {
-    const int tid = threadIdx.x;
-    if (tid == 0) {
-        sh.blk = nbp;
-        sh.sel = T;
-    }
-    // this thread's consecutive blocks
-    const int per = (nbp + 255) / 256;
-    const int b0 = min(tid * per, nbp), b1 = min(b0 + per, nbp);
+// Row of pick c >= 1 of one segment (one wave; the row to every lane) from the
+// minima md and block statistics st of the distance pass of pick c: blocks of
+// 64 RPL rows.  kmeans_core.cpp:160-181.
+template <int RPL>
+__device__ int pp_pick_row(const float* md, const PpBlock* st, int nb, int T, double canon) {
+    const int lane = lane_id();
+    constexpr int SPER = 4;
+    const int per = (nb + 63) / 64;
     int emin = 0x7FFFFFFF, emax = 0;
-    for (int bb = b0; bb < b1; ++bb) {
-        emin = min(emin, st[bb].emin);
-        emax = max(emax, st[bb].emax);
+    double sums[SPER];
+#pragma unroll
+    for (int u = 0; u < SPER; ++u) sums[u] = 0.0;
+    if (per <= SPER) {
+        PpBlock e[SPER];
+#pragma unroll
+        for (int u = 0; u < SPER; ++u) e[u] = st[min(SPER * lane + u, nb - 1)];
+#pragma unroll
+        for (int u = 0; u < SPER; ++u)
+            if (SPER * lane + u < nb) {
+                sums[u] = e[u].sum;
+                emin = min(emin, e[u].emin);
+                emax = max(emax, e[u].emax);
+            }
+    } else {   // a run of `per` blocks per lane, searched again below
+        const int b1 = min((lane + 1) * per, nb);
+        for (int b = lane * per; b < b1; ++b) {
+            const PpBlock e = st[b];
+            sums[0] += e.sum;
+            emin = min(emin, e.emin);
+            emax = max(emax, e.emax);
+        }
     }
-    const int w = tid >> 6;
-    emin = wave_min_i(emin);
-    emax = wave_max_i(emax);
-    if (lane_id() == 0) {
-        sh.e[0][w] = emin;
-        sh.e[1][w] = emax;
-    }
-    __syncthreads();
-    const int e_lo = min(min(sh.e[0][0], sh.e[0][1]), min(sh.e[0][2], sh.e[0][3]));
-    const int e_hi = max(max(sh.e[1][0], sh.e[1][1]), max(sh.e[1][2], sh.e[1][3]));
+    emin = wave_emin(emin);
+    emax = wave_emax(emax);
     int logT = 0;
     while ((1ll << logT) < static_cast<long long>(T)) ++logT;
-    const bool any = e_lo != 0x7FFFFFFF;
-    const bool exact = !any || (e_hi - e_lo) + 24 + logT <= 53;
-    if (exact) {
-        const int emin_eff = any ? e_lo : 1;
-        long long mine = 0;
-        for (int bb = b0; bb < b1; ++bb)
-            if (st[bb].emin != 0x7FFFFFFF)
-                mine += static_cast<long long>(st[bb].units << (st[bb].emin - emin_eff));
-        long long total_u;
-        const long long base = block_excl_scan_ll(mine, sh.sc, total_u);
-        const double scale = ldexp(1.0, emin_eff - 150);
-        const double total = static_cast<double>(total_u) * scale;
-        const double target = canon * total + 0.0;
-        const double tu = target / scale;
-        // the first block whose inclusive prefix reaches the target
-        long long run = base;
-        for (int bb = b0; bb < b1; ++bb) {
-            const long long ub =
-                st[bb].emin != 0x7FFFFFFF ? static_cast<long long>(st[bb].units << (st[bb].emin - emin_eff)) : 0;
-            if (static_cast<double>(run + ub) >= tu) {
-                atomicMin(&sh.blk, bb);
-                break;
-            }
-            run += ub;
-        }
-        __syncthreads();
-        const int blk = sh.blk;
-        if (blk < nbp) {
-            // the exclusive prefix of that block, from the thread that holds it
-            if (blk >= b0 && blk < b1) {
-                long long r = base;
-                for (int bb = b0; bb < blk; ++bb)
-                    if (st[bb].emin != 0x7FFFFFFF)
-                        r += static_cast<long long>(st[bb].units << (st[bb].emin - emin_eff));
-                sh.base = r;
-            }
-            __syncthreads();
-            // rows of that block: kPpRPT consecutive rows per thread, as the distance pass
-            const int r0 = blk * kPpRows + tid * kPpRPT;
-            long long uj[kPpRPT];
-            long long ut = 0;
-#pragma unroll
-            for (int j = 0; j < kPpRPT; ++j) {
-                uj[j] = r0 + j < T ? static_cast<long long>(pp_units(md[r0 + j], emin_eff)) : 0;
-                ut += uj[j];
-            }
-            long long tot;
-            long long rr = sh.base + block_excl_scan_ll(ut, sh.sc, tot);
-#pragma unroll
-            for (int j = 0; j < kPpRPT; ++j) {
-                rr += uj[j];
-                if (r0 + j < T && static_cast<double>(rr) >= tu) {
-                    atomicMin(&sh.sel, r0 + j);
+    if (emin != 0x7FFFFFFF && (emax - emin) + 24 + logT > 53) {
+        int pick = 0;
+        if (lane == 0) {   // the sequential loops
+            double tw = 0.0;
+            for (int i = 0; i < T; ++i) tw += static_cast<double>(md[i]);
+            const double target = canon * tw + 0.0;
+            double cs = 0.0;
+            for (int i = 0; i < T; ++i) {
+                cs += static_cast<double>(md[i]);
+                if (cs >= target) {
+                    pick = i;
                     break;
                 }
             }
         }
-    } else if (tid == 0) {
-        double tw = 0.0;
-        for (int i = 0; i < T; ++i) tw += static_cast<double>(md[i]);
-        const double target = canon * tw + 0.0;
-        double cs = 0.0;
-        int pick = 0;
-        for (int i = 0; i < T; ++i) {
-            cs += static_cast<double>(md[i]);
-            if (cs >= target) {
-                pick = i;
+        return __builtin_amdgcn_readfirstlane(pick);
+    }
+    const double total = readlane_f64(wave_incl_scan_f64((sums[0] + sums[1]) + (sums[2] + sums[3])), 63);
+    const double target = canon * total + 0.0;
+    double base;
+    int blk;
+    if (per <= SPER) {
+        blk = pp_first_reaching<SPER>(sums, 0.0, target, nb, base);
+    } else {
+        const double one[1] = {sums[0]};
+        const int run = pp_first_reaching<1>(one, 0.0, target, 64, base);
+        blk = min(run * per, nb - 1);
+        for (int b0 = run * per; b0 < min((run + 1) * per, nb); b0 += 64) {   // one round up to 4096 blocks
+            const double v[1] = {b0 + lane < min((run + 1) * per, nb) ? st[b0 + lane].sum : 0.0};
+            const double all = readlane_f64(wave_incl_scan_f64(v[0]), 63);
+            if (base + all >= target) {
+                const double b = base;
+                blk = b0 + pp_first_reaching<1>(v, b, target, 64, base);
                 break;
             }
+            base += all;
         }
-        sh.sel = pick;
     }
-    __syncthreads();
-    return sh.sel < T ? sh.sel : 0;
+    // RPL consecutive rows per lane
+    typedef float __attribute__((ext_vector_type(4), aligned(4))) f4;
+    const int r0 = blk * 64 * RPL + lane * RPL;
+    double v[RPL];
+    if (r0 + RPL <= T) {
+        f4 m[RPL / 4];
+#pragma unroll
+        for (int u = 0; u < RPL / 4; ++u) m[u] = *reinterpret_cast<const f4*>(md + r0 + 4 * u);
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) v[u] = static_cast<double>(m[u / 4][u % 4]);
+    } else {
+#pragma unroll
+        for (int u = 0; u < RPL; ++u) v[u] = r0 + u < T ? static_cast<double>(md[r0 + u]) : 0.0;
+    }
+    const int rows = min(64 * RPL, T - blk * 64 * RPL);
+    return blk * 64 * RPL + pp_first_reaching<RPL>(v, base, target, rows, base);
 }
+
+typedef unsigned int __attribute__((ext_vector_type(4))) pp_u32x4_t;
 
 struct PpStep {
     int c;                       // launch index: pick c - 1, distances to it
@@ -878,151 +902,397 @@ struct PpStep {
     float* md_out;               // [seg][T]
     const PpBlock* st_in;        // [seg][nbp] statistics of launch c - 1
     PpBlock* st_out;
+    // the 8-bit copy by groups of 256 rows (RPT per block): [group][DP / 16][256]
+    // rows' 16-byte chunks, their norms [group][256], the group's scales
+    // [group][DP] and error bound [group]
+    pp_u32x4_t* q;
+    float* qn;
+    float* qs;
+    float* qe;
 };
 
-template <int DP>
-__global__ __launch_bounds__(256) void km_pp_step_kernel(KmParams a, PpStep ps) {
-    __shared__ __attribute__((aligned(16))) float cur[DP];
-    __shared__ int s_e[2][4];
-    __shared__ long long s_u[4];
-    __shared__ PpShared sh;
-    // one round of 256 rows at a padded stride
-    constexpr int CH = DP / 8;   // 16-byte chunks per row
-    extern __shared__ __attribute__((aligned(16))) pp_u32x4_t s_rows[];   // [256][CH + 1]
-    const int nb = ps.nbp, c = ps.c, nsub = ps.nsub;
-    const int seg = blockIdx.y, wb = blockIdx.x, tid = threadIdx.x;
-    const int h = seg / a.P, p = seg % a.P;
-    if (c - 1 >= a.k[p]) return;
-    const bool dist = c < a.k[p];   // false: pick c - 1 is the segment's last
-    if (!dist && wb != 0) return;
-    const int T = a.T;
-    const float* mdi = ps.md_in + static_cast<int64_t>(seg) * T;
-    float* mdo = ps.md_out + static_cast<int64_t>(seg) * T;
-    const uint16_t* xb = a.keys + static_cast<int64_t>(h) * a.hs + p * DP;
-    const int blk0 = wb * nsub, blk1 = min(blk0 + nsub, nb);
-    // Block bk: rows bk * kPpRows + 256 j + tid (j < kPpRPT) for the thread;
-    // each round of 256 rows is loaded coalesced (consecutive lanes read
-    // consecutive 16-byte chunks, so one wave instruction covers whole rows)
-    // and staged in LDS, from which each thread takes its own row.  The first
-    // block's previous minima and first round do not depend on the pick:
-    // they are loaded before it.
-    float prev[kPpRPT];
-    pp_u32x4_t ld[CH];
-    if (dist) {
-        const int r0 = blk0 * kPpRows;
-#pragma unroll
-        for (int j = 0; j < kPpRPT; ++j) {   // c == 1: no distances yet (FLT_MAX)
-            const int r = r0 + 256 * j + tid;
-            prev[j] = (c > 1 && r < T) ? mdi[r] : 3.402823466e38f;
-        }
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            const int f = tid + 256 * k, row = f / CH, ch = f % CH;
-            const int r = min(r0 + row, T - 1);
-            ld[k] = reinterpret_cast<const pp_u32x4_t*>(xb + static_cast<int64_t>(r) * a.ts)[ch];
-        }
-    }
+// The new pick's row: found by the first wave, widened into cur (LDS) and, by
+// the segment's first workgroup, written as a centroid.
+template <int DP, int RPL>
+__device__ __forceinline__ void pp_take_pick(const KmParams& a, const PpStep& ps, int seg, int p, const uint16_t* xb,
+                                             float* cur) {
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x, c = ps.c;
     const int sel = c == 1 ? ps.first[p]
-                           : pp_pick_row(mdi, ps.st_in + static_cast<int64_t>(seg) * nb, nb, T, ps.canon[p], sh);
-    if (tid < CH) {
-        const pp_u32x4_t v = reinterpret_cast<const pp_u32x4_t*>(xb + static_cast<int64_t>(sel) * a.ts)[tid];
+                           : pp_pick_row<RPL>(ps.md_in + static_cast<int64_t>(seg) * a.T,
+                                              ps.st_in + static_cast<int64_t>(seg) * ps.nbp, ps.nbp, a.T, ps.canon[p]);
+    if (lane < DP / 8) {
+        const pp_u32x4_t v = reinterpret_cast<const pp_u32x4_t*>(xb + static_cast<int64_t>(sel) * a.ts)[lane];
         const float4 f0 = make_float4(bf16_lo(v.x), bf16_hi(v.x), bf16_lo(v.y), bf16_hi(v.y));
         const float4 f1 = make_float4(bf16_lo(v.z), bf16_hi(v.z), bf16_lo(v.w), bf16_hi(v.w));
-        reinterpret_cast<float4*>(cur)[2 * tid] = f0;
-        reinterpret_cast<float4*>(cur)[2 * tid + 1] = f1;
-        if (wb == 0) {
+        reinterpret_cast<float4*>(cur)[2 * lane] = f0;
+        reinterpret_cast<float4*>(cur)[2 * lane + 1] = f1;
+        if (blockIdx.x == 0) {
             float4* dst = reinterpret_cast<float4*>(a.cent + (static_cast<int64_t>(seg) * a.kmax + c - 1) * DP);
-            dst[2 * tid] = f0;
-            dst[2 * tid + 1] = f1;
-        }
-    }
-    if (!dist) return;
-    const int w = tid >> 6;
-    for (int bk = blk0; bk < blk1; ++bk) {
-        const int r0 = bk * kPpRows;
-        if (bk > blk0) {
-#pragma unroll
-            for (int j = 0; j < kPpRPT; ++j) {
-                const int r = r0 + 256 * j + tid;
-                prev[j] = (c > 1 && r < T) ? mdi[r] : 3.402823466e38f;
-            }
-        }
-        float m[kPpRPT];
-        int emin = 0x7FFFFFFF, emax = 0;
-#pragma unroll
-        for (int j = 0; j < kPpRPT; ++j) {
-            if (j > 0 || bk > blk0) {
-#pragma unroll
-                for (int k = 0; k < CH; ++k) {
-                    const int f = tid + 256 * k, row = f / CH, ch = f % CH;
-                    const int r = min(r0 + 256 * j + row, T - 1);
-                    ld[k] = reinterpret_cast<const pp_u32x4_t*>(xb + static_cast<int64_t>(r) * a.ts)[ch];
-                }
-                __syncthreads();   // the previous round's rows are read
-            }
-#pragma unroll
-            for (int k = 0; k < CH; ++k) {
-                const int f = tid + 256 * k, row = f / CH, ch = f % CH;
-                s_rows[row * (CH + 1) + ch] = ld[k];
-            }
-            __syncthreads();   // (and cur, before the first round)
-            pp_u32x4_t v[CH];
-#pragma unroll
-            for (int k = 0; k < CH; ++k) v[k] = s_rows[tid * (CH + 1) + k];
-            const int r = r0 + 256 * j + tid;
-            const float d = l2_lanes8_bf16<DP>(v, cur);
-            float mm = prev[j];
-            if (d < mm) mm = d;
-            m[j] = r < T ? mm : 0.0f;
-            if (r < T) mdo[r] = mm;
-            if (m[j] > 0.0f) {
-                emin = min(emin, pp_exp(m[j]));
-                emax = max(emax, pp_exp(m[j]));
-            }
-        }
-        emin = wave_min_i(emin);
-        emax = wave_max_i(emax);
-        if (lane_id() == 0) {
-            s_e[0][w] = emin;
-            s_e[1][w] = emax;
-        }
-        __syncthreads();
-        const int be = min(min(s_e[0][0], s_e[0][1]), min(s_e[0][2], s_e[0][3]));
-        const int bx = max(max(s_e[1][0], s_e[1][1]), max(s_e[1][2], s_e[1][3]));
-        unsigned long long u = 0;
-        if (be != 0x7FFFFFFF) {
-#pragma unroll
-            for (int j = 0; j < kPpRPT; ++j) u += pp_units(m[j], be);
-        }
-        const long long us = wave_incl_scan_ll(static_cast<long long>(u));
-        if (lane_id() == 63) s_u[w] = us;
-        __syncthreads();
-        if (tid == 0) {
-            PpBlock o;
-            o.units = static_cast<unsigned long long>(((s_u[0] + s_u[1]) + s_u[2]) + s_u[3]);
-            o.emin = be;
-            o.emax = bx;
-            ps.st_out[static_cast<int64_t>(seg) * nb + bk] = o;
+            dst[2 * lane] = f0;
+            dst[2 * lane + 1] = f1;
         }
     }
 }
 
+// Statistics of a block from its waves' (all 256 threads; one barrier).
+__device__ __forceinline__ void pp_block_stats(double sum, int emin, int emax, PpBlock* sh, PpBlock* out) {
+    const int w = threadIdx.x >> 6;
+    const double s = readlane_f64(wave_incl_scan_f64(sum), 63);
+    emin = wave_emin(emin);
+    emax = wave_emax(emax);
+    if (lane_id() == 0) sh[w] = PpBlock{s, emin, emax};
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        PpBlock o = sh[0];
+        for (int i = 1; i < 4; ++i) {
+            o.sum += sh[i].sum;
+            o.emin = min(o.emin, sh[i].emin);
+            o.emax = max(o.emax, sh[i].emax);
+        }
+        *out = o;
+    }
+}
+
+// Rows are loaded coalesced (consecutive lanes read consecutive 16-byte
+// chunks) and staged in LDS, from which each thread takes its own row.  RPT =
+// 0: blocks of 256 rows; else launch 1 of the screened form, blocks of RPT
+// such groups, whose 8-bit copy it writes.
+template <int DP, int RPT>
+__global__ __launch_bounds__(256) void km_pp_exact_kernel(KmParams a, PpStep ps) {
+    constexpr bool FIRST = RPT > 0;
+    __shared__ __attribute__((aligned(16))) float cur[DP];
+    __shared__ PpBlock s_st[2][4];
+    __shared__ float s_part[FIRST ? 512 : 1];
+    __shared__ __attribute__((aligned(16))) float s_scale[FIRST ? DP : 4];
+    __shared__ __attribute__((aligned(16))) float s_inv[FIRST ? DP : 4];
+    __shared__ float s_err[4];
+    constexpr int CH = DP / 8;   // 16-byte chunks per row
+    constexpr int GROUPS = FIRST ? RPT : 1;
+    extern __shared__ __attribute__((aligned(16))) pp_u32x4_t s_rows[];   // [256][CH + 1]
+    const int nb = ps.nbp, c = ps.c;
+    const int seg = blockIdx.y, tid = threadIdx.x;
+    const int h = seg / a.P, p = seg % a.P;
+    if (c - 1 >= a.k[p]) return;
+    const bool dist = c < a.k[p];   // false: pick c - 1 is the segment's last
+    if (!dist && blockIdx.x != 0) return;
+    const int T = a.T;
+    const float* mdi = ps.md_in + static_cast<int64_t>(seg) * T;
+    float* mdo = ps.md_out + static_cast<int64_t>(seg) * T;
+    const uint16_t* xb = a.keys + static_cast<int64_t>(h) * a.hs + p * DP;
+    const int blk0 = blockIdx.x * ps.nsub, blk1 = min(blk0 + ps.nsub, nb);
+    // the first group does not depend on the pick: it is loaded before it
+    pp_u32x4_t ld[CH];
+    float prev = kFltMax;   // launch 1: no distances yet
+    auto load_group = [&](int r0) {
+        if (c > 1) prev = mdi[min(r0 + tid, T - 1)];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const int f = tid + 256 * i;
+            ld[i] = reinterpret_cast<const pp_u32x4_t*>(xb + static_cast<int64_t>(min(r0 + f / CH, T - 1)) * a.ts)[f % CH];
+        }
+    };
+    if (dist) load_group(blk0 * 256 * GROUPS);
+    pp_take_pick<DP, 4 * GROUPS>(a, ps, seg, p, xb, cur);
+    if (!dist) return;
+    for (int bk = blk0; bk < blk1; ++bk) {
+        double sum = 0.0;
+        int emin = 0x7FFFFFFF, emax = 0;
+#pragma unroll 1
+        for (int g = 0; g < GROUPS; ++g) {
+            const int r0 = (bk * GROUPS + g) * 256;
+            if (bk > blk0 || g > 0) {
+                load_group(r0);
+                __syncthreads();   // the previous group's rows are read
+            }
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+                const int f = tid + 256 * i;
+                s_rows[(f / CH) * (CH + 1) + f % CH] = ld[i];
+            }
+            __syncthreads();   // (and cur, before the first group)
+            pp_u32x4_t v[CH];
+#pragma unroll
+            for (int i = 0; i < CH; ++i) v[i] = s_rows[tid * (CH + 1) + i];
+            const int r = r0 + tid;
+            const float d = l2_lanes8_bf16<DP>(v, cur);
+            const float m = r < T ? (d < prev ? d : prev) : 0.0f;
+            if (r < T) mdo[r] = m;
+            sum += static_cast<double>(m);
+            pp_range(m, emin, emax);
+            if constexpr (FIRST) {
+                // largest magnitude per dim: a dword column (two dims) per
+                // thread over 256 / PARTS of the group's rows
+                constexpr int COLS = DP / 2, PARTS = 256 / COLS;
+                const uint32_t* words = reinterpret_cast<const uint32_t*>(s_rows);
+                const int col = tid % COLS, part = tid / COLS;
+                uint32_t lo = 0, hi = 0;   // |bf16| bits order like the values
+                const int n = min(256, T - r0);
+                for (int i = part * (256 / PARTS); i < (part + 1) * (256 / PARTS) && i < n; ++i) {
+                    const uint32_t w = words[i * 4 * (CH + 1) + col] & 0x7FFF7FFFu;
+                    lo = max(lo, w & 0xFFFFu);
+                    hi = max(hi, w >> 16);
+                }
+                s_part[part * DP + 2 * col] = __uint_as_float(lo << 16);
+                s_part[part * DP + 2 * col + 1] = __uint_as_float(hi << 16);
+                __syncthreads();
+                const int64_t group = (static_cast<int64_t>(seg) * nb + bk) * RPT + g;
+                if (tid < DP) {
+                    float m4 = 0.0f;   // (a NaN's bits give a NaN here, an infinity an infinite scale)
+                    for (int i = 0; i < PARTS; ++i) m4 = s_part[i * DP + tid] > m4 || s_part[i * DP + tid] != s_part[i * DP + tid] ? s_part[i * DP + tid] : m4;
+                    const float sc = m4 * (1.0f / 127.0f);
+                    s_scale[tid] = sc;
+                    s_inv[tid] = sc > 0.0f ? 1.0f / sc : 0.0f;
+                    ps.qs[group * DP + tid] = sc;
+                }
+                __syncthreads();
+                float nrm = 0.0f, err = 0.0f;
+#pragma unroll
+                for (int i = 0; i < DP / 16; ++i) {
+                    pp_u32x4_t o;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {   // four dims per dword
+                        const uint32_t x01 = v[2 * i + w / 2][2 * (w % 2)], x23 = v[2 * i + w / 2][2 * (w % 2) + 1];
+                        const float x[4] = {bf16_lo(x01), bf16_hi(x01), bf16_lo(x23), bf16_hi(x23)};
+                        uint32_t b = 0;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int j = 16 * i + 4 * w + e;
+                            const float t = fminf(fmaxf(rintf(x[e] * s_inv[j]), -127.0f), 127.0f);
+                            const float xh = t * s_scale[j];
+                            nrm = __builtin_fmaf(xh, xh, nrm);
+                            err = __builtin_fmaf(x[e] - xh, x[e] - xh, err);
+                            b |= (static_cast<uint32_t>(static_cast<int>(t)) & 0xFFu) << (8 * e);
+                        }
+                        o[w] = b;
+                    }
+                    ps.q[(group * (DP / 16) + i) * 256 + tid] = o;
+                }
+                ps.qn[group * 256 + tid] = nrm;
+                // error bound of the group's rows; a non-finite one rules nothing out
+                float e = r < T ? sqrtf(err) * (1.0f + 0x1p-14f) + 1e-30f : 0.0f;
+                e = e <= 1e30f ? e : INFINITY;
+                e = wave_max(e);
+                if (lane_id() == 0) s_err[tid >> 6] = e;
+                __syncthreads();
+                if (tid == 0) ps.qe[group] = fmaxf(fmaxf(s_err[0], s_err[1]), fmaxf(s_err[2], s_err[3]));
+            }
+        }
+        pp_block_stats(sum, emin, emax, s_st[(bk - blk0) & 1], ps.st_out + static_cast<int64_t>(seg) * nb + bk);
+    }
+}
+
+// Launch c >= 2 of the screened form, over blocks of RPT groups of 256 rows.  A
+// wave screens RPT rows per lane of one group (RPT = 4: group `wave` of the
+// block; RPT = 1: a quarter of its only group, for inputs that would otherwise
+// leave CUs idle): it weighs the group's scales with the pick, screens,
+// queues the rows it cannot rule out and computes their distances 8 lanes per
+// row (lane part j sums dims j, j + 8, .., the reference's lane j; row shifts
+// add the eight sums left to right).  Only the block statistics cross waves.
+//
+// Bound by the copy's bytes (76 per 64-dim row with norm and minima) for large
+// inputs, by the pick's dependent loads for small ones.  Per pick, 64 dims,
+// 16 segments: 33.3 us at 128k tokens (55 us reading the keys), 147 us at 512k
+// (250 us).  Two of the four rows
+// loaded at a time keep four waves per SIMD (36.4 us with all four and three
+// waves); the next block's loads are issued before the queue.
+template <int DP, int RPT>
+__global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(KmParams a, PpStep ps) {
+    constexpr int CH = DP / 16;                   // 16-byte chunks per copied row
+    constexpr int LR = RPT < 2 || DP < 64 ? RPT : 2;   // rows per thread loaded together
+    constexpr int DL = DP > 64 ? DP / 64 : 1;     // dims per lane of the weights
+    __shared__ __attribute__((aligned(16))) float cur[DP];
+    __shared__ PpBlock s_st[2][4];
+    __shared__ __attribute__((aligned(16))) uint8_t s_w[4][2][DP];   // per wave: high and low weight bytes
+    __shared__ uint16_t s_queue[4][64 * RPT];
+    __shared__ float s_dist[4][64 * RPT];
+    const int nb = ps.nbp, c = ps.c;
+    const int seg = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int h = seg / a.P, p = seg % a.P;
+    if (c - 1 >= a.k[p]) return;
+    const bool dist = c < a.k[p];
+    if (!dist && blockIdx.x != 0) return;
+    const int T = a.T;
+    const float* mdi = ps.md_in + static_cast<int64_t>(seg) * T;
+    float* mdo = ps.md_out + static_cast<int64_t>(seg) * T;
+    const uint16_t* xb = a.keys + static_cast<int64_t>(h) * a.hs + p * DP;
+    const int blk0 = blockIdx.x * ps.nsub, blk1 = min(blk0 + ps.nsub, nb);
+    pp_u32x4_t q[LR][CH];
+    float m[RPT], nrm[RPT], sc[DL], err;
+    // the wave's group of block bk, its first row there and in the segment
+    const int g_in = RPT == 4 ? wave : 0, row_in = RPT == 4 ? 0 : 64 * wave;
+    static_assert(RPT == 4 || RPT == 1, "groups per block");
+    auto group_of = [&](int bk) { return (static_cast<int64_t>(seg) * nb + bk) * RPT + g_in; };
+    auto row_of = [&](int bk) { return (bk * RPT + g_in) * 256 + row_in; };
+    auto load_rows = [&](int64_t group, int i0) {
+#pragma unroll
+        for (int i = 0; i < LR; ++i)
+#pragma unroll
+            for (int k = 0; k < CH; ++k) q[i][k] = ps.q[(group * CH + k) * 256 + row_in + 64 * (i0 + i) + lane];
+    };
+    auto load_group = [&](int bk) {
+        const int64_t group = group_of(bk);
+        const int r0 = row_of(bk);
+#pragma unroll
+        for (int u = 0; u < DL; ++u) sc[u] = ps.qs[group * DP + (64 * u + lane) % DP];
+        err = ps.qe[group];
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            m[i] = mdi[min(r0 + 64 * i + lane, T - 1)];
+            nrm[i] = ps.qn[group * 256 + row_in + 64 * i + lane];
+        }
+        load_rows(group, 0);
+    };
+    if (dist) load_group(blk0);   // does not depend on the pick
+    pp_take_pick<DP, 4 * RPT>(a, ps, seg, p, xb, cur);
+    if (!dist) return;
+    __syncthreads();
+    float cj[DL], cc = 0.0f;   // the pick's dims of this lane, |c|^2
+#pragma unroll
+    for (int u = 0; u < DL; ++u) {
+        cj[u] = cur[(64 * u + lane) % DP];
+        cc = __builtin_fmaf(cj[u], cj[u], cc);
+    }
+    cc = wave_sum(DP < 64 && lane >= DP ? 0.0f : cc);
+    float cp[DP / 8];   // dims part, part + 8, .. for the distances
+#pragma unroll
+    for (int i = 0; i < DP / 8; ++i) cp[i] = cur[8 * i + (lane & 7)];
+#pragma unroll 1
+    for (int bk = blk0; bk < blk1; ++bk) {
+        const int64_t group = group_of(bk);
+        const int r0 = row_of(bk);
+        // 16-bit weights s_j c_j / W in two signed bytes
+        float wj[DL], wmax = 0.0f;
+#pragma unroll
+        for (int u = 0; u < DL; ++u) {
+            wj[u] = sc[u] * cj[u];
+            wmax = fmaxf(wmax, fabsf(wj[u]));
+        }
+        wmax = wave_max(wmax);
+        const float W = wmax * (1.0f / 32512.0f), iw = wmax > 0.0f ? 32512.0f / wmax : 0.0f;
+#pragma unroll
+        for (int u = 0; u < DL; ++u) {
+            if (DP >= 64 || lane < DP) {
+                const int t = static_cast<int>(fminf(fmaxf(rintf(wj[u] * iw), -32512.0f), 32512.0f));
+                const int hi = (t + 128) >> 8;
+                s_w[wave][0][64 * u + lane] = static_cast<uint8_t>(hi);
+                s_w[wave][1][64 * u + lane] = static_cast<uint8_t>(t - 256 * hi);
+            }
+        }
+        km_wave_lds_sync();
+        // the weights' rounding: at most W (1/2 + 2^-8) per dim times |q| <= 127, twice
+        const float slack = 130.0f * DP * W + 0x1p-14f * cc + 1e-30f;
+        uint32_t need = 0;
+#pragma unroll
+        for (int i0 = 0; i0 < RPT; i0 += LR) {
+            if (i0 > 0) load_rows(group, i0);
+            int hi[LR], lo[LR];
+#pragma unroll
+            for (int i = 0; i < LR; ++i) hi[i] = lo[i] = 0;
+#pragma unroll
+            for (int k = 0; k < CH; ++k) {
+                const pp_u32x4_t wh = *reinterpret_cast<const pp_u32x4_t*>(&s_w[wave][0][16 * k]);
+                const pp_u32x4_t wl = *reinterpret_cast<const pp_u32x4_t*>(&s_w[wave][1][16 * k]);
+#pragma unroll
+                for (int i = 0; i < LR; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        hi[i] = __builtin_amdgcn_sdot4(static_cast<int>(q[i][k][e]), static_cast<int>(wh[e]), hi[i], false);
+                        lo[i] = __builtin_amdgcn_sdot4(static_cast<int>(q[i][k][e]), static_cast<int>(wl[e]), lo[i], false);
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < LR; ++i) {
+                const float dot = W * static_cast<float>(256 * hi[i] + lo[i]);
+                const float n = nrm[i0 + i];
+                const float low = (n + cc) - 2.0f * dot - (slack + 0x1p-14f * n);
+                const float reach = (__builtin_amdgcn_sqrtf(m[i0 + i]) + err) * (1.0f + 0x1p-14f);
+                const bool in = r0 + 64 * (i0 + i) + lane < T;
+                // (norms past 1e37 could overflow where the distance does not)
+                const bool out = low >= reach * reach && n + cc <= 1e37f;
+                if (in && m[i0 + i] != 0.0f && !out) need |= 1u << (i0 + i);
+            }
+        }
+        // the next block's loads overlap with the queue's
+        float mc[RPT];
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) mc[i] = m[i];
+        if (bk + 1 < blk1) load_group(bk + 1);
+        // the queue: this wave's rows in (i, lane) order
+        int nq = 0;
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            const bool in = (need >> i) & 1u;
+            const uint64_t bal = __ballot(in);
+            if (in) s_queue[wave][nq + __popcll(bal & lanemask_lt())] = static_cast<uint16_t>(64 * i + lane);
+            nq += __popcll(bal);
+        }
+        km_wave_lds_sync();
+#pragma unroll 1
+        for (int e0 = 0; e0 < nq; e0 += 16) {   // 16 rows, two per 8 lanes
+            int id[2];
+            uint16_t xv[2][DP / 8];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                id[u] = s_queue[wave][min(e0 + 8 * u + (lane >> 3), nq - 1)];
+                const uint16_t* row = xb + static_cast<int64_t>(r0 + id[u]) * a.ts + (lane & 7);
+#pragma unroll
+                for (int i = 0; i < DP / 8; ++i) xv[u][i] = row[8 * i];
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float acc = 0.0f;
+#pragma unroll
+                for (int i = 0; i < DP / 8; ++i) {
+                    const float d = bf16_to_f32(xv[u][i]) - cp[i];
+                    acc = __builtin_fmaf(d, d, acc);
+                }
+                float d = acc;
+                d = d + dpp_row_shl<1>(acc);
+                d = d + dpp_row_shl<2>(acc);
+                d = d + dpp_row_shl<3>(acc);
+                d = d + dpp_row_shl<4>(acc);
+                d = d + dpp_row_shl<5>(acc);
+                d = d + dpp_row_shl<6>(acc);
+                d = d + dpp_row_shl<7>(acc);
+                if ((lane & 7) == 0) s_dist[wave][id[u]] = d;
+            }
+        }
+        km_wave_lds_sync();
+        double sum = 0.0;
+        int emin = 0x7FFFFFFF, emax = 0;
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            const int r = r0 + 64 * i + lane;
+            float v = mc[i];
+            if ((need >> i) & 1u) {
+                const float d = s_dist[wave][64 * i + lane];
+                if (d < v) v = d;
+            }
+            if (r < T) {
+                mdo[r] = v;
+                sum += static_cast<double>(v);
+                pp_range(v, emin, emax);
+            }
+        }
+        pp_block_stats(sum, emin, emax, s_st[(bk - blk0) & 1], ps.st_out + static_cast<int64_t>(seg) * nb + bk);
+    }
+}
+
 // The last pick c of every segment with k == c + 1 (c == 0: the first row)
-// from the minima and statistics of launch c.
-template <int DP>
-__global__ __launch_bounds__(256) void km_pp_pick_kernel(KmParams a, PpStep ps) {
-    __shared__ PpShared sh;
-    const int seg = blockIdx.x, tid = threadIdx.x;
+// from the minima and statistics of launch c (blocks of 64 RPL rows).
+template <int DP, int RPL>
+__global__ __launch_bounds__(64) void km_pp_pick_kernel(KmParams a, PpStep ps) {
+    const int seg = blockIdx.x, lane = threadIdx.x;
     const int h = seg / a.P, p = seg % a.P;
     const int c = ps.c;
     if (c >= a.k[p]) return;
-    const int T = a.T, nb = ps.nbp;
     const uint16_t* xb = a.keys + static_cast<int64_t>(h) * a.hs + p * DP;
     const int sel = c == 0 ? ps.first[p]
-                           : pp_pick_row(ps.md_in + static_cast<int64_t>(seg) * T,
-                                         ps.st_in + static_cast<int64_t>(seg) * nb, nb, T, ps.canon[p], sh);
+                           : pp_pick_row<RPL>(ps.md_in + static_cast<int64_t>(seg) * a.T,
+                                              ps.st_in + static_cast<int64_t>(seg) * ps.nbp, ps.nbp, a.T, ps.canon[p]);
     float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + c) * DP;
-    for (int d = tid; d < DP; d += 256) dst[d] = bf16_to_f32(xb[static_cast<int64_t>(sel) * a.ts + d]);
+    for (int d = lane; d < DP; d += 64) dst[d] = bf16_to_f32(xb[static_cast<int64_t>(sel) * a.ts + d]);
 }
 
 // Early stop (kmeans_core.cpp:244-262) of one segment.  The inertia has a fixed
@@ -1632,6 +1902,102 @@ void superblocks(int T, int segs, int& sbt, int& nsb) {
     nsb = static_cast<int>((static_cast<int64_t>(T) + sbt - 1) / sbt);
 }
 
+// Whether kmeans++ screens its rows over an 8-bit copy: from 16 MB of keys
+// (below, a pick is bound by its dependent loads and the copy would not pay;
+// 8k tokens, 16 segments) while the copy stays below 4 GB.
+bool pp_screened(int T, int segs, int dp) {
+    const int64_t elems = static_cast<int64_t>(T) * segs * dp;
+    return 2 * elems >= kPpScreenBytes && elems <= kPpCopyBytes;
+}
+
+// Groups of 256 rows per block of the screened passes: four, but one while
+// blocks of four would be fewer than kPpFewBlocks (two workgroups per CU): 8
+// heads of 16k tokens over 128 dims (128 blocks of four) take 7.1 us per pick
+// with one group, 9.1 us with four and 17.5 us reading the keys; 40k tokens
+// over 64 dims, 16 segments (640 blocks) 16.2, 15.1 and 22 us.
+constexpr int kPpFewBlocks = 512;
+int pp_groups(int T, int segs) {
+    return static_cast<int64_t>((T + 1023) / 1024) * segs >= kPpFewBlocks ? 4 : 1;
+}
+
+template <int DP, int RPT>
+int run_plusplus(const KmParams& p, const imi_kmeans_args* a, int segs, hipStream_t stream) {
+    // kmeans++ seeds 42, 43, 44, 45 by subspace, the same for every head
+    // (kmeans_core.cpp:459, 469; IVF: seed 42, kmeans_core.cpp:548-556)
+    PpStep ps{};
+    std::vector<double> canon[4];
+    for (int part = 0; part < a->parts; ++part) {
+        std::mt19937_64 rng(static_cast<uint64_t>(42 + part));
+        std::uniform_int_distribution<int32_t> first(0, a->n_tokens - 1);
+        ps.first[part] = first(rng);
+        canon[part].assign(a->k[part], 0.0);
+        for (int c = 1; c < a->k[part]; ++c)
+            canon[part][c] = std::generate_canonical<double, std::numeric_limits<double>::digits>(rng);
+    }
+    constexpr bool screened = RPT > 0;
+    const int rows = screened ? 256 * RPT : 256;
+    const int nbp = (p.T + rows - 1) / rows;
+    ps.nbp = nbp;
+    ps.q = reinterpret_cast<pp_u32x4_t*>(p.ppq);
+    ps.qn = p.ppqn;
+    ps.qs = p.ppqs;
+    ps.qe = p.ppqe;
+    PpBlock* st = static_cast<PpBlock*>(p.ppstats);
+    // minima and statistics alternate between two buffers (one of them the
+    // member lists' `sorted`, free until the first M-step)
+    float* md[2] = {p.ppmd, reinterpret_cast<float*>(p.sorted)};
+    PpBlock* sts[2] = {st, st + static_cast<size_t>(segs) * nbp};
+    const size_t lds = static_cast<size_t>(256) * (DP / 8 + 1) * 16;
+    // one resident round of workgroups, each over nsub consecutive blocks
+    const auto sub_blocks = [&](const void* fn, size_t dyn) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, dyn) != hipSuccess || per_cu <= 0) per_cu = 1;
+        const int64_t want = static_cast<int64_t>(per_cu) * device_cus();
+        return static_cast<int>(std::max<int64_t>(1, (static_cast<int64_t>(nbp) * segs + want - 1) / want));
+    };
+    const void* exact_fn = reinterpret_cast<const void*>(&km_pp_exact_kernel<DP, RPT>);
+    if (DP == 128)   // 68 KB of LDS per workgroup
+        IMI_HIP_CHECK(hipFuncSetAttribute(exact_fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    const int sub_first = sub_blocks(exact_fn, lds);
+    int sub_next = sub_first;
+    if constexpr (screened) sub_next = sub_blocks(reinterpret_cast<const void*>(&km_pp_screen_kernel<DP, RPT>), 0);
+    // launch c (1 <= c < kmax): pick c - 1 and the distances to it
+    for (int c = 1; c < p.kmax; ++c) {
+        ps.c = c;
+        for (int part = 0; part < a->parts; ++part)
+            ps.canon[part] = c - 1 >= 1 && c - 1 < a->k[part] ? canon[part][c - 1] : 0.0;
+        ps.md_in = md[(c - 1) & 1];
+        ps.md_out = md[c & 1];
+        ps.st_in = sts[(c - 1) & 1];
+        ps.st_out = sts[c & 1];
+        ps.nsub = c == 1 ? sub_first : sub_next;
+        const dim3 grid((nbp + ps.nsub - 1) / ps.nsub, segs);
+        if (!screened || c == 1)
+            hipLaunchKernelGGL((km_pp_exact_kernel<DP, RPT>), grid, dim3(256), lds, stream, p, ps);
+        else if constexpr (screened)
+            hipLaunchKernelGGL((km_pp_screen_kernel<DP, RPT>), grid, dim3(256), 0, stream, p, ps);
+        IMI_LAUNCH_CHECK("kmeans++ pass");
+    }
+    // the last pick of the segments with kmax centroids
+    const int c = p.kmax - 1;
+    ps.c = c;
+    for (int part = 0; part < a->parts; ++part) ps.canon[part] = c >= 1 && c < a->k[part] ? canon[part][c] : 0.0;
+    ps.md_in = md[c & 1];
+    ps.st_in = sts[c & 1];
+    ps.md_out = nullptr;
+    ps.st_out = nullptr;
+    hipLaunchKernelGGL((km_pp_pick_kernel<DP, screened ? 4 * RPT : 4>), dim3(segs), dim3(64), 0, stream, p, ps);
+    IMI_LAUNCH_CHECK("km_pp_pick_kernel");
+    return IMI_OK;
+}
+
+template <int DP>
+int seed_plusplus(const KmParams& p, const imi_kmeans_args* a, int segs, int groups, hipStream_t stream) {
+    return groups == 4   ? run_plusplus<DP, 4>(p, a, segs, stream)
+           : groups == 1 ? run_plusplus<DP, 1>(p, a, segs, stream)
+                         : run_plusplus<DP, 0>(p, a, segs, stream);
+}
+
 size_t workspace_bytes(const imi_kmeans_args* a, int kmax, KmParams* out) {
     const int segs = a->kv_heads * a->parts;
     const int nblk = (a->n_tokens + 255) / 256;
@@ -1645,9 +2011,18 @@ size_t workspace_bytes(const imi_kmeans_args* a, int kmax, KmParams* out) {
     p.prev = cv.take<float>(2 * segs);
     p.done = cv.take<int32_t>(segs);
     if (a->init_mode == 2) {
-        const int nbp = (a->n_tokens + kPpRows - 1) / kPpRows;
-        p.ppstats = cv.take<PpBlock>(static_cast<size_t>(2) * segs * nbp);   // two launches' worth
+        const int dp = a->dim / a->parts;
+        const bool screened = pp_screened(a->n_tokens, segs, dp);
+        const size_t rows = 256 * (screened ? pp_groups(a->n_tokens, segs) : 1);   // per block
+        const size_t blocks = (a->n_tokens + rows - 1) / rows * segs;
+        p.ppstats = cv.take<PpBlock>(2 * blocks);   // two launches' worth
         p.ppmd = cv.take<float>(static_cast<size_t>(segs) * a->n_tokens);
+        if (screened) {
+            p.ppq = cv.take<uint8_t>(blocks * rows * dp);
+            p.ppqn = cv.take<float>(blocks * rows);
+            p.ppqs = cv.take<float>(blocks * rows / 256 * dp);
+            p.ppqe = cv.take<float>(blocks * rows / 256);
+        }
     }
     if (out) *out = p;
     return cv.used();
@@ -1802,73 +2177,11 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
         hipLaunchKernelGGL(km_init_first_kernel, dim3(kmax, segs), dim3(64), 0, stream, p);
         IMI_LAUNCH_CHECK("km_init_first_kernel");
     } else if (a->init_mode == 2) {
-        // kmeans++ seeds 42, 43, 44, 45 by subspace, the same for every head
-        // (kmeans_core.cpp:459, 469; IVF: seed 42, kmeans_core.cpp:548-556);
-        // every segment's pick c in one pair of launches
-        PpStep ps{};
-        std::vector<double> canon[4];
-        for (int part = 0; part < a->parts; ++part) {
-            std::mt19937_64 rng(static_cast<uint64_t>(42 + part));
-            std::uniform_int_distribution<int32_t> first(0, a->n_tokens - 1);
-            ps.first[part] = first(rng);
-            canon[part].assign(a->k[part], 0.0);
-            for (int c = 1; c < a->k[part]; ++c)
-                canon[part][c] = std::generate_canonical<double, std::numeric_limits<double>::digits>(rng);
-        }
-        const int nbp = (a->n_tokens + kPpRows - 1) / kPpRows;
-        ps.nbp = nbp;
-        PpBlock* st = static_cast<PpBlock*>(p.ppstats);
-        // minima and statistics alternate between two buffers (one of them
-        // the member lists' `sorted`, free until the first M-step)
-        float* md[2] = {p.ppmd, reinterpret_cast<float*>(p.sorted)};
-        PpBlock* sts[2] = {st, st + static_cast<size_t>(segs) * nbp};
-        const size_t lds = static_cast<size_t>(256) * (dp / 8 + 1) * 16;
-        if (dp == 128)   // 68 KB of LDS per workgroup
-            IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_pp_step_kernel<128>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-        // one resident round of workgroups, each over nsub consecutive blocks
-        int per_cu = 0;
-        const void* fn = dp == 128 ? reinterpret_cast<const void*>(&km_pp_step_kernel<128>)
-                                   : (dp == 64 ? reinterpret_cast<const void*>(&km_pp_step_kernel<64>)
-                                               : reinterpret_cast<const void*>(&km_pp_step_kernel<32>));
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, lds) != hipSuccess || per_cu <= 0)
-            per_cu = 1;
-        const int64_t want = static_cast<int64_t>(per_cu) * device_cus();
-        ps.nsub = static_cast<int>(std::max<int64_t>(1, (static_cast<int64_t>(nbp) * segs + want - 1) / want));
-        const int nbw = (nbp + ps.nsub - 1) / ps.nsub;
-        // launch c (1 <= c < kmax): pick c - 1 and the distances to it
-        for (int c = 1; c < kmax; ++c) {
-            ps.c = c;
-            for (int part = 0; part < a->parts; ++part)
-                ps.canon[part] = c - 1 >= 1 && c - 1 < a->k[part] ? canon[part][c - 1] : 0.0;
-            ps.md_in = md[(c - 1) & 1];
-            ps.md_out = md[c & 1];
-            ps.st_in = sts[(c - 1) & 1];
-            ps.st_out = sts[c & 1];
-            const dim3 grid(nbw, segs);
-            if (dp == 128)
-                hipLaunchKernelGGL(km_pp_step_kernel<128>, grid, dim3(256), lds, stream, p, ps);
-            else if (dp == 64)
-                hipLaunchKernelGGL(km_pp_step_kernel<64>, grid, dim3(256), lds, stream, p, ps);
-            else
-                hipLaunchKernelGGL(km_pp_step_kernel<32>, grid, dim3(256), lds, stream, p, ps);
-            IMI_LAUNCH_CHECK("km_pp_step_kernel");
-        }
-        // the last pick of the segments with kmax centroids
-        const int c = kmax - 1;
-        ps.c = c;
-        for (int part = 0; part < a->parts; ++part) ps.canon[part] = c >= 1 && c < a->k[part] ? canon[part][c] : 0.0;
-        ps.md_in = md[c & 1];
-        ps.st_in = sts[c & 1];
-        ps.md_out = nullptr;
-        ps.st_out = nullptr;
-        if (dp == 128)
-            hipLaunchKernelGGL(km_pp_pick_kernel<128>, dim3(segs), dim3(256), 0, stream, p, ps);
-        else if (dp == 64)
-            hipLaunchKernelGGL(km_pp_pick_kernel<64>, dim3(segs), dim3(256), 0, stream, p, ps);
-        else
-            hipLaunchKernelGGL(km_pp_pick_kernel<32>, dim3(segs), dim3(256), 0, stream, p, ps);
-        IMI_LAUNCH_CHECK("km_pp_pick_kernel");
+        const int groups = pp_screened(a->n_tokens, segs, dp) ? pp_groups(a->n_tokens, segs) : 0;
+        rc = dp == 128 ? seed_plusplus<128>(p, a, segs, groups, stream)
+                       : (dp == 64 ? seed_plusplus<64>(p, a, segs, groups, stream)
+                                   : seed_plusplus<32>(p, a, segs, groups, stream));
+        if (rc) return rc;
     }
     for (int it = 0; it < a->max_iters; ++it) {
         // the inertia of iteration it enters the stop tests of it and it + 1

@@ -90,3 +90,44 @@ def test_lloyd_over_superblock_edges(oracle, H, T, ks, stop):
             assert int(iters[h, p]) == its[p], (h, p)
             assert np.array_equal(labels[h, p].cpu().numpy(), labs[p]), (h, p)
             assert np.array_equal(cent[h, p, :k].cpu().numpy(), cents[p]), (h, p)
+
+
+def _awkward(keys, form):
+    """Rows on which the 8-bit copy's bound is poor or degenerate."""
+    k = keys.float()
+    if form == "outliers":      # one huge row and one huge channel
+        k[:, 1234] *= 3000.0
+        k[:, :, 5] *= 500.0
+    elif form == "duplicates":  # 40 distinct rows: minima fall to zero
+        k = k[:, torch.arange(k.shape[1]) % 40]
+    elif form == "huge":
+        k *= 2.0 ** 60
+    elif form == "tiny":
+        k *= 2.0 ** -70
+    elif form == "zero":        # a whole group of zero rows
+        k[:, 256:1300] = 0.0
+    return k.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("H,T,ks,form", [
+    (8, 9001, (37, 20), ""), (8, 8193, (9, 9), "outliers"), (8, 9000, (45, 45), "duplicates"), (8, 8999, (12, 5), "huge"),
+    (8, 9000, (6, 6), "tiny"), (8, 10240, (8, 30), "zero"), (1, 70001, (16, 3), ""), (8, 9000, (17, 2, 30, 1), ""),
+    (8, 9007, (11, 11, 11, 11), "outliers"), (8, 8300, (70,), ""), (8, 9000, (20,), "outliers"), (1, 300100, (9, 4), ""),
+    (2, 4100, (33, 64), ""), (2, 257, (20, 1), ""), (1, 255, (64,), "duplicates")])
+def test_plusplus_screened_rows(oracle, H, T, ks, form):
+    """kmeans++ picks with the rows screened over their 8-bit copy (16 MB of
+    keys and more: 64, 32 and 128 dims, ragged blocks, more blocks than one
+    search round) and below: one Lloyd iteration from the seeds equals the
+    oracle's, so every pick does."""
+    from adaptiveimi_amd import ops, synthetic
+
+    print(f"[kmeans++] H={H} T={T} ks={ks} {form}", flush=True)
+    keys, _ = synthetic.make_kv(H, T, seed=T)
+    keys = _awkward(keys, form)
+    cent, labels, _ = ops.kmeans(keys.to(DEV), list(ks), 1, init="kmeans++")
+    kf = oracle.bf16_to_f32(_bits(keys))
+    for h in ([0, H - 1] if H > 1 else [0]):
+        labs, cents, _ = oracle.kmeans_head(kf[h], list(ks), 1, init="kmeans++")
+        for p, k in enumerate(ks):
+            assert np.array_equal(labels[h, p].cpu().numpy(), labs[p]), (h, p)
+            assert np.array_equal(cent[h, p, :k].cpu().numpy(), cents[p]), (h, p)
