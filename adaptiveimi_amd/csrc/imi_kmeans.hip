@@ -436,31 +436,74 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
             }
         };
         number_from(0);
-        // the 16 centroids of packed slot `slot`
-        auto screen_tile = [&](int slot) {
-            km_u32x4_t ah[KH], al[KH];
-#pragma unroll
-            for (int kh = 0; kh < KH; ++kh) {
-                ah[kh] = apk[((slot * KH + kh) * 2 + 0) * 64 + lane];
-                al[kh] = apk[((slot * KH + kh) * 2 + 1) * 64 + lane];
-            }
+        // f of the 16 centroids of packed slot `slot`, and the largest three with it
+        typedef km_f32x4_t Acc[4];
+        auto products = [&](int slot, Acc& acc) {
             const km_f32x4_t init = *reinterpret_cast<const km_f32x4_t*>(cch + slot * 16 + 4 * grp);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                km_f32x4_t acc = init;
+            for (int j = 0; j < 4; ++j) acc[j] = init;
 #pragma unroll
-                for (int kh = 0; kh < KH; ++kh) {
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, ah[kh]),
-                                                                  __builtin_bit_cast(km_bf16x8_t, bq[j][kh]), acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(km_bf16x8_t, al[kh]),
-                                                                  __builtin_bit_cast(km_bf16x8_t, bq[j][kh]), acc, 0, 0, 0);
+            for (int kh = 0; kh < KH; ++kh)
+#pragma unroll
+                for (int part = 0; part < 2; ++part) {
+                    const km_bf16x8_t c =
+                        __builtin_bit_cast(km_bf16x8_t, apk[((slot * KH + kh) * 2 + part) * 64 + lane]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c, __builtin_bit_cast(km_bf16x8_t, bq[j][kh]),
+                                                                         acc[j], 0, 0, 0);
                 }
+        };
+        auto largest = [&](const Acc& acc) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    top[j].add(__uint_as_float((__float_as_uint(acc[r]) & idx_mask) | num[r]));
-            }
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    top[j].add(__uint_as_float((__float_as_uint(acc[j][r]) & idx_mask) | num[r]));
 #pragma unroll
             for (int r = 0; r < 4; ++r) num[r] += 16;
+        };
+        // `n` tiles from slot s0 on: a tile's products run beside the comparisons
+        // of the tile before (one matrix operation, then its share of VALU; 59.4
+        // against 62.7 us at k = 64, 128k tokens, 485 against 501 at k = 181, 512k)
+        auto overlap = [&]() {
+#pragma unroll
+            for (int i = 0; i < 8 * KH; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            }
+        };
+        auto screen_tiles = [&](int s0, int n) {
+            Acc x, y;
+            // (128 dims: the tokens take the registers of a second tile; 32 dims:
+            // measured slower, 144 against 135 us for the 4-way index at 256k)
+            if (DP != 64) {
+#pragma unroll 1
+                for (int i = 0; i < n; ++i) {
+                    products(s0 + i, x);
+                    largest(x);
+                }
+                return;
+            }
+            products(s0, x);
+            int i = 1;
+#pragma unroll 1
+            for (; i + 1 < n; i += 2) {
+                products(s0 + i, y);
+                largest(x);
+                overlap();
+                products(s0 + i + 1, x);
+                largest(y);
+                overlap();
+            }
+            if (i < n) {
+                products(s0 + i, y);
+                largest(x);
+                overlap();
+                largest(y);
+            } else {
+                largest(x);
+            }
         };
         int chb[4] = {0, 0, 0, 0}, chs[4] = {0, 0, 0, 0};   // chunks of best and second (STREAM)
         if constexpr (STREAM) {
@@ -484,8 +527,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
                     ps[j] = top[j].s;
                 }
                 number_from(0);
-#pragma unroll 1
-                for (int i = 0; i < kChunkTiles; ++i) screen_tile((q & 1) * kChunkTiles + i);
+                screen_tiles((q & 1) * kChunkTiles, kChunkTiles);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     if (top[j].s != ps[j]) chs[j] = top[j].s == pb[j] ? chb[j] : q;
@@ -496,8 +538,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
             }
             if (blk == blk0) ccmax = reduce_ccmax(s_cc);
         } else {
-#pragma unroll 1
-            for (int ct = 0; ct < nct; ++ct) screen_tile(ct);
+            screen_tiles(0, nct);
         }
         // |x|^2: each lane has its quarter of every tile's dims
         float xs[4];
@@ -508,9 +549,9 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
             for (int kh = 0; kh < KH; ++kh)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float x0 = bf16_lo(bq[j][kh][i]), x1 = bf16_hi(bq[j][kh][i]);
-                    xs[j] = __builtin_fmaf(x0, x0, xs[j]);
-                    xs[j] = __builtin_fmaf(x1, x1, xs[j]);
+                    typedef __attribute__((ext_vector_type(2))) __bf16 b2;
+                    const b2 x2 = __builtin_bit_cast(b2, static_cast<uint32_t>(bq[j][kh][i]));
+                    xs[j] = __builtin_amdgcn_fdot2_f32_bf16(x2, x2, xs[j], false);
                 }
         }
         // row g of the wave ends with tile g: halves exchange tiles (0, 2) and
