@@ -11,7 +11,9 @@
 // The cell order is produced by an LSD sort with one stable counting pass per
 // subspace label (last subspace first), which yields tokens ordered by
 // (l0, l1, ..., token) = (global cell id, token): the reference's CSR order,
-// because compact ids are ranks of global ids.  IVF (one subspace, the
+// because compact ids are ranks of global ids.  The first pass reads every
+// label once, in token order, and carries each token's global cell id along,
+// so the later passes read sequentially too (no gathers by token).  IVF (one subspace, the
 // cluster label is the cell id; build_compact_reorg_input_ivf, 178-231) is
 // the one-pass case.
 #include "imi_common.hpp"
@@ -25,60 +27,133 @@ struct IxParams {
     int H, T, P, kmax;
     int k[4];
     int64_t ncells;
-    int nblk;
-    int32_t* hist;   // [H][kmax][nblk]
-    int32_t* rank;   // [H][T]
+    int sbt, nsb;    // tokens per superblock, superblocks per head
+    int32_t* hist;   // [H][k][nsb] digit counts of a pass, then places
     int32_t* cid;    // [H][ncells] compact id scratch
     int32_t* sums;   // [H][nchunk][2] per-chunk row and occupied totals
 };
 
-__host__ __device__ inline int bits_for(int n) {
-    int b = 0;
-    while ((1 << b) < n) ++b;
-    return b;
-}
-
 constexpr int kIvfMaxK = 4096;   // IVF clusters per head
 
-template <int NB>
-__global__ __launch_bounds__(256) void ix_rank_kernel(IxParams a, int p, const int32_t* in) {
-    __shared__ int wcnt[4 * NB];
-    const int h = blockIdx.y, blk = blockIdx.x;
-    const int pos = blk * 256 + threadIdx.x;
-    const bool valid = pos < a.T;
-    const int64_t hT = static_cast<int64_t>(h) * a.T;
-    int digit = 0;
-    if (valid) {
-        const int item = in ? in[hT + pos] : pos;
-        digit = a.labels[(static_cast<int64_t>(h) * a.P + p) * a.T + item];
-    }
-    const int r = block_digit_rank(digit, valid, a.k[p], bits_for(a.k[p]), wcnt,
-                                   a.hist + static_cast<int64_t>(h) * a.kmax * a.nblk, a.nblk, blk);
-    if (valid) a.rank[hT + pos] = r;
+// One LSD pass: items in the order of the pass before (token and cell id;
+// null in the first pass, where item i is token i), sorted by the label of
+// subspace p.  The label is (cell / div) % k with exact 32-bit division:
+// mulhi by ceil(2^32 / d) is the quotient or one above it for cells < 2^26.
+struct IxPass {
+    int p;
+    const int32_t* tok;
+    const int32_t* cell;
+    int32_t* tok_out;
+    int32_t* cell_out;
+    uint32_t div, div_magic;   // product of the k after subspace p
+    uint32_t k, k_magic;
+    bool stage;                // the slice is staged in LDS (place_lds_bytes)
+};
+
+__device__ __forceinline__ uint32_t quot(uint32_t n, uint32_t d, uint32_t magic) {
+    if (d == 1) return n;
+    const uint32_t q = __umulhi(n, magic);
+    return q * d > n ? q - 1 : q;
 }
 
-__global__ __launch_bounds__(1024) void ix_scan_kernel(IxParams a, int p) {
+// The pass's digit of item i of head h.
+__device__ __forceinline__ int pass_digit(const IxParams& a, const IxPass& s, int h, int64_t i) {
+    if (s.cell == nullptr) return a.labels[(static_cast<int64_t>(h) * a.P + s.p) * a.T + i];
+    const uint32_t q = quot(static_cast<uint32_t>(s.cell[static_cast<int64_t>(h) * a.T + i]), s.div, s.div_magic);
+    return static_cast<int>(q - quot(q, s.k, s.k_magic) * s.k);
+}
+
+// A pass is three launches: digit counts of each superblock, an exclusive scan
+// of them in (digit, superblock) order, and the places.  What bounds it is the
+// latency of one superblock's loads and LDS rounds up to 128k tokens, and past
+// that the scattered writes.  Superblocks of 1024 .. 8192 items keep the scan
+// short (at 256 items per histogram, one workgroup per head scanned 2k values
+// per 512 tokens) and write each digit's items in runs; carrying the cell id
+// makes every read sequential.  Measured per pass against per-256 histograms
+// with labels gathered by token: 8 x 128k tokens, k = 90: 4.6 + 4.1 + 16.9 us
+// (was 10.2 + 14.9 + 11.4); 8 x 1M: 10 + 6.5 + 89 us (was 85 + 210 + 104); the
+// scan of 8 x 512k at k = 256: 4.7 us (was 180).  All passes of a short head on
+// one workgroup, one launch in place of six, took longer: 35 us against 29 at
+// 8k tokens.
+
+// Digit counts of each superblock.
+__global__ __launch_bounds__(1024) void ix_hist_kernel(IxParams a, IxPass s) {
+    extern __shared__ int smem_i[];
+    const int h = blockIdx.y, sb = blockIdx.x, k = static_cast<int>(s.k);
+    for (int c = threadIdx.x; c < k; c += blockDim.x) smem_i[c] = 0;
+    __syncthreads();
+    const int base = sb * a.sbt, m = min(a.sbt, a.T - base);
+    for (int i0 = 0; i0 < m; i0 += 4 * blockDim.x) {
+        int d[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            d[u] = pass_digit(a, s, h, base + min(i0 + u * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x), m - 1));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i0 + u * blockDim.x + threadIdx.x < m) atomicAdd(&smem_i[d[u]], 1);
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < k; c += blockDim.x)
+        a.hist[(static_cast<int64_t>(h) * k + c) * a.nsb + sb] = smem_i[c];
+}
+
+__global__ __launch_bounds__(1024) void ix_scan_kernel(IxParams a, int k) {
     __shared__ int sh[40];
     const int h = blockIdx.x;
-    block_exclusive_scan_1024(a.hist + static_cast<int64_t>(h) * a.kmax * a.nblk,
-                              static_cast<int64_t>(a.k[p]) * a.nblk, sh);
+    block_exclusive_scan_1024(a.hist + static_cast<int64_t>(h) * k * a.nsb, static_cast<int64_t>(k) * a.nsb, sh);
 }
 
-__global__ __launch_bounds__(256) void ix_scatter_kernel(IxParams a, int p, const int32_t* in, int32_t* out) {
-    const int h = blockIdx.y, blk = blockIdx.x;
-    const int pos = blk * 256 + threadIdx.x;
-    if (pos >= a.T) return;
+// Places of each superblock's items: its slice in digit order, each digit's
+// run at its scanned place.  Staged in LDS, so that each digit's run is written
+// together, where the slice fits (always up to 4M tokens per head).
+inline size_t place_lds_bytes(int waves, int k, int sbt, bool stage) {
+    return (static_cast<size_t>(waves + 2) * k + 32) * sizeof(int) + (stage ? 4 * static_cast<size_t>(sbt) : 0);
+}
+
+__global__ __launch_bounds__(1024) void ix_place_kernel(IxParams a, IxPass s) {
+    extern __shared__ int smem_i[];
+    const int k = static_cast<int>(s.k);
+    int* cnt = smem_i;                              // [waves][k]
+    int* first = cnt + (blockDim.x >> 6) * k;       // [k] first place in the slice
+    int* dst = first + k;                           // [k] first place in the output
+    int* wsum = dst + k;                            // [16]
+    uint16_t* item = reinterpret_cast<uint16_t*>(wsum + 32);   // [sbt]
+    uint16_t* dig = item + a.sbt;                              // [sbt]
+    const bool stage = s.stage;
+    const int h = blockIdx.y, sb = blockIdx.x;
+    const int base = sb * a.sbt, m = min(a.sbt, a.T - base);
     const int64_t hT = static_cast<int64_t>(h) * a.T;
-    const int item = in ? in[hT + pos] : pos;
-    const int digit = a.labels[(static_cast<int64_t>(h) * a.P + p) * a.T + item];
-    const int dst = a.hist[(static_cast<int64_t>(h) * a.kmax + digit) * a.nblk + blk] + a.rank[hT + pos];
-    out[hT + dst] = item;
-}
-
-__device__ __forceinline__ int64_t cell_of(const IxParams& a, int h, int t) {
-    int64_t g = 0;
-    for (int p = 0; p < a.P; ++p) g = g * a.k[p] + a.labels[(static_cast<int64_t>(h) * a.P + p) * a.T + t];
-    return g;
+    for (int c = threadIdx.x; c < k; c += blockDim.x) dst[c] = a.hist[(static_cast<int64_t>(h) * k + c) * a.nsb + sb];
+    const auto write = [&](int i, int64_t to) {   // local item i
+        const int64_t at = hT + base + i;
+        int cell = 0;
+        if (s.cell) {
+            cell = s.cell[at];
+        } else {
+            for (int p = 0; p < a.P; ++p) cell = cell * a.k[p] + a.labels[(static_cast<int64_t>(h) * a.P + p) * a.T + base + i];
+        }
+        s.tok_out[hT + to] = s.tok ? s.tok[at] : base + i;
+        s.cell_out[hT + to] = cell;
+    };
+    // (its first barrier also publishes dst)
+    superblock_sort(
+        m, a.sbt, k, cnt, wsum, [&](int i) { return pass_digit(a, s, h, base + i); },
+        [&](int c, int f) { first[c] = f; },
+        [&](int i, int at) {
+            const int d = pass_digit(a, s, h, base + i);
+            if (stage) {
+                item[at] = static_cast<uint16_t>(i);
+                dig[at] = static_cast<uint16_t>(d);
+            } else {
+                write(i, dst[d] + (at - first[d]));
+            }
+        });
+    if (!stage) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < m; i += blockDim.x) {
+        const int d = dig[i];
+        write(item[i], dst[d] + (i - first[d]));
+    }
 }
 
 __global__ void ix_zero_kernel(int32_t* x, int64_t n) {
@@ -87,15 +162,16 @@ __global__ void ix_zero_kernel(int32_t* x, int64_t n) {
         x[i] = 0;
 }
 
-// Cell counts over the tokens in cell order (perm = the stable cell sort):
-// equal cells are contiguous, so each wave adds one count per run of equal
-// cells (one atomic per run instead of one per token).
-__global__ __launch_bounds__(256) void ix_count_kernel(IxParams a, const int32_t* perm, int32_t* count) {
+// Cell counts over the sorted cell ids: equal cells are contiguous, so each
+// wave adds one count per run of equal cells (one atomic per run instead of
+// one per token).  Reading sorted ids: 16 us at 8 x 1M tokens, 160 when each
+// token's labels were gathered in cell order.
+__global__ __launch_bounds__(256) void ix_count_kernel(IxParams a, const int32_t* cells, int32_t* count) {
     const int h = blockIdx.y;
     const int i = blockIdx.x * 256 + threadIdx.x;
     const int lane = lane_id();
-    const int64_t c = i < a.T ? cell_of(a, h, perm[static_cast<int64_t>(h) * a.T + i]) : -1;
-    const int64_t cp = __shfl(c, lane > 0 ? lane - 1 : 0);
+    const int c = i < a.T ? cells[static_cast<int64_t>(h) * a.T + i] : -1;
+    const int cp = __shfl(c, lane > 0 ? lane - 1 : 0);
     const uint64_t starts = __builtin_amdgcn_ballot_w64(lane == 0 || c != cp);
     if (c >= 0 && (lane == 0 || c != cp)) {
         const uint64_t after = lane < 63 ? starts >> (lane + 1) : 0ull;
@@ -366,19 +442,26 @@ int validate(const imi_index_args* a, int& kmax, int64_t& ncells) {
     return IMI_OK;
 }
 
-size_t workspace_bytes(const imi_index_args* a, int kmax, int64_t ncells, IxParams* p, int32_t** tmp) {
-    const int nblk = (a->n_tokens + 255) / 256;
+// tmp: the second token order and the two cell orders of the LSD passes
+size_t workspace_bytes(const imi_index_args* a, int kmax, int64_t ncells, IxParams* p, int32_t* (*tmp)[3]) {
+    const size_t items = static_cast<size_t>(a->kv_heads) * a->n_tokens;
     Carver cv(a->workspace);
     IxParams q{};
-    q.hist = cv.take<int32_t>(static_cast<size_t>(a->kv_heads) * kmax * nblk);
-    q.rank = cv.take<int32_t>(static_cast<size_t>(a->kv_heads) * a->n_tokens);
+    superblocks(a->n_tokens, a->kv_heads, q.sbt, q.nsb);
+    q.hist = cv.take<int32_t>(static_cast<size_t>(a->kv_heads) * kmax * q.nsb);
     q.cid = cv.take<int32_t>(static_cast<size_t>(a->kv_heads) * ncells);
     q.sums = cv.take<int32_t>(static_cast<size_t>(a->kv_heads) * 2 * ((ncells + kOffCells - 1) / kOffCells));
-    int32_t* t = cv.take<int32_t>(static_cast<size_t>(a->kv_heads) * a->n_tokens);
+    int32_t* t[3];
+    t[0] = cv.take<int32_t>(a->parts > 1 ? items : 1);
+    t[1] = cv.take<int32_t>(items);
+    t[2] = cv.take<int32_t>(a->parts > 1 ? items : 1);
     if (p) *p = q;
-    if (tmp) *tmp = t;
+    if (tmp)
+        for (int i = 0; i < 3; ++i) (*tmp)[i] = t[i];
     return cv.used();
 }
+
+uint32_t magic(uint32_t d) { return d > 1 ? static_cast<uint32_t>((uint64_t{1} << 32) / d + ((uint64_t{1} << 32) % d != 0)) : 0u; }
 
 }  // namespace
 }  // namespace imi
@@ -411,8 +494,8 @@ extern "C" int imi_build_index(const imi_index_args* a, imi_stream_t stream_) {
     IMI_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= need, IMI_ERR_WORKSPACE,
                 "imi_build_index: workspace %zu bytes < %zu required", a->workspace_bytes, need);
     IxParams p;
-    int32_t* scratch;
-    workspace_bytes(a, kmax, ncells, &p, &scratch);
+    int32_t* tmp_items[3];
+    workspace_bytes(a, kmax, ncells, &p, &tmp_items);
     p.labels = a->labels;
     p.H = a->kv_heads;
     p.T = a->n_tokens;
@@ -420,32 +503,44 @@ extern "C" int imi_build_index(const imi_index_args* a, imi_stream_t stream_) {
     p.kmax = kmax;
     for (int i = 0; i < 4; ++i) p.k[i] = i < a->parts ? a->k[i] : 1;
     p.ncells = ncells;
-    p.nblk = (a->n_tokens + 255) / 256;
     const bool compact = a->compact_gid != nullptr;
     if (!compact) p.cid = nullptr;
 
-    // LSD passes: last subspace first; the final pass lands in a->perm.
-    const int32_t* in = nullptr;
-    for (int pass = 0; pass < a->parts; ++pass) {
-        const int part = a->parts - 1 - pass;
-        int32_t* out = ((a->parts - 1 - pass) % 2 == 0) ? a->perm : scratch;
-        if (a->k[part] <= 256)
-            hipLaunchKernelGGL(ix_rank_kernel<256>, dim3(p.nblk, p.H), dim3(256), 0, stream, p, part, in);
-        else
-            hipLaunchKernelGGL(ix_rank_kernel<kIvfMaxK>, dim3(p.nblk, p.H), dim3(256), 0, stream, p, part, in);
-        IMI_LAUNCH_CHECK("ix_rank_kernel");
-        hipLaunchKernelGGL(ix_scan_kernel, dim3(p.H), dim3(1024), 0, stream, p, part);
+    // LSD passes: last subspace first; the final pass lands in a->perm and
+    // tmp_items[1] (the sorted cell ids).
+    IxPass s{};
+    const int waves = sort_waves(kmax);
+    s.stage = p.sbt <= kStagedItems && place_lds_bytes(waves, kmax, p.sbt, true) <= 150 * 1024;
+    const size_t lds = place_lds_bytes(waves, kmax, p.sbt, s.stage);
+    if (lds > 64 * 1024)
+        IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&ix_place_kernel),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    uint32_t div = 1;
+    for (int part = a->parts - 1; part >= 0; --part) {
+        s.p = part;
+        s.tok = s.tok_out;
+        s.cell = s.cell_out;
+        s.tok_out = part % 2 == 0 ? a->perm : tmp_items[0];
+        s.cell_out = part % 2 == 0 ? tmp_items[1] : tmp_items[2];
+        s.k = static_cast<uint32_t>(a->k[part]);
+        s.div = div;
+        s.div_magic = magic(s.div);
+        s.k_magic = magic(s.k);
+        div *= s.k;
+        hipLaunchKernelGGL(ix_hist_kernel, dim3(p.nsb, p.H), dim3(64 * waves), s.k * sizeof(int), stream, p, s);
+        IMI_LAUNCH_CHECK("ix_hist_kernel");
+        hipLaunchKernelGGL(ix_scan_kernel, dim3(p.H), dim3(1024), 0, stream, p, static_cast<int>(s.k));
         IMI_LAUNCH_CHECK("ix_scan_kernel");
-        hipLaunchKernelGGL(ix_scatter_kernel, dim3(p.nblk, p.H), dim3(256), 0, stream, p, part, in, out);
-        IMI_LAUNCH_CHECK("ix_scatter_kernel");
-        in = out;
+        hipLaunchKernelGGL(ix_place_kernel, dim3(p.nsb, p.H), dim3(64 * waves), lds, stream, p, s);
+        IMI_LAUNCH_CHECK("ix_place_kernel");
     }
 
     const int64_t cells_total = ncells * p.H;
     hipLaunchKernelGGL(ix_zero_kernel, dim3(static_cast<unsigned>((cells_total + 255) / 256 < 65535 ? (cells_total + 255) / 256 : 65535)),
                        dim3(256), 0, stream, a->cell_count, cells_total);
     IMI_LAUNCH_CHECK("ix_zero_kernel");
-    hipLaunchKernelGGL(ix_count_kernel, dim3(p.nblk, p.H), dim3(256), 0, stream, p, a->perm, a->cell_count);
+    hipLaunchKernelGGL(ix_count_kernel, dim3((a->n_tokens + 255) / 256, p.H), dim3(256), 0, stream, p, tmp_items[1],
+                       a->cell_count);
     IMI_LAUNCH_CHECK("ix_count_kernel");
     const int nchunk = static_cast<int>((ncells + kOffCells - 1) / kOffCells);
     hipLaunchKernelGGL(ix_chunk_sums_kernel, dim3(nchunk, p.H), dim3(256), 0, stream, p, a->cell_count, p.sums,

@@ -92,14 +92,7 @@ struct Draws {
 };
 
 constexpr int kDraws = 256;      // empty-cluster draws one launch carries
-constexpr int kMaxSuper = 512;   // superblocks of the member lists
 constexpr int kIvfMaxK = 4096;   // IVF clusters per head
-
-__host__ __device__ inline int bits_for(int n) {
-    int b = 0;
-    while ((1 << b) < n) ++b;
-    return b;
-}
 
 __global__ __launch_bounds__(64) void km_init_first_kernel(KmParams a) {
     const int c = blockIdx.x, seg = blockIdx.y;
@@ -187,14 +180,6 @@ typedef __attribute__((ext_vector_type(4))) unsigned int km_u32x4_t;
 typedef __attribute__((ext_vector_type(2))) unsigned int km_u32x2_t;
 typedef __attribute__((ext_vector_type(4))) short km_s16x4_t;
 typedef __attribute__((address_space(3))) km_s16x4_t km_lds_s16x4_t;
-
-// Intra-wave LDS hand-off (compiler ordering only; a wave's LDS instructions
-// execute in order).
-__device__ __forceinline__ void km_wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 constexpr float kFltMax = 3.402823466e38f;
 constexpr int kChunkTiles = 4;   // 16-centroid tiles per streamed chunk
@@ -1220,7 +1205,7 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
                 s_w[wave][1][64 * u + lane] = static_cast<uint8_t>(t - 256 * hi);
             }
         }
-        km_wave_lds_sync();
+        wave_lds_order();
         // the weights' rounding: at most W (1/2 + 2^-8) per dim times |q| <= 127, twice
         const float slack = 130.0f * DP * W + 0x1p-14f * cc + 1e-30f;
         uint32_t need = 0;
@@ -1268,7 +1253,7 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
             if (in) s_queue[wave][nq + __popcll(bal & lanemask_lt())] = static_cast<uint16_t>(64 * i + lane);
             nq += __popcll(bal);
         }
-        km_wave_lds_sync();
+        wave_lds_order();
 #pragma unroll 1
         for (int e0 = 0; e0 < nq; e0 += 16) {   // 16 rows, two per 8 lanes
             int id[2];
@@ -1299,7 +1284,7 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
                 if ((lane & 7) == 0) s_dist[wave][id[u]] = d;
             }
         }
-        km_wave_lds_sync();
+        wave_lds_order();
         double sum = 0.0;
         int emin = 0x7FFFFFFF, emax = 0;
 #pragma unroll
@@ -1385,98 +1370,43 @@ __global__ __launch_bounds__(1024) void km_stop_kernel(KmParams a, int it) {
 // Member lists by superblocks of a.sbt tokens: each workgroup puts its
 // tokens in label order (ascending token inside a label) into its own slice
 // of `sorted` and writes the superblock's row of label offsets (loff[0 .. k]:
-// first place of each label, then the token count).  A stable counting sort:
-// label counts per wave (a wave owns consecutive tokens), one scan over
-// (label, wave), then every round of 64 tokens takes its places from the
-// wave's running offsets.  The ordered slice goes through LDS (coalesced
-// stores) up to kStagedTokens tokens.  11.6 us at 128k tokens, 16 segments;
-// superblocks of thousands of tokens keep the M-step's member search and its
-// column of label offsets short (62 us per M-step, 68 us with one row of
-// offsets per 256 tokens), and serve any T (a scan over per-block histograms
-// and a scatter took 340 us at 512k tokens, k = 181; this kernel 34 us).
-constexpr int kStagedTokens = 32768;
-
+// first place of each label, then the token count).  The ordered slice goes
+// through LDS (coalesced stores) up to kStagedItems tokens.  11.6 us at 128k
+// tokens, 16 segments; superblocks of thousands of tokens keep the M-step's
+// member search and its column of label offsets short (62 us per M-step, 68 us
+// with one row of offsets per 256 tokens), and serve any T (a scan over
+// per-block histograms and a scatter took 340 us at 512k tokens, k = 181; this
+// kernel 34 us).
 __host__ __device__ inline size_t members_lds_bytes(int waves, int kmax, int sbt) {
-    return (static_cast<size_t>(waves) * kmax + 32) * sizeof(int) + (sbt <= kStagedTokens ? 2 * static_cast<size_t>(sbt) : 0);
+    return (static_cast<size_t>(waves) * kmax + 32) * sizeof(int) + (sbt <= kStagedItems ? 2 * static_cast<size_t>(sbt) : 0);
 }
 
 __global__ __launch_bounds__(1024) void km_members_kernel(KmParams a) {
     extern __shared__ int smem_i[];
     const int seg = blockIdx.y, sb = blockIdx.x;
     if (a.done && a.done[seg]) return;
-    const int k = a.k[seg % a.P], bits = bits_for(k);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int nthr = blockDim.x, nw = nthr >> 6;
-    int* cnt = smem_i;                          // [nw][k]
-    int* wsum = smem_i + nw * a.kmax;           // [16]
-    uint16_t* place = reinterpret_cast<uint16_t*>(wsum + 32);
-    const bool staged = a.sbt <= kStagedTokens;
+    const int k = a.k[seg % a.P];
+    int* cnt = smem_i;                                          // [waves][k]
+    int* wsum = smem_i + (blockDim.x >> 6) * a.kmax;            // [16]
+    uint16_t* staged = reinterpret_cast<uint16_t*>(wsum + 32);  // [sbt]
+    const bool stage = a.sbt <= kStagedItems;
     const int base = sb * a.sbt;
     const int m = min(a.sbt, a.T - base);
     const int32_t* lab = a.labels + static_cast<int64_t>(seg) * a.T + base;
-    const int span = a.sbt / nw;                // tokens per wave (a multiple of 64)
-    const int w0 = wave * span, w1 = min(w0 + span, m);
-    for (int i = tid; i < nw * k; i += nthr) cnt[i] = 0;
-    __syncthreads();
-    int* mine = cnt + wave * k;
-    for (int i = w0; i < w1; i += 256) {
-        int l[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) l[u] = lab[min(i + 64 * u + lane, m - 1)];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (i + 64 * u + lane < w1) atomicAdd(&mine[l[u]], 1);
-    }
-    __syncthreads();
-    // exclusive offsets over (label, wave): consecutive labels per thread
-    const int per = (k + nthr - 1) / nthr;
-    const int c0 = min(tid * per, k), c1 = min(c0 + per, k);
-    int local = 0;
-    for (int c = c0; c < c1; ++c)
-        for (int w = 0; w < nw; ++w) local += cnt[w * k + c];
-    const int incl = wave_incl_scan(local);
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int run = incl - local;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-    int32_t* row = a.loff + (static_cast<int64_t>(seg) * a.nsb + sb) * (a.kmax + 1);
-    for (int c = c0; c < c1; ++c) {
-        row[c] = run;
-        for (int w = 0; w < nw; ++w) {
-            const int n = cnt[w * k + c];
-            cnt[w * k + c] = run;
-            run += n;
-        }
-    }
-    if (tid == 0) row[k] = m;
-    __syncthreads();
     int32_t* out = a.sorted + static_cast<int64_t>(seg) * a.T + base;
-    for (int i = w0; i < w1; i += 256) {
-        int l[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) l[u] = lab[min(i + 64 * u + lane, m - 1)];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (i + 64 * u >= w1) break;
-            const int tk = i + 64 * u + lane;
-            const bool in = tk < w1;
-            const uint64_t peers = match_peers(static_cast<uint32_t>(l[u]), bits, __ballot(in));
-            const int rank = __popcll(peers & lanemask_lt());
-            const int at = in ? mine[l[u]] : 0;
-            km_wave_lds_sync();
-            if (in) {
-                if (rank == 0) mine[l[u]] = at + __popcll(peers);
-                if (staged)
-                    place[at + rank] = static_cast<uint16_t>(tk);
-                else
-                    out[at + rank] = base + tk;
-            }
-            km_wave_lds_sync();
-        }
-    }
-    if (!staged) return;
+    int32_t* row = a.loff + (static_cast<int64_t>(seg) * a.nsb + sb) * (a.kmax + 1);
+    if (threadIdx.x == 0) row[k] = m;
+    superblock_sort(
+        m, a.sbt, k, cnt, wsum, [&](int i) { return lab[i]; }, [&](int c, int first) { row[c] = first; },
+        [&](int i, int at) {
+            if (stage)
+                staged[at] = static_cast<uint16_t>(i);
+            else
+                out[at] = base + i;
+        });
+    if (!stage) return;
     __syncthreads();
-    for (int i = tid; i < m; i += nthr) out[i] = base + place[i];
+    for (int i = threadIdx.x; i < m; i += blockDim.x) out[i] = base + staged[i];
 }
 
 // M-step, one workgroup per cluster: wave 0 keeps the chains (lane d =
@@ -1822,7 +1752,7 @@ __global__ __launch_bounds__(64 * kWaveClusters) void km_update_wave_kernel(KmPa
         }
         n += __builtin_amdgcn_readlane(incl, 63);
     }
-    km_wave_lds_sync();
+    wave_lds_order();
     int32_t* empty = a.empties + static_cast<int64_t>(seg) * a.kmax + c;
     if (n == 0) {
         int e = 0;   // empty labels below c
@@ -1931,16 +1861,6 @@ int validate(const imi_kmeans_args* a, int& kmax, int& dp) {
     IMI_REQUIRE((reinterpret_cast<uintptr_t>(a->keys) & 15) == 0, IMI_ERR_INVALID,
                 "imi_kmeans: keys must be 16-byte aligned");
     return IMI_OK;
-}
-
-// Superblocks of the member lists: about two rounds of workgroups over the
-// device, 1024 .. 8192 tokens each (a segment's slice then sorts in LDS), and
-// at most kMaxSuper of them.
-void superblocks(int T, int segs, int& sbt, int& nsb) {
-    sbt = 1024;
-    while (sbt < 8192 && static_cast<int64_t>(sbt) * 2 * device_cus() < static_cast<int64_t>(T) * segs) sbt *= 2;
-    while ((static_cast<int64_t>(T) + sbt - 1) / sbt > kMaxSuper) sbt *= 2;
-    nsb = static_cast<int>((static_cast<int64_t>(T) + sbt - 1) / sbt);
 }
 
 // Whether kmeans++ screens its rows over an 8-bit copy: from 16 MB of keys
@@ -2149,7 +2069,7 @@ int run_update(const KmParams& p, int segs, const Draws& dr, int it, hipStream_t
 }
 
 int run_members(const KmParams& p, int segs, hipStream_t stream) {
-    const int waves = p.kmax <= kImiMaxK ? 16 : 4;   // label counts per wave in LDS
+    const int waves = sort_waves(p.kmax);
     const size_t lds = members_lds_bytes(waves, p.kmax, p.sbt);
     if (lds > 64 * 1024)
         IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_members_kernel),
