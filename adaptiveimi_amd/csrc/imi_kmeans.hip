@@ -49,7 +49,7 @@ struct KmParams {
     int32_t* done;     // [seg] or null
     int32_t* iters;    // [seg] or null
     void* ppstats;     // kmeans++ block statistics, two launches' (init_mode 2)
-    uint8_t* ppq;      // kmeans++ 8-bit copy and its norms, scales, error bounds (or null)
+    uint8_t *ppq, *ppqd;   // kmeans++ 8-bit copy, its dims' order, norms, scales, error bounds (or null)
     float *ppqn, *ppqs, *ppqe;
     int nblk;          // 256-token blocks
     int max_iters;
@@ -738,9 +738,14 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 // relative in the two norms, 2^-22 elsewhere, 2^-19 in the reference's
 // distance) is covered by 2^-14 of the operands' magnitudes, subnormal
 // effects by 1e-30; NaN, infinities and norms past 1e37 get the distance.
-// The copy is half of the keys' bytes; over 63 picks of the benchmark's keys
-// the rows that change are 3.3 passes in total and those the copy cannot rule
-// out 3.9.
+//
+// The distance over some of the dims is a bound as well: each group's dims are
+// copied in descending order of their scale, and a pick reads the first half
+// of them (a quarter of the keys' bytes).  Only where a wave's rows that this
+// half cannot rule out are more than half of them (keys without dominant
+// channels, early picks) does it read the other half.  With the benchmark's
+// keys (k = 64, 64 dims) 6 % of the rows change per pick, the whole copy
+// leaves 7.8 % and its first half 9.8 %; k = 181: 2.5, 3.3 and 4.5 %.
 constexpr int kPpScreenBytes = 16 << 20;   // key bytes from which the rows are copied to 8 bits
 constexpr int64_t kPpCopyBytes = int64_t{4} << 30;   // largest copy
 
@@ -929,9 +934,11 @@ struct PpStep {
     const PpBlock* st_in;        // [seg][nbp] statistics of launch c - 1
     PpBlock* st_out;
     // the 8-bit copy by groups of 256 rows (RPT per block): [group][DP / 16][256]
-    // rows' 16-byte chunks, their norms [group][256], the group's scales
-    // [group][DP] and error bound [group]
+    // rows' 16-byte chunks, their norms over the first half of the dims and
+    // over all [group][2][256], the group's dims in the copy's order [group][DP]
+    // and their scales, error bound [group]
     pp_u32x4_t* q;
+    uint8_t* qd;
     float* qn;
     float* qs;
     float* qe;
@@ -992,6 +999,7 @@ __global__ __launch_bounds__(256) void km_pp_exact_kernel(KmParams a, PpStep ps)
     __shared__ float s_part[FIRST ? 512 : 1];
     __shared__ __attribute__((aligned(16))) float s_scale[FIRST ? DP : 4];
     __shared__ __attribute__((aligned(16))) float s_inv[FIRST ? DP : 4];
+    __shared__ uint8_t s_dim[FIRST ? DP : 4];
     __shared__ float s_err[4];
     constexpr int CH = DP / 8;   // 16-byte chunks per row
     constexpr int GROUPS = FIRST ? RPT : 1;
@@ -1066,35 +1074,51 @@ __global__ __launch_bounds__(256) void km_pp_exact_kernel(KmParams a, PpStep ps)
                 if (tid < DP) {
                     float m4 = 0.0f;   // (a NaN's bits give a NaN here, an infinity an infinite scale)
                     for (int i = 0; i < PARTS; ++i) m4 = s_part[i * DP + tid] > m4 || s_part[i * DP + tid] != s_part[i * DP + tid] ? s_part[i * DP + tid] : m4;
-                    const float sc = m4 * (1.0f / 127.0f);
-                    s_scale[tid] = sc;
-                    s_inv[tid] = sc > 0.0f ? 1.0f / sc : 0.0f;
-                    ps.qs[group * DP + tid] = sc;
+                    s_part[tid] = m4;   // (only this thread reads column tid of the parts)
                 }
                 __syncthreads();
+                if (tid < DP) {
+                    // place in descending order of magnitude (of its bits: a
+                    // total order also over NaN), equal ones by dim
+                    const uint32_t mine = __float_as_uint(s_part[tid]);
+                    int at = 0;
+#pragma unroll 8
+                    for (int j = 0; j < DP; ++j) {
+                        const uint32_t other = __float_as_uint(s_part[j]);
+                        at += other > mine || (other == mine && j < tid) ? 1 : 0;
+                    }
+                    const float sc = s_part[tid] * (1.0f / 127.0f);
+                    s_dim[at] = static_cast<uint8_t>(tid);
+                    s_scale[at] = sc;
+                    s_inv[at] = sc > 0.0f ? 1.0f / sc : 0.0f;
+                    ps.qs[group * DP + at] = sc;
+                    ps.qd[group * DP + at] = static_cast<uint8_t>(tid);
+                }
+                __syncthreads();
+                const uint16_t* own = reinterpret_cast<const uint16_t*>(s_rows + tid * (CH + 1));
                 float nrm = 0.0f, err = 0.0f;
 #pragma unroll
                 for (int i = 0; i < DP / 16; ++i) {
                     pp_u32x4_t o;
 #pragma unroll
                     for (int w = 0; w < 4; ++w) {   // four dims per dword
-                        const uint32_t x01 = v[2 * i + w / 2][2 * (w % 2)], x23 = v[2 * i + w / 2][2 * (w % 2) + 1];
-                        const float x[4] = {bf16_lo(x01), bf16_hi(x01), bf16_lo(x23), bf16_hi(x23)};
                         uint32_t b = 0;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const int j = 16 * i + 4 * w + e;
-                            const float t = fminf(fmaxf(rintf(x[e] * s_inv[j]), -127.0f), 127.0f);
+                            const float x = bf16_to_f32(own[s_dim[j]]);
+                            const float t = fminf(fmaxf(rintf(x * s_inv[j]), -127.0f), 127.0f);
                             const float xh = t * s_scale[j];
                             nrm = __builtin_fmaf(xh, xh, nrm);
-                            err = __builtin_fmaf(x[e] - xh, x[e] - xh, err);
+                            err = __builtin_fmaf(x - xh, x - xh, err);
                             b |= (static_cast<uint32_t>(static_cast<int>(t)) & 0xFFu) << (8 * e);
                         }
                         o[w] = b;
                     }
                     ps.q[(group * (DP / 16) + i) * 256 + tid] = o;
+                    if (i == DP / 32 - 1) ps.qn[group * 512 + tid] = nrm;
                 }
-                ps.qn[group * 256 + tid] = nrm;
+                ps.qn[group * 512 + 256 + tid] = nrm;
                 // error bound of the group's rows; a non-finite one rules nothing out
                 float e = r < T ? sqrtf(err) * (1.0f + 0x1p-14f) + 1e-30f : 0.0f;
                 e = e <= 1e30f ? e : INFINITY;
@@ -1116,16 +1140,18 @@ __global__ __launch_bounds__(256) void km_pp_exact_kernel(KmParams a, PpStep ps)
 // row (lane part j sums dims j, j + 8, .., the reference's lane j; row shifts
 // add the eight sums left to right).  Only the block statistics cross waves.
 //
-// Bound by the copy's bytes (76 per 64-dim row with norm and minima) for large
-// inputs, by the pick's dependent loads for small ones.  Per pick, 64 dims,
-// 16 segments: 33.3 us at 128k tokens (55 us reading the keys), 147 us at 512k
-// (250 us).  Two of the four rows
-// loaded at a time keep four waves per SIMD (36.4 us with all four and three
-// waves); the next block's loads are issued before the queue.
+// Bound by the copy's bytes (44 per 64-dim row with norm and minima, 76 when
+// both halves are read) and the queue's dependent loads for large inputs, by
+// the pick's dependent loads for small ones.  Per pick, 64 dims, 16 segments:
+// 29.5 us at 128k tokens (22 us for the late picks; 33 us with the whole copy
+// read, 55 us reading the keys), 106 us at 512k (146 and 250 us); keys without
+// dominant channels read both halves one after the other, 7 % slower than the
+// whole copy at once.  The next block's loads are issued before the queue (8
+// lanes per row there: one row per lane spilled over 64 dims, 65 us).
 template <int DP, int RPT>
 __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(KmParams a, PpStep ps) {
     constexpr int CH = DP / 16;                   // 16-byte chunks per copied row
-    constexpr int LR = RPT < 2 || DP < 64 ? RPT : 2;   // rows per thread loaded together
+    constexpr int HC = CH / 2;                    // of the first half of the dims
     constexpr int DL = DP > 64 ? DP / 64 : 1;     // dims per lane of the weights
     __shared__ __attribute__((aligned(16))) float cur[DP];
     __shared__ PpBlock s_st[2][4];
@@ -1143,43 +1169,35 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
     float* mdo = ps.md_out + static_cast<int64_t>(seg) * T;
     const uint16_t* xb = a.keys + static_cast<int64_t>(h) * a.hs + p * DP;
     const int blk0 = blockIdx.x * ps.nsub, blk1 = min(blk0 + ps.nsub, nb);
-    pp_u32x4_t q[LR][CH];
+    pp_u32x4_t q[RPT][HC];
     float m[RPT], nrm[RPT], sc[DL], err;
+    int dim[DL];
     // the wave's group of block bk, its first row there and in the segment
     const int g_in = RPT == 4 ? wave : 0, row_in = RPT == 4 ? 0 : 64 * wave;
     static_assert(RPT == 4 || RPT == 1, "groups per block");
     auto group_of = [&](int bk) { return (static_cast<int64_t>(seg) * nb + bk) * RPT + g_in; };
     auto row_of = [&](int bk) { return (bk * RPT + g_in) * 256 + row_in; };
-    auto load_rows = [&](int64_t group, int i0) {
-#pragma unroll
-        for (int i = 0; i < LR; ++i)
-#pragma unroll
-            for (int k = 0; k < CH; ++k) q[i][k] = ps.q[(group * CH + k) * 256 + row_in + 64 * (i0 + i) + lane];
-    };
     auto load_group = [&](int bk) {
         const int64_t group = group_of(bk);
         const int r0 = row_of(bk);
 #pragma unroll
-        for (int u = 0; u < DL; ++u) sc[u] = ps.qs[group * DP + (64 * u + lane) % DP];
+        for (int u = 0; u < DL; ++u) {
+            sc[u] = ps.qs[group * DP + (64 * u + lane) % DP];
+            dim[u] = ps.qd[group * DP + (64 * u + lane) % DP];
+        }
         err = ps.qe[group];
 #pragma unroll
         for (int i = 0; i < RPT; ++i) {
             m[i] = mdi[min(r0 + 64 * i + lane, T - 1)];
-            nrm[i] = ps.qn[group * 256 + row_in + 64 * i + lane];
+            nrm[i] = ps.qn[group * 512 + row_in + 64 * i + lane];
+#pragma unroll
+            for (int k = 0; k < HC; ++k) q[i][k] = ps.q[(group * CH + k) * 256 + row_in + 64 * i + lane];
         }
-        load_rows(group, 0);
     };
     if (dist) load_group(blk0);   // does not depend on the pick
     pp_take_pick<DP, 4 * RPT>(a, ps, seg, p, xb, cur);
     if (!dist) return;
     __syncthreads();
-    float cj[DL], cc = 0.0f;   // the pick's dims of this lane, |c|^2
-#pragma unroll
-    for (int u = 0; u < DL; ++u) {
-        cj[u] = cur[(64 * u + lane) % DP];
-        cc = __builtin_fmaf(cj[u], cj[u], cc);
-    }
-    cc = wave_sum(DP < 64 && lane >= DP ? 0.0f : cc);
     float cp[DP / 8];   // dims part, part + 8, .. for the distances
 #pragma unroll
     for (int i = 0; i < DP / 8; ++i) cp[i] = cur[8 * i + (lane & 7)];
@@ -1187,14 +1205,19 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
     for (int bk = blk0; bk < blk1; ++bk) {
         const int64_t group = group_of(bk);
         const int r0 = row_of(bk);
-        // 16-bit weights s_j c_j / W in two signed bytes
-        float wj[DL], wmax = 0.0f;
+        // 16-bit weights s_j c_j / W in two signed bytes; |c|^2 over the first
+        // half of the dims and over all
+        float wj[DL], wmax = 0.0f, cc1 = 0.0f, cc = 0.0f;
 #pragma unroll
         for (int u = 0; u < DL; ++u) {
-            wj[u] = sc[u] * cj[u];
+            const float cj = DP >= 64 || lane < DP ? cur[dim[u]] : 0.0f;
+            wj[u] = sc[u] * cj;
             wmax = fmaxf(wmax, fabsf(wj[u]));
+            if (64 * u + lane < DP / 2) cc1 = __builtin_fmaf(cj, cj, cc1);
+            cc = __builtin_fmaf(cj, cj, cc);
         }
         wmax = wave_max(wmax);
+        cc1 = wave_sum(cc1);
         const float W = wmax * (1.0f / 32512.0f), iw = wmax > 0.0f ? 32512.0f / wmax : 0.0f;
 #pragma unroll
         for (int u = 0; u < DL; ++u) {
@@ -1206,38 +1229,58 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
             }
         }
         wave_lds_order();
-        // the weights' rounding: at most W (1/2 + 2^-8) per dim times |q| <= 127, twice
-        const float slack = 130.0f * DP * W + 0x1p-14f * cc + 1e-30f;
+        int hi[RPT], lo[RPT];
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) hi[i] = lo[i] = 0;
+        auto dot16 = [&](const pp_u32x4_t& x, int k, int i) {   // chunk k of row i
+            const pp_u32x4_t wh = *reinterpret_cast<const pp_u32x4_t*>(&s_w[wave][0][16 * k]);
+            const pp_u32x4_t wl = *reinterpret_cast<const pp_u32x4_t*>(&s_w[wave][1][16 * k]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                hi[i] = __builtin_amdgcn_sdot4(static_cast<int>(x[e]), static_cast<int>(wh[e]), hi[i], false);
+                lo[i] = __builtin_amdgcn_sdot4(static_cast<int>(x[e]), static_cast<int>(wl[e]), lo[i], false);
+            }
+        };
+        // whether row i keeps its minimum: n = |x^|^2, c2 = |c|^2 over the dims
+        // of the dot product.  The weights' rounding: at most W (1/2 + 2^-8) per
+        // dim times |q| <= 127, twice.
+        auto ruled_out = [&](int i, float n, float c2) {
+            const float slack = 130.0f * DP * W + 0x1p-14f * c2 + 1e-30f;
+            const float dot = W * static_cast<float>(256 * hi[i] + lo[i]);
+            const float low = (n + c2) - 2.0f * dot - (slack + 0x1p-14f * n);
+            const float reach = (__builtin_amdgcn_sqrtf(m[i]) + err) * (1.0f + 0x1p-14f);
+            // (norms past 1e37 could overflow where the distance does not)
+            return low >= reach * reach && n + c2 <= 1e37f;
+        };
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+#pragma unroll
+            for (int i = 0; i < RPT; ++i) dot16(q[i][k], k, i);
         uint32_t need = 0;
+        int left = 0;
 #pragma unroll
-        for (int i0 = 0; i0 < RPT; i0 += LR) {
-            if (i0 > 0) load_rows(group, i0);
-            int hi[LR], lo[LR];
+        for (int i = 0; i < RPT; ++i) {
+            const bool in = r0 + 64 * i + lane < T && m[i] != 0.0f && !ruled_out(i, nrm[i], cc1);
+            if (in) need |= 1u << i;
+            left += __popcll(__ballot(in));
+        }
+        // a row's distance costs four times what its other half does
+        if (left > 32 * RPT) {
+            const float c2 = wave_sum(cc);
+            float all[RPT];
 #pragma unroll
-            for (int i = 0; i < LR; ++i) hi[i] = lo[i] = 0;
+            for (int i = 0; i < RPT; ++i) {
+                all[i] = ps.qn[group * 512 + 256 + row_in + 64 * i + lane];
 #pragma unroll
-            for (int k = 0; k < CH; ++k) {
-                const pp_u32x4_t wh = *reinterpret_cast<const pp_u32x4_t*>(&s_w[wave][0][16 * k]);
-                const pp_u32x4_t wl = *reinterpret_cast<const pp_u32x4_t*>(&s_w[wave][1][16 * k]);
-#pragma unroll
-                for (int i = 0; i < LR; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        hi[i] = __builtin_amdgcn_sdot4(static_cast<int>(q[i][k][e]), static_cast<int>(wh[e]), hi[i], false);
-                        lo[i] = __builtin_amdgcn_sdot4(static_cast<int>(q[i][k][e]), static_cast<int>(wl[e]), lo[i], false);
-                    }
+                for (int k = 0; k < HC; ++k) q[i][k] = ps.q[(group * CH + HC + k) * 256 + row_in + 64 * i + lane];
             }
 #pragma unroll
-            for (int i = 0; i < LR; ++i) {
-                const float dot = W * static_cast<float>(256 * hi[i] + lo[i]);
-                const float n = nrm[i0 + i];
-                const float low = (n + cc) - 2.0f * dot - (slack + 0x1p-14f * n);
-                const float reach = (__builtin_amdgcn_sqrtf(m[i0 + i]) + err) * (1.0f + 0x1p-14f);
-                const bool in = r0 + 64 * (i0 + i) + lane < T;
-                // (norms past 1e37 could overflow where the distance does not)
-                const bool out = low >= reach * reach && n + cc <= 1e37f;
-                if (in && m[i0 + i] != 0.0f && !out) need |= 1u << (i0 + i);
-            }
+            for (int k = 0; k < HC; ++k)
+#pragma unroll
+                for (int i = 0; i < RPT; ++i) dot16(q[i][k], HC + k, i);
+#pragma unroll
+            for (int i = 0; i < RPT; ++i)
+                if (ruled_out(i, all[i], c2)) need &= ~(1u << i);
         }
         // the next block's loads overlap with the queue's
         float mc[RPT];
@@ -1900,6 +1943,7 @@ int run_plusplus(const KmParams& p, const imi_kmeans_args* a, int segs, hipStrea
     const int nbp = (p.T + rows - 1) / rows;
     ps.nbp = nbp;
     ps.q = reinterpret_cast<pp_u32x4_t*>(p.ppq);
+    ps.qd = p.ppqd;
     ps.qn = p.ppqn;
     ps.qs = p.ppqs;
     ps.qe = p.ppqe;
@@ -1980,7 +2024,8 @@ size_t workspace_bytes(const imi_kmeans_args* a, int kmax, KmParams* out) {
         p.ppmd = cv.take<float>(static_cast<size_t>(segs) * a->n_tokens);
         if (screened) {
             p.ppq = cv.take<uint8_t>(blocks * rows * dp);
-            p.ppqn = cv.take<float>(blocks * rows);
+            p.ppqd = cv.take<uint8_t>(blocks * rows / 256 * dp);
+            p.ppqn = cv.take<float>(2 * blocks * rows);
             p.ppqs = cv.take<float>(blocks * rows / 256 * dp);
             p.ppqe = cv.take<float>(blocks * rows / 256);
         }
