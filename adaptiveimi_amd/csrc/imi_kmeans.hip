@@ -1852,18 +1852,29 @@ __global__ __launch_bounds__(64 * kWaveClusters) void km_update_wave_kernel(KmPa
     *reinterpret_cast<float2*>(dst + 2 * lane) = make_float2(x0 * inv, x1 * inv);
 }
 
-// Empty clusters whose ordinal falls in [e0, e0 + kDraws): the draws of
+// Empty clusters whose ordinal falls in [e0, e0 + kMoreDraws): the draws of
 // that slice (clusters beyond kDraws empty ones only occur when k > kDraws).
-__global__ __launch_bounds__(64) void km_reseed_kernel(KmParams a, Draws draws, int e0) {
-    const int c = blockIdx.x, seg = blockIdx.y;
-    const int h = seg / a.P, p = seg % a.P;
-    if (c >= a.k[p]) return;
+// A thread per cluster looks, its wave copies the rows of those that it finds
+// (seldom any).  768 draws are 3 KB of kernel arguments: one launch up to k =
+// 1024 (8 x 1018 clusters: 4.6 us per iteration; three launches of 256 draws
+// with a workgroup per cluster 14 us).
+constexpr int kMoreDraws = 768;
+struct MoreDraws {
+    int32_t v[kMoreDraws];
+};
+
+__global__ __launch_bounds__(256) void km_reseed_kernel(KmParams a, MoreDraws draws, int e0) {
+    const int c = blockIdx.x * 256 + threadIdx.x, seg = blockIdx.y;
+    const int h = seg / a.P, p = seg % a.P, lane = lane_id();
     if (a.done && a.done[seg]) return;
-    const int e = a.empties[static_cast<int64_t>(seg) * a.kmax + c] - e0;
-    if (e < 0 || e >= kDraws) return;
-    const uint16_t* row = a.keys + h * a.hs + p * a.DP + static_cast<int64_t>(draws.v[e]) * a.ts;
-    float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + c) * a.DP;
-    for (int d = threadIdx.x; d < a.DP; d += 64) dst[d] = bf16_to_f32(row[d]);
+    const int e = c < a.k[p] ? a.empties[static_cast<int64_t>(seg) * a.kmax + c] - e0 : -1;
+    for (uint64_t hit = __ballot(e >= 0 && e < kMoreDraws); hit; hit &= hit - 1) {
+        const int l = __builtin_ctzll(hit);
+        const int tok = draws.v[__builtin_amdgcn_readlane(e, l)];
+        const uint16_t* row = a.keys + h * a.hs + p * a.DP + static_cast<int64_t>(tok) * a.ts;
+        float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + (c - lane + l)) * a.DP;
+        for (int d = lane; d < a.DP; d += 64) dst[d] = bf16_to_f32(row[d]);
+    }
 }
 
 __global__ void km_reset_kernel(KmParams a) {
@@ -2214,9 +2225,10 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
                        : (dp == 64 ? run_update<64>(p, segs, dr, it, stream) : run_update<32>(p, segs, dr, it, stream));
         if (rc) return rc;
         // the draws of empty ordinals kDraws and up (IVF, k > kDraws)
-        for (int e0 = kDraws; e0 < kmax; e0 += kDraws) {
-            for (int e = e0; e < std::min(kmax, e0 + kDraws); ++e) dr.v[e - e0] = dist(rng);
-            hipLaunchKernelGGL(km_reseed_kernel, dim3(kmax, segs), dim3(64), 0, stream, p, dr, e0);
+        for (int e0 = kDraws; e0 < kmax; e0 += kMoreDraws) {
+            MoreDraws more;
+            for (int e = e0; e < std::min(kmax, e0 + kMoreDraws); ++e) more.v[e - e0] = dist(rng);
+            hipLaunchKernelGGL(km_reseed_kernel, dim3((kmax + 255) / 256, segs), dim3(256), 0, stream, p, more, e0);
             IMI_LAUNCH_CHECK("km_reseed_kernel");
         }
     }

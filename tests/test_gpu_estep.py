@@ -92,6 +92,23 @@ def test_lloyd_over_superblock_edges(oracle, H, T, ks, stop):
             assert np.array_equal(cent[h, p, :k].cpu().numpy(), cents[p]), (h, p)
 
 
+@pytest.mark.parametrize("H,T,k", [(1, 1500, 296), (2, 1500, 297), (1, 2000, 1064), (1, 2000, 1065), (2, 2000, 1900)])
+def test_reseed_slices(oracle, H, T, k):
+    """40 distinct rows leave k - 40 clusters empty: around the 256 draws of the
+    M-step's launch, the 768 of each later one, and more than two of those."""
+    from adaptiveimi_amd import ops, synthetic
+
+    print(f"[reseed] H={H} T={T} k={k}", flush=True)
+    keys, _ = synthetic.make_kv(H, T, seed=k)
+    keys = _awkward(keys, "duplicates")
+    cent, labels, _ = ops.kmeans(keys.to(DEV), [k], 2)
+    kf = oracle.bf16_to_f32(_bits(keys))
+    for h in range(H):
+        labs, cents, _ = oracle.kmeans_head(kf[h], [k], 2)
+        assert np.array_equal(labels[h, 0].cpu().numpy(), labs[0]), h
+        assert np.array_equal(cent[h, 0, :k].cpu().numpy(), cents[0]), h
+
+
 def _awkward(keys, form):
     """Rows on which the 8-bit copy's bound is poor or degenerate."""
     k = keys.float()
