@@ -736,8 +736,20 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 // against s_j c_j rounded to 16 bits (two 8-bit parts, exact integer sums, the
 // rounding at most W / 2 per dim bounded apart).  fp32 rounding (at most 2^-17
 // relative in the two norms, 2^-22 elsewhere, 2^-19 in the reference's
-// distance) is covered by 2^-14 of the operands' magnitudes, subnormal
-// effects by 1e-30; NaN, infinities and norms past 1e37 get the distance.
+// distance) is covered by 2^-14 of the operands' magnitudes; NaN, infinities
+// and norms past 1e37 get the distance.  What has no relative bound:
+//   - a weight s_j c_j is rounded to a step W of at least kPpLeastWeight /
+//     32512, so W / 2 holds for the smallest ones too and the quotient
+//     32512 / (largest weight) stays finite;
+//   - a product below the normal range (fp32 subnormals are kept) is off by at
+//     most 2^-150: 2 * 128 * 127 of them in the dot product, 128 in each sum
+//     of squares, together below 1e-40;
+//   - an error e whose squares underflow is at most 5e-22 too small, and the
+//     square root may take a subnormal minimum for zero (1.1e-19): beside
+//     sqrt(m) + e <= 1e-9 their effect on the square, 2 (sqrt(m) + e) 5e-22
+//     and 2 e 1.1e-19 + 1.2e-38, is below 1e-30 up to e = 4e-12 and below
+//     2^-14 of the square beyond.
+// The last two are the 1e-30 of the slack.
 //
 // The distance over some of the dims is a bound as well: each group's dims are
 // copied in descending order of their scale, and a pick reads the first half
@@ -748,6 +760,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 // leaves 7.8 % and its first half 9.8 %; k = 181: 2.5, 3.3 and 4.5 %.
 constexpr int kPpScreenBytes = 16 << 20;   // key bytes from which the rows are copied to 8 bits
 constexpr int64_t kPpCopyBytes = int64_t{4} << 30;   // largest copy
+constexpr float kPpLeastWeight = 1e-30f;   // largest weight of a group that the steps of its 16 bits still follow
 
 struct PpBlock {    // per (segment, block)
     double sum;     // of its min distances (exact when the exponent spread allows)
@@ -1218,7 +1231,11 @@ __global__ __launch_bounds__(256, DP == 128 ? 2 : 4) void km_pp_screen_kernel(Km
         }
         wmax = wave_max(wmax);
         cc1 = wave_sum(cc1);
-        const float W = wmax * (1.0f / 32512.0f), iw = wmax > 0.0f ? 32512.0f / wmax : 0.0f;
+        // (weights below kPpLeastWeight are held at its steps: 32512 / wmax
+        // would overflow from 9.6e-35 down, and a quotient of infinity makes
+        // every weight, zero ones too, a largest one)
+        const float wtop = fmaxf(wmax, kPpLeastWeight);
+        const float W = wtop * (1.0f / 32512.0f), iw = 32512.0f / wtop;
 #pragma unroll
         for (int u = 0; u < DL; ++u) {
             if (DP >= 64 || lane < DP) {

@@ -151,3 +151,36 @@ def test_plusplus_screened_rows(oracle, H, T, ks, form):
         for p, k in enumerate(ks):
             assert np.array_equal(labels[h, p].cpu().numpy(), labs[p]), (h, p)
             assert np.array_equal(cent[h, p, :k].cpu().numpy(), cents[p]), (h, p)
+
+
+@pytest.mark.parametrize("ks,seed", [((10,), 0), ((10,), 1), ((10,), 2), ((10, 10), 0), ((10, 10), 1), ((10, 10), 2)])
+def test_plusplus_weights_below_the_quotient_range(oracle, ks, seed):
+    """Picks of norm 2^-53 with one non-zero dim, so that the largest weight of
+    a group (its scale times the pick, 8.5e-35) is below 2^-113, where 32512
+    divided by it is infinite, while the rows' distances are above the 1e-30
+    the bound allows for: most rows (0.875 a, 0, ..), the first pick
+    (-0.875 a, 0, ..), ten groups of entries a or a / 2 with dim 0 negated in
+    every other one, which the second pick of the first kind is nearer to."""
+    from adaptiveimi_amd import ops
+
+    print(f"[kmeans++ small weights] ks={ks} seed={seed}", flush=True)
+    H, T, dp, a = 1, 65536, 128 // len(ks), 2.0 ** -53
+    rng = np.random.default_rng(seed)
+    x = np.zeros((T, 128), np.float32)
+    x[:, ::dp] = 0.875 * a
+    for i, g in enumerate(rng.permutation(T // 256)[:10]):
+        rows = np.where(rng.random((256, 128)) < 0.5, a, a / 2)
+        if i % 2:
+            rows[:, ::dp] *= -1
+        x[256 * g:256 * g + 256] = rows
+    number = np.arange(T, dtype=np.float32)[:, None]
+    for p in range(len(ks)):   # the row that the seed's first draw takes
+        first = int(oracle.kmeanspp_init(number, 1, 42 + p)[0, 0])
+        x[first, p * dp:(p + 1) * dp] = 0
+        x[first, p * dp] = -0.875 * a
+    keys = torch.from_numpy(x)[None].to(torch.bfloat16)
+    cent, labels, _ = ops.kmeans(keys.to(DEV), list(ks), 1, init="kmeans++")
+    labs, cents, _ = oracle.kmeans_head(x, list(ks), 1, init="kmeans++")
+    for p, k in enumerate(ks):
+        assert np.array_equal(labels[0, p].cpu().numpy(), labs[p]), p
+        assert np.array_equal(cent[0, p, :k].cpu().numpy(), cents[p]), p
