@@ -23,6 +23,7 @@
 // register rings and an LDS hand-off.
 #include <limits>
 #include <random>
+#include <utility>
 #include <vector>
 
 #include "imi_common.hpp"
@@ -133,32 +134,55 @@ __device__ __forceinline__ float l2_lanes8_bf16(const V (&v)[DP / 8], const floa
 }
 
 // ------------------------------------------------------------------ E-step
-// Matrix-core screening for any k.  For token x and centroid c the value
-//   f(c) = x.c - |c|^2 / 2 = (|x|^2 - D(x, c)) / 2
-// orders the centroids like the distance (largest f first).  x.c runs on
-// v_mfma_f32_16x16x32_bf16: x is bf16 already and c enters as two bf16 parts
-// (hi = bf16(c), lo = bf16(c - hi), |c - hi - lo| <= 2^-16 |c|); the
-// accumulators start at -|c|^2 / 2.  Rounding analysis with mag = |x|^2 +
-// max|c|^2, every partial sum of f bounded by |x||c| + |c|^2 / 2 <= mag: at
-// most 256 accumulations of at most 2^-23 each (2^-15, also if the matrix
-// core truncates), the split of c (2^-18 |x||c|) and the norm's chain
-// (2^-17 |c|^2) stay below 2^-14.6 mag, and the reference's own distance (8 FMA
-// chains + 7 adds) adds less than 2^-18.  So the reference's winner satisfies
-// f >= max f - 2^-13.5 mag - 1e-30 (the last term for flushed subnormals).
+// Matrix-core screening for any k.  With the mean of the segment's first and
+// middle centroid as the origin m (subspaces; m = 0 for IVF) and c' = c - m, the
+// value
+//   f(c) = x.c' - (m.c' + |c'|^2 / 2) = (|x - m|^2 - D(x, c)) / 2
+// orders the centroids like the distance (largest f first), and its terms
+// don't grow with a common offset of keys and centroids beyond the first
+// power.  x.c' runs on v_mfma_f32_16x16x32_bf16: x is bf16 already and c'
+// enters as two bf16 parts (hi = bf16(c'), lo = bf16(c' - hi)); the
+// accumulators start at the second term.  Rounding analysis with C = max|c'|,
+// N = |x|^2 + |m|^2 and R = sqrt(2 N) C + C^2 / 2, which bounds every partial
+// sum of f.  Relative to R: 2 DP accumulations of at most 2^-23 each (also if
+// the matrix core truncates), the split of c' (two round-to-nearest bf16 steps:
+// 2^-18), the second term's chains (DP / 4 + 4 operations of 2^-24), the
+// rounding of c' itself (2^-23): 3.63e-5, 2.04e-5 and 1.23e-5 for 128, 64 and
+// 32 dims, and twice that (e_sum, with 5 %) between two centroids.  The
+// reference's own distance is off by at most (DP / 8 + 9) 2^-24 of D (8 FMA
+// chains + 7 adds, the square of a rounded difference); the best centroid's D
+// is at most 2 (N + C^2): e_ref (N + C^2).
 //
 // Each lane keeps the three largest f of its token (a max and two med3 per
 // value), each value carrying its centroid's number in its lowest bits, which
-// moves a value by less than 2^(bits - 23) mag; for IVF the number inside its
-// chunk of 64, the chunk beside it.  With E = (2^-13 + 2^(bits - 22)) mag + 1e-30:
+// moves a value by less than 2^(bits - 23) of it; for IVF the number inside its
+// chunk of 64, the chunk beside it.  So the reference's winner has f >= best - E,
+//   E = e_sum R + 2^(bits - 22) |best| + e_ref (N + C^2) + 1e-30
+// (the last term for subnormals):
 //   second < best - E   the best is the reference's label;
 //   third < best - E    best and second get the exact reference distance
 //                       (l2 in 8 lanes, strict '<' over ascending c);
-//   otherwise, for non-finite or huge magnitudes (mag > 1e37), and for equal
-//   best and second values (their chunks cannot be told apart), every
-//   centroid does.
+//   otherwise, for equal best and second values (IVF: their chunks cannot be
+//   told apart) and for non-finite or huge magnitudes (N + C^2 > 1e37), the
+//   token is undecided.  Up to kFewTokens undecided tokens of a wave get every
+//   centroid's distance one token at a time.  More of them: the block is
+//   screened again, the centroids that reach each token's bound are queued
+//   and get the distance, 64 pairs at a time; where they are more than k / 4
+//   per token, where magnitudes are huge, and for IVF, every lane goes
+//   through all centroids for its token (nearest_of_all).
 // With k-means centroids over the benchmark's keys 0.5-1 % of the tokens take
 // the second form and 0.01 % the third (k = 32..1018).  Outputs (labels, min
 // distances, inertia partials) are those of the exhaustive loop.
+//
+// The origin and the queue matter for keys unlike those.  Lloyd over 8 x 128k
+// keys of N(0, 1), k = 64, 10 iterations, and k = 181, 6 iterations, with the
+// bound in |x|^2 + max|c|^2 and every centroid for each undecided token ->
+// now: four channels of mean 30: 10.6 -> 1.40 and 22.6 -> 1.36 ms; means of
+// deviation 10: 22.9 -> 1.49 and 41.7 -> 1.62 ms, of 100: 27.9 -> 8.4 and
+// 47.6 -> 6.8; 60 % of the keys within 0.05 of one: 21.3 -> 4.2 and 35.7 ->
+// 4.2; row lengths log-normal: 28.4 -> 7.3 and 46.2 -> 8.4.  IVF, 16k, k =
+// 1018, 10 iterations: means of deviation 10: 35.4 -> 10.9 ms (8 x 16k x
+// 1018 distances in 1 ms).
 //
 // A wave owns 64 tokens (four 16-token tiles) and shares nothing with the
 // other waves but the packed centroids, so the loop over its token blocks has
@@ -166,13 +190,14 @@ __device__ __forceinline__ float l2_lanes8_bf16(const V (&v)[DP / 8], const floa
 // block's tokens are loaded while the one before is re-checked.  The
 // centroids are packed into LDS in the matrix-core operand layout by the
 // workgroup: all of them at once for subspaces (4 DP bytes each), in double-
-// buffered chunks of 64 for IVF (STREAM).
+// buffered chunks of 64 for IVF (STREAM; an origin would cost it 11 % on the
+// benchmark's keys, since every block of tokens packs the centroids again).
 //
 // Bound by: reading the keys up to k = 64 (64 x 64, 128k tokens, 8 heads: 268
 // MB in 59 us, 4.5 TB/s; a barrier-synchronised form with the label ranks in
 // it took 85 us), the three VALU operations and the and-or per value beside
-// the matrix work beyond (k = 181, 512k tokens: 515 us; 4.65 ms as fp32
-// distances to every centroid; IVF, k = 1018, 16k tokens, 8 heads: 106 us,
+// the matrix work beyond (k = 181, 512k tokens: 485 us; 4.65 ms as fp32
+// distances to every centroid; IVF, k = 1018, 16k tokens, 8 heads: 104 us,
 // 1.02 ms as such).
 typedef __attribute__((ext_vector_type(8))) __bf16 km_bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float km_f32x4_t;
@@ -211,10 +236,20 @@ __device__ __forceinline__ float max_raw(float a, float b) {
 }
 
 // One lane's share of a 16-centroid tile: dims 32 kh + 8 (lane / 16) .. + 7 of
-// centroid 16 ct + lane % 16 as hi and lo bf16 operands; sq += the dims' squares.
-__device__ __forceinline__ void pack_centroid(const float4 v0, const float4 v1, km_u32x4_t& hi, km_u32x4_t& lo,
-                                              float& sq) {
-    const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+// centroid 16 ct + lane % 16, less the origin's (ORIGIN), as hi and lo bf16
+// operands; sq += the dims' squares, dot += their products with the origin's.
+template <bool ORIGIN>
+__device__ __forceinline__ void pack_centroid(const float4 (&c)[2], const float4* org, km_u32x4_t& hi, km_u32x4_t& lo,
+                                              float& sq, float& dot) {
+    float v[8] = {c[0].x, c[0].y, c[0].z, c[0].w, c[1].x, c[1].y, c[1].z, c[1].w};
+    if constexpr (ORIGIN) {
+        const float m[8] = {org[0].x, org[0].y, org[0].z, org[0].w, org[1].x, org[1].y, org[1].z, org[1].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            v[i] = v[i] - m[i];
+            dot = __builtin_fmaf(v[i], m[i], dot);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const uint32_t h = pack_bf16(v[2 * i], v[2 * i + 1]);
@@ -291,6 +326,90 @@ __device__ __forceinline__ Top3Ids swap_merge(Top3Ids x, Top3Ids y) {
     return x;
 }
 
+// The value, computed where it is used: what depends on it isn't kept in
+// registers over the loop around a seldom taken branch.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// Tokens of a wave up to which the exhaustive form takes them one by one, its
+// lanes over the centroids; beyond, every lane takes its own token.
+constexpr int kFewTokens = 8;
+
+// The exhaustive form for a wave's 64 tokens, all lanes active: each lane has
+// its token's widened row; a centroid is spread over every row of 16 lanes
+// (lane q: dims DP / 16 q ..) and broadcast as an operand modifier of the
+// subtraction (row_newbcast), so a dim takes two VALU operations and no load.
+// The next centroid's part is loaded meanwhile.  (c - x) has the square of
+// (x - c).
+template <int K>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + K, 0xF, 0xF, true));
+}
+
+template <int DP, int... I>
+__device__ __forceinline__ float l2_lanes8_spread(const float (&x)[DP], const float (&c)[DP / 16],
+                                                  std::integer_sequence<int, I...>) {
+    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    const auto dim = [&](auto i) {
+        constexpr int N = decltype(i)::value;
+        const float d = row_bcast<N / (DP / 16)>(c[N % (DP / 16)]) - x[N];
+        acc[N % 8] = __builtin_fmaf(d, d, acc[N % 8]);
+    };
+    (dim(std::integral_constant<int, I>{}), ...);
+    float t = acc[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) t = t + acc[j];
+    return t;
+}
+
+template <int DP>
+__device__ __forceinline__ void load_spread(const float* row, int q, float (&c)[DP / 16]) {
+#pragma unroll
+    for (int e = 0; e < DP / 16; e += 2) {
+        const float2 v = *reinterpret_cast<const float2*>(row + DP / 16 * q + e);
+        c[e] = v.x;
+        c[e + 1] = v.y;
+    }
+}
+
+// Smallest distance of the lane's row and the lowest centroid that has it.
+template <int DP>
+__device__ __forceinline__ void nearest_of_all(const uint16_t* row, const float* cg, int k, float& best, int& arg) {
+    float x[DP];
+#pragma unroll
+    for (int i = 0; i < DP / 8; ++i) {
+        const km_u32x4_t v = reinterpret_cast<const km_u32x4_t*>(row)[i];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[8 * i + 2 * e] = bf16_lo(v[e]);
+            x[8 * i + 2 * e + 1] = bf16_hi(v[e]);
+        }
+    }
+    best = kFltMax;
+    arg = 0;
+    float next[DP / 16];
+    const int q = opaque(lane_id()) & 15;
+    load_spread<DP>(cg, q, next);
+#pragma unroll 1
+    for (int c = 0; c < k; ++c) {
+        float cv[DP / 16];
+#pragma unroll
+        for (int e = 0; e < DP / 16; ++e) cv[e] = next[e];
+        load_spread<DP>(cg + static_cast<int64_t>(min(c + 1, k - 1)) * DP, q, next);
+        __builtin_amdgcn_sched_barrier(0);   // above the chains, its wait below them
+        const float d = l2_lanes8_spread<DP>(x, cv, std::make_integer_sequence<int, DP>{});
+        // (a load of this round, not of the next one's values)
+#pragma unroll
+        for (int e = 0; e < DP / 16; ++e) asm volatile("" : "+v"(next[e]));
+        if (d < best) {
+            best = d;
+            arg = c;
+        }
+    }
+}
+
 template <int DP>
 struct ScreenLds {
     static constexpr int KH = DP / 32;
@@ -299,9 +418,10 @@ struct ScreenLds {
 };
 
 template <int DP, int NW, bool STREAM, int EXACT>
-__global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXACT ? 3 : 4)) void km_screen_kernel(KmParams a, int chunks) {
+__global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXACT ? 3 : DP == 32 ? 5 : 4)) void km_screen_kernel(KmParams a, int chunks) {
     constexpr int KH = DP / 32;   // 32-dim K steps per subvector
     constexpr int CS = DP + 4;    // padded fp32 row
+    constexpr bool ORIGIN = !STREAM;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int seg = blockIdx.y;
     if (a.done && a.done[seg]) return;
@@ -310,7 +430,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
     const int nct = (k + 15) >> 4;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int grp = lane >> 4;
-    // packed tiles [tile][KH][hi, lo][64 lanes], then -|c|^2 / 2 [tile][16]
+    // packed tiles [tile][KH][hi, lo][64 lanes], then f's second term [tile][16]
     const int tiles = STREAM ? 2 * kChunkTiles : nct;
     km_u32x4_t* apk = reinterpret_cast<km_u32x4_t*>(smem_raw);
     float* cch = reinterpret_cast<float*>(apk + tiles * KH * 2 * 64);
@@ -320,10 +440,15 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
     // bits of the centroid number a value carries (of its number in the chunk)
     const int nbits = STREAM ? bits_for(16 * kChunkTiles) : bits_for(nct * 16);
     const uint32_t idx_mask = ~((1u << nbits) - 1u);
-    const float e_rel = 0x1p-13f + ldexpf(1.0f, nbits - 22);
+    constexpr float e_ref = DP == 128 ? 0x1.ap-19f : DP == 64 ? 0x1.2p-19f : 0x1.bp-20f;
+    constexpr float e_sum = DP == 128 ? 0x1.4p-14f : DP == 64 ? 0x1.7p-15f : 0x1.bp-16f;
+    const float e_num = ldexpf(1.0f + 0x1p-10f, nbits - 22);
     // the lane's rows of a 16-token tile
     const uint16_t* lane_rows = kb + static_cast<int64_t>(lane & 15) * a.ts + 8 * grp;
-    float ccmax = 0.0f;   // of the lane's own centroids until the reduction
+    float ccmax = 0.0f;   // largest |c - m|^2: of the lane's own centroids until the reduction
+    float mm = 0.0f;      // |m|^2
+    float e_root = 0.0f, e_const = 0.0f;   // E's factor of sqrt(N) and its terms of C alone
+    auto scalar = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
 
     // tile ct -> slot: one wave packs it; padding centroids are zero rows
     // whose f stays at -3e38
@@ -336,21 +461,26 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
             v[2 * kh + 1] = row[8 * kh + 2 * grp + 1];
         }
     };
-    auto store_tile = [&](int ct, int slot, float4 (&v)[2 * KH]) {
+    auto store_tile = [&](int ct, int slot, float4 (&v)[2 * KH], const float4* org) {
         const bool real = 16 * ct + (lane & 15) < k;
-        float sq = 0.0f;
+        float sq = 0.0f, dot = 0.0f;
 #pragma unroll
         for (int kh = 0; kh < KH; ++kh) {
             km_u32x4_t hi, lo;
-            pack_centroid(v[2 * kh], v[2 * kh + 1], hi, lo, sq);
+            const float4 part[2] = {v[2 * kh], v[2 * kh + 1]};
+            pack_centroid<ORIGIN>(part, org + 2 * kh, hi, lo, sq, dot);
             const km_u32x4_t zero = km_u32x4_t{0u, 0u, 0u, 0u};
             apk[((slot * KH + kh) * 2 + 0) * 64 + lane] = real ? hi : zero;
             apk[((slot * KH + kh) * 2 + 1) * 64 + lane] = real ? lo : zero;
         }
         sq += xor16(sq);
         sq += xor32(sq);
+        if constexpr (ORIGIN) {
+            dot += xor16(dot);
+            dot += xor32(dot);
+        }
         if (real) ccmax = sq > ccmax || sq != sq ? sq : ccmax;   // a NaN norm stays
-        if (lane < 16) cch[slot * 16 + lane] = real ? -0.5f * sq : -3e38f;
+        if (lane < 16) cch[slot * 16 + lane] = real ? -__builtin_fmaf(0.5f, sq, dot) : -3e38f;
     };
     auto reduce_ccmax = [&](float* sh) {
         // (fmax would drop a NaN: an infinite bound stands for it)
@@ -361,7 +491,9 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         m = sh[0];
 #pragma unroll
         for (int w = 1; w < NW; ++w) m = fmaxf(m, sh[w]);
-        return m;
+        ccmax = scalar(m);
+        e_root = scalar(e_sum * 1.4142137f * __builtin_amdgcn_sqrtf(m));
+        e_const = scalar((0.5f * e_sum + e_ref) * m + 1e-30f);
     };
     const int nblk = (a.T + 64 * NW - 1) / (64 * NW);
     const int blk0 = blockIdx.x * chunks, blk1 = min(blk0 + chunks, nblk);
@@ -387,18 +519,44 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
     // later block's while the one before is re-checked and stored
     load_tokens(blk0);
     __shared__ float s_cc[NW];
+    // (distance, centroid) of a wave's tokens and its queue of (token, centroid)
+    // pairs (more than one centroid reaches the bound of many tokens)
+    __shared__ unsigned long long s_won[STREAM ? 1 : NW][64];
+    __shared__ uint16_t s_pairs[STREAM ? 1 : NW][128];
     if constexpr (!STREAM) {
-        for (int ct = wave; ct < nct; ct += NW) {
-            float4 v[2 * KH];
-            load_tile(ct, v);
-            store_tile(ct, ct, v);
+        float4 v[2 * KH], org[2 * KH], far[2 * KH];
+        load_tile(wave, v);
+        const float4* row0 = reinterpret_cast<const float4*>(cg);
+        const float4* row1 = reinterpret_cast<const float4*>(cg + static_cast<int64_t>(k / 2) * DP);
+#pragma unroll
+        for (int i = 0; i < 2 * KH; ++i) {
+            org[i] = row0[8 * (i / 2) + 2 * grp + i % 2];
+            far[i] = row1[8 * (i / 2) + 2 * grp + i % 2];
         }
+#pragma unroll
+        for (int i = 0; i < 2 * KH; ++i)
+            org[i] = make_float4(0.5f * org[i].x + 0.5f * far[i].x, 0.5f * org[i].y + 0.5f * far[i].y,
+                                 0.5f * org[i].z + 0.5f * far[i].z, 0.5f * org[i].w + 0.5f * far[i].w);
+        for (int ct = wave; ct < nct; ct += NW) {
+            store_tile(ct, ct, v, org);
+            if (ct + NW < nct) load_tile(ct + NW, v);
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * KH; ++i) {
+            mm = __builtin_fmaf(org[i].x, org[i].x, mm);
+            mm = __builtin_fmaf(org[i].y, org[i].y, mm);
+            mm = __builtin_fmaf(org[i].z, org[i].z, mm);
+            mm = __builtin_fmaf(org[i].w, org[i].w, mm);
+        }
+        mm += xor16(mm);
+        mm += xor32(mm);
+        mm = scalar(mm);
         if constexpr (EXACT == kExactLds) {
             for (int i = tid; i < k * (DP / 4); i += 64 * NW)
                 *reinterpret_cast<float4*>(cs + (i / (DP / 4)) * CS + 4 * (i % (DP / 4))) =
                     reinterpret_cast<const float4*>(cg)[i];
         }
-        ccmax = reduce_ccmax(s_cc);
+        reduce_ccmax(s_cc);
     }
 
 #pragma unroll 1
@@ -499,7 +657,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
             float4 v[2 * KH];
             load_tile(wave, v);
             __syncthreads();   // the previous block's reads are done
-            store_tile(wave, wave, v);
+            store_tile(wave, wave, v, v);
             __syncthreads();
 #pragma unroll 1
             for (int q = 0; q < nch; ++q) {
@@ -518,10 +676,10 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
                     if (top[j].s != ps[j]) chs[j] = top[j].s == pb[j] ? chb[j] : q;
                     if (top[j].b != pb[j]) chb[j] = q;
                 }
-                if (q + 1 < nch) store_tile(nxt, ((q + 1) & 1) * kChunkTiles + wave, v);
+                if (q + 1 < nch) store_tile(nxt, ((q + 1) & 1) * kChunkTiles + wave, v, v);
                 __syncthreads();
             }
-            if (blk == blk0) ccmax = reduce_ccmax(s_cc);
+            if (blk == blk0) reduce_ccmax(s_cc);
         } else {
             screen_tiles(0, nct);
         }
@@ -545,7 +703,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         swap32(xs[1], xs[3]);
         float x02 = xs[0] + xs[2], x13 = xs[1] + xs[3];
         swap16(x02, x13);
-        const float mag = (x02 + x13) + ccmax;
+        const float norms = (x02 + x13) + mm;
         Top3Ids own[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -557,8 +715,11 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         const Top3Ids m13 = swap_merge<true, STREAM>(own[1], own[3]);
         const Top3Ids mi = swap_merge<false, STREAM>(m02, m13);
         const Top3 m = mi.v;
-        const float lim = m.b - (e_rel * mag + 1e-30f);
-        const bool every = !(mag <= 1e37f) || !(m.t < lim) || m.s == m.b;
+        // E: what depends on C alone is made once
+        const float lim = m.b - ((e_root * __builtin_amdgcn_sqrtf(norms) + e_const) +
+                                 (e_num * fabsf(m.b) + e_ref * norms));
+        const bool wild = !(norms + ccmax <= 1e37f);
+        const bool every = wild || !(m.t < lim) || m.s == m.b;
         const bool pair = !every && !(m.s < lim);
         const int c1 = STREAM ? mi.ib : static_cast<int>(__float_as_uint(m.b) & ~idx_mask);
         const int c2 = STREAM ? mi.is : static_cast<int>(__float_as_uint(m.s) & ~idx_mask);
@@ -568,18 +729,82 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         // each token on its own lane
         uint64_t full = __ballot(every && valid);
         if (full) {
-            if (__popcll(full) > 8) {
-                if (every && valid) {
-                    const uint16_t* row = kb + static_cast<int64_t>(t) * a.ts;
+            if (__popcll(full) > kFewTokens) {
+                bool found = false;
+                const int fl = opaque(lane), fw = opaque(wave);
+                if constexpr (!STREAM) {
+                    // the block is screened again: the centroids that reach a
+                    // token's bound are counted and, where they are few, get
+                    // the exact distance, 64 (token, centroid) pairs at a time
+                    float lims[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        lims[j] = __shfl(every && valid ? lim : INFINITY, 16 * j + (fl & 15));
+                    auto reaching = [&](int ct) {
+                        Acc acc;
+                        products(ct, acc);
+                        uint32_t mask = 0;   // bit 4 j + r
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) mask |= acc[j][r] >= lims[j] ? 1u << (4 * j + r) : 0u;
+                        return mask;
+                    };
+                    int pairs = 0;
 #pragma unroll 1
-                    for (int c = 0; c < k; ++c) {
-                        const float d = l2_lanes8_rolled<DP>(row, cg + static_cast<int64_t>(c) * DP);
-                        if (d < best) {
-                            best = d;
-                            arg = c;
+                    for (int i = 0; i < nct; ++i) pairs += __popc(reaching(i));
+                    if (__ballot(every && valid && wild) == 0 && wave_sum_i(pairs) <= 16 * k) {
+                        s_won[fw][fl] = ~0ull;
+                        auto settle = [&](int n) {   // the queue's first n pairs
+                            wave_lds_order();
+                            if (fl < n) {
+                                const int code = s_pairs[fw][fl], tk = code >> 9, c = code & 511;
+                                const float d = l2_lanes8_rolled<DP>(kb + static_cast<int64_t>(t0 + tk) * a.ts,
+                                                                     cg + static_cast<int64_t>(c) * DP);
+                                if (d < kFltMax)
+                                    atomicMin(&s_won[fw][tk], (static_cast<unsigned long long>(__float_as_uint(d)) << 32) |
+                                                                    static_cast<uint32_t>(c));
+                            }
+                        };
+                        int nq = 0;
+#pragma unroll 1
+                        for (int i = 0; i < nct; ++i) {
+                            uint32_t mask = reaching(i);
+#pragma unroll 1
+                            while (const uint64_t has = __ballot(mask != 0)) {
+                                if (mask != 0) {
+                                    const int b = __builtin_ctz(mask);
+                                    mask &= mask - 1;
+                                    s_pairs[fw][nq + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(has >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(has), 0u))] = static_cast<uint16_t>(
+                                        (16 * (b >> 2) + (fl & 15)) << 9 | (16 * i + 4 * (fl >> 4) + (b & 3)));
+                                }
+                                nq += __popcll(has);
+                                if (nq < 64) continue;
+                                settle(64);
+                                nq -= 64;
+                                const uint16_t rest = s_pairs[fw][64 + fl];
+                                wave_lds_order();
+                                s_pairs[fw][fl] = rest;
+                            }
+                        }
+                        settle(nq);
+                        wave_lds_order();
+                        found = true;
+                        const unsigned long long key = s_won[fw][fl];
+                        if (every && key != ~0ull) {
+                            arg = static_cast<int>(static_cast<uint32_t>(key));
+                            best = __uint_as_float(static_cast<uint32_t>(key >> 32));
                         }
                     }
-                    if (!(best < kFltMax)) arg = 0;
+                }
+                if (!found) {
+                    float d;
+                    int at;
+                    nearest_of_all<DP>(kb + static_cast<int64_t>(min(t0 + fl, a.T - 1)) * a.ts, cg, k, d, at);
+                    if (every) {
+                        best = d;
+                        arg = at;
+                    }
                 }
             } else {
                 while (full) {
@@ -588,7 +813,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
                     const uint16_t* row = kb + static_cast<int64_t>(t0 + tk) * a.ts;
                     unsigned long long key = ~0ull;
 #pragma unroll 1
-                    for (int c = lane; c < k; c += 64) {
+                    for (int c = opaque(lane); c < k; c += 64) {
                         const float d = l2_lanes8_rolled<DP>(row, cg + static_cast<int64_t>(c) * DP);
                         const unsigned long long kv =
                             (static_cast<unsigned long long>(__float_as_uint(d)) << 32) | static_cast<uint32_t>(c);
@@ -633,7 +858,14 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
                 }
             }
         }
-        if (blk + 1 < blk1) load_tokens(blk + 1);
+        if (blk + 1 < blk1) {
+            load_tokens(blk + 1);
+        } else {   // (or the last block's would have to outlive the exhaustive form)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int kh = 0; kh < KH; ++kh) bq[j][kh] = km_u32x4_t{0u, 0u, 0u, 0u};
+        }
         if constexpr (EXACT == kLabelsOnly) {
             if (!every) arg = c1;
             // Tokens with two candidates, four at a time: lanes 16 i .. + 7
@@ -652,7 +884,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
                 const int tk = grp == 0 ? s[0] : grp == 1 ? s[1] : grp == 2 ? s[2] : s[3];
                 const int ca = __shfl(min(c1, c2), tk), cb = __shfl(max(c1, c2), tk);
                 const int c = lane & 8 ? cb : ca;
-                const int part = lane & 7;
+                const int part = opaque(lane) & 7;
                 const uint16_t* xrow = kb + static_cast<int64_t>(t0 + tk) * a.ts + part;
                 const float* crow = cg + static_cast<int64_t>(c) * DP + part;
                 uint16_t xv[DP / 8];
@@ -2075,8 +2307,21 @@ int launch_screen(const KmParams& p, int segs, size_t lds, hipStream_t stream) {
         per_cu <= 0)
         per_cu = 1;
     const int nblk = (p.T + 64 * NW - 1) / (64 * NW);
-    const int64_t want = static_cast<int64_t>(per_cu) * device_cus();
-    const int chunks = static_cast<int>(std::max<int64_t>(1, (static_cast<int64_t>(nblk) * segs + want - 1) / want));
+    // or one fewer per CU, where the CU with the most blocks then has at least
+    // 1/16 fewer of them (4-way at 64k tokens, 8 heads: 5 workgroups of 7 blocks
+    // on some CUs and 4 on others took 16 % longer than 4 of 8 on each)
+    int chunks = 1;
+    int64_t most = 0;
+    for (int w = per_cu; w >= std::max(1, per_cu - 1); --w) {
+        const int64_t want = static_cast<int64_t>(w) * device_cus();
+        const int64_t c = std::max<int64_t>(1, (static_cast<int64_t>(nblk) * segs + want - 1) / want);
+        const int64_t groups = (nblk + c - 1) / c * segs;
+        const int64_t blocks = (groups + device_cus() - 1) / device_cus() * c;
+        if (most == 0 || 16 * blocks <= 15 * most) {
+            chunks = static_cast<int>(c);
+            most = blocks;
+        }
+    }
     hipLaunchKernelGGL((km_screen_kernel<DP, NW, STREAM, EXACT>), dim3((nblk + chunks - 1) / chunks, segs),
                        dim3(64 * NW), lds, stream, p, chunks);
     IMI_LAUNCH_CHECK("km_screen_kernel");

@@ -22,10 +22,13 @@ def _bits(t):
 def _copies(rng, cent, form):
     """Exact ties: each of a few centroids repeated once (two candidates), or
     three times more (every centroid is searched, for a few tokens or, with
-    every centroid equal, for whole waves)."""
+    every centroid equal, for whole waves), or all of them in groups of four."""
     k = cent.shape[0]
     if form == "equal":
         cent[:] = cent[0]
+    elif form == "fours":   # every token has four candidates, in queued pairs
+        cent[:] = cent[np.arange(k) // 4 * 4]
+        cent[2::4] *= np.float32(1 + 2.0 ** -23)
     elif form != "distinct" and k >= 8:
         n = 1 if form == "pairs" else 3
         at = rng.permutation(k)
@@ -39,7 +42,9 @@ def _copies(rng, cent, form):
     (511, 17, 2, "pairs"), (1000, 64, 4, "few"), (513, 65, 2, "equal"), (777, 129, 2, "pairs"), (1025, 181, 2, "few"),
     (600, 208, 2, "distinct"), (600, 209, 2, "pairs"), (900, 257, 2, "few"), (700, 511, 2, "equal"),
     (700, 512, 2, "pairs"), (65, 1, 1, "distinct"), (130, 5, 1, "equal"), (257, 63, 1, "pairs"), (600, 64, 1, "few"),
-    (600, 65, 1, "distinct"), (500, 1018, 1, "pairs"), (300, 4095, 1, "few"), (257, 4096, 1, "equal")])
+    (600, 65, 1, "distinct"), (500, 1018, 1, "pairs"), (300, 4095, 1, "few"), (257, 4096, 1, "equal"),
+    (77, 16, 2, "fours"), (600, 62, 4, "fours"), (1000, 64, 2, "fours"), (513, 181, 2, "fours"), (515, 300, 4, "fours"),
+    (700, 512, 2, "fours"), (400, 100, 1, "fours")])
 def test_estep_edges(oracle, T, k, parts, form):
     from adaptiveimi_amd import ops, synthetic
 
@@ -54,6 +59,53 @@ def test_estep_edges(oracle, T, k, parts, form):
             sub = kf[h][:, p * Dp:(p + 1) * Dp]
             cent[h, p] = sub[rng.integers(0, T, k)] + 0.1 * cent[h, p]
             _copies(rng, cent[h, p], form)
+    kd, cd = keys.to(DEV), torch.from_numpy(cent).to(DEV)
+    plain, _ = ops.kmeans_assign(kd, cd, [k] * parts, with_distance=False)
+    labels, mind = ops.kmeans_assign(kd, cd, [k] * parts)
+    for h in range(H):
+        for p in range(parts):
+            ref, rmind, _ = oracle.estep(np.ascontiguousarray(kf[h][:, p * Dp:(p + 1) * Dp]), cent[h, p])
+            assert np.array_equal(plain[h, p].cpu().numpy(), ref), (h, p)
+            assert np.array_equal(labels[h, p].cpu().numpy(), ref), (h, p)
+            assert np.array_equal(mind[h, p].cpu().numpy(), rmind), (h, p)
+
+
+@pytest.mark.parametrize("form", ["means 10", "means 100", "channels 30", "channels 300", "ball", "lengths", "huge rows"])
+@pytest.mark.parametrize("T,k,parts", [(1030, 64, 2), (700, 181, 2), (515, 512, 2), (1000, 32, 4), (600, 250, 4),
+                                       (600, 130, 1)])
+def test_estep_undecided_tokens(oracle, T, k, parts, form):
+    """Keys on which many tokens of a wave are undecided after the screen:
+    offsets far above the spread, keys crowded around one, row lengths over
+    three decades and rows past the magnitude bound among ordinary ones.  The
+    centroids are keys and means of four, the first one (the screen's origin)
+    an ordinary or a far one."""
+    from adaptiveimi_amd import ops
+
+    print(f"[undecided] T={T} k={k} parts={parts} {form}", flush=True)
+    H, Dp = 2, 128 // parts
+    g = torch.Generator().manual_seed(T + k)
+    x = torch.randn((H, T, 128), generator=g)
+    size = float(form.split()[1]) if form[-1].isdigit() else 0.0
+    if form.startswith("means"):
+        x = x + size * torch.randn((H, 1, 128), generator=g)
+    elif form.startswith("channels"):
+        x[:, :, ::16] += size
+    elif form == "ball":
+        x = torch.where(torch.rand((1, T, 1), generator=g) < 0.6, x[:, :1] + 0.05 * x, x)
+    elif form == "lengths":
+        x = x * torch.exp(2.0 * torch.randn((H, T, 1), generator=g))
+    else:
+        x[:, torch.rand(T, generator=g) < 0.3] *= 2.0 ** 61
+    keys = x.to(torch.bfloat16)
+    kf = oracle.bf16_to_f32(_bits(keys))
+    rng = np.random.default_rng(T * 31 + k)
+    cent = np.empty((H, parts, k, Dp), np.float32)
+    for h in range(H):
+        for p in range(parts):
+            sub = kf[h][:, p * Dp:(p + 1) * Dp]
+            cent[h, p] = sub[rng.integers(0, T, k)]
+            cent[h, p, ::2] = sub[rng.integers(0, T, (cent[h, p, ::2].shape[0], 4))].mean(1)
+    cent[1, :, 0] += np.float32(50.0)
     kd, cd = keys.to(DEV), torch.from_numpy(cent).to(DEV)
     plain, _ = ops.kmeans_assign(kd, cd, [k] * parts, with_distance=False)
     labels, mind = ops.kmeans_assign(kd, cd, [k] * parts)
