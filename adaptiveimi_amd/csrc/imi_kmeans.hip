@@ -23,6 +23,7 @@
 // register rings and an LDS hand-off.
 #include <limits>
 #include <random>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -1701,6 +1702,61 @@ __global__ __launch_bounds__(1024) void km_members_kernel(KmParams a) {
     for (int i = threadIdx.x; i < m; i += blockDim.x) out[i] = base + staged[i];
 }
 
+// Empty clusters whose ordinal falls in [e0, e0 + kMoreDraws): the draws of
+// that slice (clusters beyond kDraws empty ones only occur when k > kDraws).
+// A thread per cluster (256 of them from 256 blk on) looks, its wave copies
+// the rows of those that it finds (seldom any).  768 draws are 3 KB of kernel
+// arguments: one launch up to k = 1024 (8 x 1018 clusters: 4.6 us per
+// iteration; three launches of 256 draws with a workgroup per cluster 14 us).
+constexpr int kMoreDraws = 768;
+struct MoreDraws {
+    int32_t v[kMoreDraws];
+};
+
+__device__ __forceinline__ void reseed(const KmParams& a, const MoreDraws& draws, int e0, int blk, int seg) {
+    const int c = blk * 256 + threadIdx.x;
+    const int h = seg / a.P, p = seg % a.P, lane = lane_id();
+    const int e = c < a.k[p] ? a.empties[static_cast<int64_t>(seg) * a.kmax + c] - e0 : -1;
+    for (uint64_t hit = __ballot(e >= 0 && e < kMoreDraws); hit; hit &= hit - 1) {
+        const int l = __builtin_ctzll(hit);
+        const int tok = draws.v[__builtin_amdgcn_readlane(e, l)];
+        const uint16_t* row = a.keys + h * a.hs + p * a.DP + static_cast<int64_t>(tok) * a.ts;
+        float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + (c - lane + l)) * a.DP;
+        for (int d = lane; d < a.DP; d += 64) dst[d] = bf16_to_f32(row[d]);
+    }
+}
+
+__global__ __launch_bounds__(256) void km_reseed_kernel(KmParams a, MoreDraws draws, int e0) {
+    const int seg = blockIdx.y;
+    if (a.done && a.done[seg]) return;
+    reseed(a, draws, e0, blockIdx.x, seg);
+}
+
+// Members up to which one wave sums a cluster (km_update_wave_kernel); of a
+// larger one it leaves -1 minus its size in `empties`.
+constexpr int kWaveMost = 512;
+
+// The n-th of those clusters of a segment, or -1 (every wave looks).
+__device__ __forceinline__ int nth_large(const KmParams& a, int seg, int n) {
+    const int k = a.k[seg % a.P], lane = lane_id();
+    const int32_t* size = a.empties + static_cast<int64_t>(seg) * a.kmax;
+    for (int c0 = 0; c0 < k; c0 += 256) {
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = size[min(c0 + 64 * u + lane, k - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            uint64_t hit = __ballot(v[u] < -1 && c0 + 64 * u + lane < k);
+            if (n < __popcll(hit)) {
+                for (; n > 0; --n) hit &= hit - 1;
+                return c0 + 64 * u + __builtin_ctzll(hit);
+            }
+            n -= __popcll(hit);
+        }
+    }
+    return -1;
+}
+
 // M-step, one workgroup per cluster: wave 0 keeps the chains (lane d =
 // dimension d, members in ascending token order, one dependent fp32 add
 // each) while waves 1..3 gather the member rows, so a large cluster streams
@@ -1717,9 +1773,14 @@ __global__ __launch_bounds__(1024) void km_members_kernel(KmParams a) {
 // contexts the two launches this saves cost more than the scan: at 11k
 // tokens, k = 32, 4 heads, 11.8 us against 8.3 + 4.8 us (and 3.1 us for a stop
 // test) plus the launches between.
-template <int DP, int SUPER>
-__global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws draws, int it) {
+// Draw = MoreDraws: what km_update_wave_kernel leaves, the n_th cluster of
+// more than kWaveMost members for workgroup n of the first a.T / (kWaveMost +
+// 1), and behind them the empty clusters past its draws (it: their first
+// ordinal).
+template <int DP, int SUPER, typename Draw>
+__global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draw draws, int it) {
     constexpr bool SCAN = SUPER == 0;
+    constexpr bool REST = std::is_same<Draw, MoreDraws>::value;
     constexpr int PARTS = DP / 8;    // 16-byte parts per row
     constexpr int RPL = 64 / PARTS;  // rows per load instruction
     constexpr int LPB = PARTS;       // load instructions per 64-row batch
@@ -1740,10 +1801,20 @@ __global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws 
     __shared__ int s_stop;
     __shared__ uint8_t s_seen[SCAN ? kImiMaxK : 1];
     extern __shared__ uint16_t s_list[];   // SCAN: [4][span]
-    const int c = blockIdx.x, seg = blockIdx.y;
+    const int seg = blockIdx.y;
     const int h = seg / a.P, p = seg % a.P;
-    if (c >= a.k[p]) return;
     if (a.done && a.done[seg]) return;
+    int c = blockIdx.x;
+    if constexpr (REST) {
+        const int large = gridDim.x - (a.kmax + 255) / 256;
+        if (c >= large) {
+            reseed(a, draws, it, c - large, seg);
+            return;
+        }
+        c = nth_large(a, seg, c);
+        if (c < 0) return;
+    }
+    if (c >= a.k[p]) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const uint16_t* kbase = a.keys + h * a.hs + p * DP;
     float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + c) * DP;
@@ -1825,7 +1896,7 @@ __global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws 
         __syncthreads();
     }
     const int n = (s_wt[0] + s_wt[1]) + (s_wt[2] + s_wt[3]);
-    if (n == 0) {
+    if (!REST && n == 0) {
         // the empty ordinal: labels below c with no member
         if constexpr (SCAN) {
             for (int c2 = tid; c2 < c; c2 += 256) s_seen[c2] = 0;
@@ -1851,7 +1922,7 @@ __global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws 
         }
         return;
     }
-    if (tid == 0) a.empties[static_cast<int64_t>(seg) * a.kmax + c] = -1;
+    if (!REST && tid == 0) a.empties[static_cast<int64_t>(seg) * a.kmax + c] = -1;
     const int nb = (n + 63) >> 6;              // 64-row batches
     const int rounds = (nb + NL - 1) / NL;     // = local batches of loader 1
     const int32_t* lst = a.sorted + static_cast<int64_t>(seg) * a.T;
@@ -2015,7 +2086,10 @@ __global__ __launch_bounds__(256) void km_update_block_kernel(KmParams a, Draws 
 // per cluster, lane l the chains of dims 2l and 2l + 1, kWaveRows member rows
 // (one dword per lane) in flight.  A workgroup per cluster spends its time on
 // the hand-off between its waves: 120 us per M-step for 8 x 1018 clusters of
-// 16 members.
+// 16 members, 17 us here.  Bound by its loads' latency, 65 ns per member, so a
+// cluster of more than kWaveMost members goes to a workgroup of the launch
+// that follows anyway for the re-seeding (12 ns per member): with 8k of 16k
+// keys in one cluster an M-step takes 0.12 ms, 0.5 when its wave summed it.
 constexpr int kWaveRows = 32;
 constexpr int kWaveClusters = 4;
 constexpr int kWaveMaxMean = 64;   // mean members per cluster up to which it is used
@@ -2065,7 +2139,8 @@ __global__ __launch_bounds__(64 * kWaveClusters) void km_update_wave_kernel(KmPa
         }
         return;
     }
-    if (lane == 0) *empty = -1;
+    if (lane == 0) *empty = n > kWaveMost ? -1 - n : -1;
+    if (n > kWaveMost) return;
     const int32_t* lst = a.sorted + static_cast<int64_t>(seg) * a.T;
     auto member = [&](int j) {   // as in km_update_block_kernel
         int b = 0;
@@ -2099,31 +2174,6 @@ __global__ __launch_bounds__(64 * kWaveClusters) void km_update_wave_kernel(KmPa
     }
     const float inv = 1.0f / static_cast<float>(n);
     *reinterpret_cast<float2*>(dst + 2 * lane) = make_float2(x0 * inv, x1 * inv);
-}
-
-// Empty clusters whose ordinal falls in [e0, e0 + kMoreDraws): the draws of
-// that slice (clusters beyond kDraws empty ones only occur when k > kDraws).
-// A thread per cluster looks, its wave copies the rows of those that it finds
-// (seldom any).  768 draws are 3 KB of kernel arguments: one launch up to k =
-// 1024 (8 x 1018 clusters: 4.6 us per iteration; three launches of 256 draws
-// with a workgroup per cluster 14 us).
-constexpr int kMoreDraws = 768;
-struct MoreDraws {
-    int32_t v[kMoreDraws];
-};
-
-__global__ __launch_bounds__(256) void km_reseed_kernel(KmParams a, MoreDraws draws, int e0) {
-    const int c = blockIdx.x * 256 + threadIdx.x, seg = blockIdx.y;
-    const int h = seg / a.P, p = seg % a.P, lane = lane_id();
-    if (a.done && a.done[seg]) return;
-    const int e = c < a.k[p] ? a.empties[static_cast<int64_t>(seg) * a.kmax + c] - e0 : -1;
-    for (uint64_t hit = __ballot(e >= 0 && e < kMoreDraws); hit; hit &= hit - 1) {
-        const int l = __builtin_ctzll(hit);
-        const int tok = draws.v[__builtin_amdgcn_readlane(e, l)];
-        const uint16_t* row = a.keys + h * a.hs + p * a.DP + static_cast<int64_t>(tok) * a.ts;
-        float* dst = a.cent + (static_cast<int64_t>(seg) * a.kmax + (c - lane + l)) * a.DP;
-        for (int d = lane; d < a.DP; d += 64) dst[d] = bf16_to_f32(row[d]);
-    }
 }
 
 __global__ void km_reset_kernel(KmParams a) {
@@ -2360,9 +2410,15 @@ bool scans_labels(const KmParams& p) {
     return p.DP <= 64 && p.T <= 16384 && static_cast<int64_t>(p.T) * p.kmax <= (1 << 19);
 }
 
+// Whether one wave sums a cluster (km_update_wave_kernel; the large ones are
+// left to the launches of run_rest).
+bool sums_by_wave(const KmParams& p) {
+    return p.DP == 128 && p.T <= static_cast<int64_t>(kWaveMaxMean) * p.kmax;
+}
+
 template <int DP>
 int run_update(const KmParams& p, int segs, const Draws& dr, int it, hipStream_t stream) {
-    if (DP == 128 && p.T <= static_cast<int64_t>(kWaveMaxMean) * p.kmax) {
+    if (sums_by_wave(p)) {
         const dim3 grid((p.kmax + kWaveClusters - 1) / kWaveClusters, segs);
         if (p.nsb <= 32)
             hipLaunchKernelGGL(km_update_wave_kernel<32>, grid, dim3(64 * kWaveClusters), 0, stream, p, dr);
@@ -2375,14 +2431,35 @@ int run_update(const KmParams& p, int segs, const Draws& dr, int it, hipStream_t
     if (DP <= 64 && scans_labels(p)) {
         constexpr int W = DP <= 64 ? DP : 64;
         const size_t lists = static_cast<size_t>((p.T + 255) / 256) * 512;   // beside the ring and its like
-        IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_update_block_kernel<W, 0>),
+        IMI_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&km_update_block_kernel<W, 0, Draws>),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lists)));
-        hipLaunchKernelGGL((km_update_block_kernel<W, 0>), grid, dim3(256), lists, stream, p, dr, it);
+        hipLaunchKernelGGL((km_update_block_kernel<W, 0, Draws>), grid, dim3(256), lists, stream, p, dr, it);
     } else if (p.nsb <= 32)
-        hipLaunchKernelGGL((km_update_block_kernel<DP, 32>), grid, dim3(256), 0, stream, p, dr, it);
+        hipLaunchKernelGGL((km_update_block_kernel<DP, 32, Draws>), grid, dim3(256), 0, stream, p, dr, it);
     else
-        hipLaunchKernelGGL((km_update_block_kernel<DP, kMaxSuper>), grid, dim3(256), 0, stream, p, dr, it);
+        hipLaunchKernelGGL((km_update_block_kernel<DP, kMaxSuper, Draws>), grid, dim3(256), 0, stream, p, dr, it);
     IMI_LAUNCH_CHECK("km_update_block_kernel");
+    return IMI_OK;
+}
+
+// After run_update: the clusters too large for one wave, and the draws of
+// empty ordinals kDraws and up (`draw` continues the iteration's sequence).
+template <typename Next>
+int run_rest(const KmParams& p, int segs, Next draw, hipStream_t stream) {
+    int large = sums_by_wave(p) ? p.T / (kWaveMost + 1) : 0;
+    for (int e0 = kDraws; e0 < p.kmax || large > 0; e0 += kMoreDraws) {
+        MoreDraws more;
+        for (int e = e0; e < std::min(p.kmax, e0 + kMoreDraws); ++e) more.v[e - e0] = draw();
+        const dim3 grid(large + (p.kmax + 255) / 256, segs);
+        if (large == 0)
+            hipLaunchKernelGGL(km_reseed_kernel, grid, dim3(256), 0, stream, p, more, e0);
+        else if (p.nsb <= 32)
+            hipLaunchKernelGGL((km_update_block_kernel<128, 32, MoreDraws>), grid, dim3(256), 0, stream, p, more, e0);
+        else
+            hipLaunchKernelGGL((km_update_block_kernel<128, kMaxSuper, MoreDraws>), grid, dim3(256), 0, stream, p, more, e0);
+        IMI_LAUNCH_CHECK("the launch after the M-step");
+        large = 0;
+    }
     return IMI_OK;
 }
 
@@ -2486,13 +2563,8 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
         rc = dp == 128 ? run_update<128>(p, segs, dr, it, stream)
                        : (dp == 64 ? run_update<64>(p, segs, dr, it, stream) : run_update<32>(p, segs, dr, it, stream));
         if (rc) return rc;
-        // the draws of empty ordinals kDraws and up (IVF, k > kDraws)
-        for (int e0 = kDraws; e0 < kmax; e0 += kMoreDraws) {
-            MoreDraws more;
-            for (int e = e0; e < std::min(kmax, e0 + kMoreDraws); ++e) more.v[e - e0] = dist(rng);
-            hipLaunchKernelGGL(km_reseed_kernel, dim3((kmax + 255) / 256, segs), dim3(256), 0, stream, p, more, e0);
-            IMI_LAUNCH_CHECK("km_reseed_kernel");
-        }
+        rc = run_rest(p, segs, [&] { return dist(rng); }, stream);
+        if (rc) return rc;
     }
     return IMI_OK;
 }

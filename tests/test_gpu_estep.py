@@ -144,6 +144,38 @@ def test_lloyd_over_superblock_edges(oracle, H, T, ks, stop):
             assert np.array_equal(cent[h, p, :k].cpu().numpy(), cents[p]), (h, p)
 
 
+@pytest.mark.parametrize("H,T,k,sizes", [
+    (2, 3000, 64, (512, 513, 1100)), (1, 2500, 40, (511, 512, 1400)), (1, 9000, 290, (514, 513, 515, 516, 1023, 1025, 2500)),
+    (2, 9000, 600, (513, 4097)), (1, 40001, 700, (513, 600, 20000, 512)), (1, 16000, 250, (15700,))])
+def test_large_clusters_among_small(oracle, H, T, k, sizes):
+    """IVF clusters around the size that one wave sums, far larger ones, several
+    per segment, with fewer and more re-seeded clusters than the draws of one
+    launch, and more than 32 superblocks: copies of the first rows, so that
+    the sizes are what they are set to."""
+    from adaptiveimi_amd import ops
+
+    print(f"[large clusters] H={H} T={T} k={k} sizes={sizes}", flush=True)
+    rng = np.random.default_rng(T + k)
+    at = np.empty((H, T), np.int64)
+    for h in range(H):
+        own = rng.permutation(k)[:len(sizes)]
+        rest = np.concatenate([np.full(n - 1, c) for n, c in zip(sizes, own)])
+        small = np.setdiff1d(np.arange(k), own)
+        # half of the others stay alone
+        small = np.concatenate([rest, rng.choice(small[:max(1, len(small) // 2)], T - k - len(rest))])
+        at[h] = np.concatenate([np.arange(k), rng.permutation(small)])
+    rows = torch.randn((H, k, 128), generator=torch.Generator().manual_seed(k)).to(torch.bfloat16)
+    if k > 256:   # two thirds of the rows equal: more than 256 empty clusters at k = 600 and 700
+        rows[:, k // 3:] = rows[:, :1]
+    keys = torch.gather(rows, 1, torch.from_numpy(at)[..., None].expand(-1, -1, 128))
+    cent, labels, _ = ops.kmeans(keys.to(DEV), [k], 2)
+    kf = oracle.bf16_to_f32(_bits(keys))
+    for h in range(H):
+        labs, cents, _ = oracle.kmeans_head(kf[h], [k], 2)
+        assert np.array_equal(labels[h, 0].cpu().numpy(), labs[0]), h
+        assert np.array_equal(cent[h, 0, :k].cpu().numpy(), cents[0]), h
+
+
 @pytest.mark.parametrize("H,T,k", [(1, 1500, 296), (2, 1500, 297), (1, 2000, 1064), (1, 2000, 1065), (2, 2000, 1900)])
 def test_reseed_slices(oracle, H, T, k):
     """40 distinct rows leave k - 40 clusters empty: around the 256 draws of the
