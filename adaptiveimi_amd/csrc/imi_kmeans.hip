@@ -237,8 +237,8 @@ __device__ __forceinline__ float max_raw(float a, float b) {
 }
 
 // One lane's share of a 16-centroid tile: dims 32 kh + 8 (lane / 16) .. + 7 of
-// centroid 16 ct + lane % 16, less the origin's (ORIGIN), as hi and lo bf16
-// operands; sq += the dims' squares, dot += their products with the origin's.
+// centroid 16 ct + lane % 16, less the origin's (ORIGIN: half of org), as hi
+// and lo bf16 operands; sq += the dims' squares, dot += their products with org.
 template <bool ORIGIN>
 __device__ __forceinline__ void pack_centroid(const float4 (&c)[2], const float4* org, km_u32x4_t& hi, km_u32x4_t& lo,
                                               float& sq, float& dot) {
@@ -247,7 +247,7 @@ __device__ __forceinline__ void pack_centroid(const float4 (&c)[2], const float4
         const float m[8] = {org[0].x, org[0].y, org[0].z, org[0].w, org[1].x, org[1].y, org[1].z, org[1].w};
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            v[i] = v[i] - m[i];
+            v[i] = __builtin_fmaf(-0.5f, m[i], v[i]);
             dot = __builtin_fmaf(v[i], m[i], dot);
         }
     }
@@ -448,8 +448,10 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
     const uint16_t* lane_rows = kb + static_cast<int64_t>(lane & 15) * a.ts + 8 * grp;
     float ccmax = 0.0f;   // largest |c - m|^2: of the lane's own centroids until the reduction
     float mm = 0.0f;      // |m|^2
-    float e_root = 0.0f, e_const = 0.0f;   // E's factor of sqrt(N) and its terms of C alone
-    auto scalar = [](float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); };
+    // what E takes from the centroids: the factor of sqrt(N), the terms of C
+    // alone, the factor of |best|; C^2 (read where they are used: in registers
+    // they would spill)
+    __shared__ float4 s_bound[1];
 
     // tile ct -> slot: one wave packs it; padding centroids are zero rows
     // whose f stays at -3e38
@@ -481,7 +483,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
             dot += xor32(dot);
         }
         if (real) ccmax = sq > ccmax || sq != sq ? sq : ccmax;   // a NaN norm stays
-        if (lane < 16) cch[slot * 16 + lane] = real ? -__builtin_fmaf(0.5f, sq, dot) : -3e38f;
+        if (lane < 16) cch[slot * 16 + lane] = real ? -0.5f * (sq + dot) : -3e38f;
     };
     auto reduce_ccmax = [&](float* sh) {
         // (fmax would drop a NaN: an infinite bound stands for it)
@@ -492,9 +494,10 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         m = sh[0];
 #pragma unroll
         for (int w = 1; w < NW; ++w) m = fmaxf(m, sh[w]);
-        ccmax = scalar(m);
-        e_root = scalar(e_sum * 1.4142137f * __builtin_amdgcn_sqrtf(m));
-        e_const = scalar((0.5f * e_sum + e_ref) * m + 1e-30f);
+        ccmax = m;
+        // (every wave writes the values it reads)
+        s_bound[0] = make_float4(e_sum * 1.4142137f * __builtin_amdgcn_sqrtf(m), (0.5f * e_sum + e_ref) * m + 1e-30f, e_num, m);
+        wave_lds_order();
     };
     const int nblk = (a.T + 64 * NW - 1) / (64 * NW);
     const int blk0 = blockIdx.x * chunks, blk1 = min(blk0 + chunks, nblk);
@@ -507,9 +510,10 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 #pragma unroll
         for (int j = 0; j < 4; ++j) src[j] = lane_rows + static_cast<int64_t>(t0 + 16 * j) * a.ts;
         if (t0 + 64 > a.T) {
+            const int l = opaque(lane);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                src[j] = kb + static_cast<int64_t>(min(t0 + 16 * j + (lane & 15), a.T - 1)) * a.ts + 8 * grp;
+                src[j] = kb + static_cast<int64_t>(min(t0 + 16 * j + (l & 15), a.T - 1)) * a.ts + 8 * (l >> 4);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -536,8 +540,11 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         }
 #pragma unroll
         for (int i = 0; i < 2 * KH; ++i)
-            org[i] = make_float4(0.5f * org[i].x + 0.5f * far[i].x, 0.5f * org[i].y + 0.5f * far[i].y,
-                                 0.5f * org[i].z + 0.5f * far[i].z, 0.5f * org[i].w + 0.5f * far[i].w);
+            org[i] = make_float4(org[i].x + far[i].x, org[i].y + far[i].y, org[i].z + far[i].z, org[i].w + far[i].w);
+        // (the tile's loads stay above, beside the origin's)
+#pragma unroll
+        for (int i = 0; i < 2 * KH; ++i) asm volatile("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));
+#pragma unroll 1
         for (int ct = wave; ct < nct; ct += NW) {
             store_tile(ct, ct, v, org);
             if (ct + NW < nct) load_tile(ct + NW, v);
@@ -551,7 +558,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         }
         mm += xor16(mm);
         mm += xor32(mm);
-        mm = scalar(mm);
+        mm = 0.25f * __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mm)));
         if constexpr (EXACT == kExactLds) {
             for (int i = tid; i < k * (DP / 4); i += 64 * NW)
                 *reinterpret_cast<float4*>(cs + (i / (DP / 4)) * CS + 4 * (i % (DP / 4))) =
@@ -704,6 +711,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         swap32(xs[1], xs[3]);
         float x02 = xs[0] + xs[2], x13 = xs[1] + xs[3];
         swap16(x02, x13);
+        const float4 e = s_bound[opaque(0)];
         const float norms = (x02 + x13) + mm;
         Top3Ids own[4];
 #pragma unroll
@@ -716,10 +724,8 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
         const Top3Ids m13 = swap_merge<true, STREAM>(own[1], own[3]);
         const Top3Ids mi = swap_merge<false, STREAM>(m02, m13);
         const Top3 m = mi.v;
-        // E: what depends on C alone is made once
-        const float lim = m.b - ((e_root * __builtin_amdgcn_sqrtf(norms) + e_const) +
-                                 (e_num * fabsf(m.b) + e_ref * norms));
-        const bool wild = !(norms + ccmax <= 1e37f);
+        const float lim = m.b - ((e.x * __builtin_amdgcn_sqrtf(norms) + e.y) + (e.z * fabsf(m.b) + e_ref * norms));
+        const bool wild = !(norms + e.w <= 1e37f);
         const bool every = wild || !(m.t < lim) || m.s == m.b;
         const bool pair = !every && !(m.s < lim);
         const int c1 = STREAM ? mi.ib : static_cast<int>(__float_as_uint(m.b) & ~idx_mask);
