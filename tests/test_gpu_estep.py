@@ -207,6 +207,11 @@ def _awkward(keys, form):
         k *= 2.0 ** -70
     elif form == "flat":        # no dominant channels: the copy's second half is read
         k = torch.randn(k.shape, generator=torch.Generator().manual_seed(7))
+    elif form == "lengths":     # distances over too many binades for exact partial sums
+        k *= torch.exp(2.0 * torch.randn(k.shape[:2], generator=torch.Generator().manual_seed(9)))[..., None]
+    elif form == "steps":       # the same, the largest distances in one run of rows
+        k[:, :k.shape[1] // 3] *= 2.0 ** -9
+        k[:, k.shape[1] // 2:k.shape[1] // 2 + 70] *= 2.0 ** 9
     elif form == "zero":        # a whole group of zero rows
         k[:, 256:1300] = 0.0
     return k.to(torch.bfloat16)
@@ -217,12 +222,15 @@ def _awkward(keys, form):
     (8, 9000, (6, 6), "tiny"), (8, 10240, (8, 30), "zero"), (1, 70001, (16, 3), ""), (8, 9000, (17, 2, 30, 1), ""),
     (8, 9007, (11, 11, 11, 11), "outliers"), (8, 8300, (70,), ""), (8, 9000, (20,), "outliers"), (1, 300100, (9, 4), ""),
     (8, 9001, (23, 40), "flat"), (8, 8300, (9, 12, 4, 17), "flat"), (8, 9003, (30,), "flat"), (1, 70001, (12, 40), "flat"),
-    (2, 4100, (33, 64), ""), (2, 257, (20, 1), ""), (1, 255, (64,), "duplicates")])
+    (2, 4100, (33, 64), ""), (2, 257, (20, 1), ""), (1, 255, (64,), "duplicates"),
+    (8, 9001, (9, 12), "lengths"), (8, 9000, (11,), "steps"), (8, 8200, (5, 9, 3, 8), "lengths"), (2, 4095, (20, 9), "lengths"),
+    (2, 4097, (17,), "steps"), (1, 63, (5, 4), "lengths"), (1, 65, (6, 6), "steps"), (1, 70001, (7, 5), "steps")])
 def test_plusplus_screened_rows(oracle, H, T, ks, form):
     """kmeans++ picks with the rows screened over their 8-bit copy (16 MB of
     keys and more: 64, 32 and 128 dims, ragged blocks, more blocks than one
-    search round, one or both halves of the copied dims) and below: one Lloyd iteration from the seeds equals the
-    oracle's, so every pick does."""
+    search round, one or both halves of the copied dims, sums that only the
+    sequential loops give) and below: one Lloyd iteration from the seeds equals
+    the oracle's, so every pick does."""
     from adaptiveimi_amd import ops, synthetic
 
     print(f"[kmeans++] H={H} T={T} ks={ks} {form}", flush=True)
