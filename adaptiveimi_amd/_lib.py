@@ -103,6 +103,7 @@ EXPORTS = {
     "imi_last_error": (ctypes.c_char_p, []),
     "imi_version": (ctypes.c_int, []),
     "imi_kmeans_workspace_size": (ctypes.c_int, [ctypes.POINTER(KmeansArgs), ctypes.POINTER(ctypes.c_size_t)]),
+    "imi_kmeans_min_workspace_size": (ctypes.c_int, [ctypes.POINTER(KmeansArgs), ctypes.POINTER(ctypes.c_size_t)]),
     "imi_kmeans_execute": (ctypes.c_int, [ctypes.POINTER(KmeansArgs), _vp]),
     "imi_kmeans_assign": (ctypes.c_int, [_vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp]),
     "imi_index_workspace_size": (ctypes.c_int, [ctypes.POINTER(IndexArgs), ctypes.POINTER(ctypes.c_size_t)]),

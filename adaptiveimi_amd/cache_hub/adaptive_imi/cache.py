@@ -408,6 +408,8 @@ class adpimi_cache:  # noqa: N801  (reference class name)
         self.buffer_size = sz["buffer_pages"]
         self.buffer_budget_pages = self.buffer_size
         self.execution_stride = self.buffer_size * self.page_size + self.static_capacity   # runtime.py:62
+        for dev in {c.device for c in self.centroids if c is not None}:
+            ops.release_build_workspaces(dev, self._build_stream)   # every layer's build is enqueued
         self.cache_prepared = True
 
     def _update_state(self, layer_idx: int) -> Optional[ops.OnlineUpdate]:

@@ -2362,7 +2362,13 @@ int seed_plusplus(const KmParams& p, const imi_kmeans_args* a, int segs, int gro
                          : run_plusplus<DP, 0>(p, a, segs, stream);
 }
 
-size_t workspace_bytes(const imi_kmeans_args* a, int kmax, KmParams* out) {
+// Whether a run's kmeans++ would screen its rows.
+bool seeds_screened(const imi_kmeans_args* a) {
+    return a->init_mode == 2 && pp_screened(a->n_tokens, a->kv_heads * a->parts, a->dim / a->parts);
+}
+
+// screened: with the 8-bit copy of a screened kmeans++ (seeds_screened).
+size_t workspace_bytes(const imi_kmeans_args* a, int kmax, bool screened, KmParams* out) {
     const int segs = a->kv_heads * a->parts;
     const int nblk = (a->n_tokens + 255) / 256;
     Carver cv(a->workspace);
@@ -2376,7 +2382,6 @@ size_t workspace_bytes(const imi_kmeans_args* a, int kmax, KmParams* out) {
     p.done = cv.take<int32_t>(segs);
     if (a->init_mode == 2) {
         const int dp = a->dim / a->parts;
-        const bool screened = pp_screened(a->n_tokens, segs, dp);
         const size_t rows = 256 * (screened ? pp_groups(a->n_tokens, segs) : 1);   // per block
         const size_t blocks = (a->n_tokens + rows - 1) / rows * segs;
         p.ppstats = cv.take<PpBlock>(2 * blocks);   // two launches' worth
@@ -2528,7 +2533,7 @@ int run_members(const KmParams& p, int segs, hipStream_t stream) {
 
 using namespace imi;
 
-extern "C" int imi_kmeans_workspace_size(const imi_kmeans_args* a, size_t* bytes) {
+static int kmeans_workspace_size(const imi_kmeans_args* a, size_t* bytes, bool least) {
     clear_error();
     int kmax, dp;
     int rc = validate(a, kmax, dp);
@@ -2536,8 +2541,16 @@ extern "C" int imi_kmeans_workspace_size(const imi_kmeans_args* a, size_t* bytes
     IMI_REQUIRE(bytes != nullptr, IMI_ERR_INVALID, "imi_kmeans_workspace_size: null output");
     imi_kmeans_args tmp = *a;
     tmp.workspace = nullptr;
-    *bytes = workspace_bytes(&tmp, kmax, nullptr);
+    *bytes = workspace_bytes(&tmp, kmax, !least && seeds_screened(a), nullptr);
     return IMI_OK;
+}
+
+extern "C" int imi_kmeans_workspace_size(const imi_kmeans_args* a, size_t* bytes) {
+    return kmeans_workspace_size(a, bytes, false);
+}
+
+extern "C" int imi_kmeans_min_workspace_size(const imi_kmeans_args* a, size_t* bytes) {
+    return kmeans_workspace_size(a, bytes, true);
 }
 
 extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_) {
@@ -2548,12 +2561,13 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
     if (rc) return rc;
     imi_kmeans_args tmp = *a;
     tmp.workspace = nullptr;
-    const size_t need = workspace_bytes(&tmp, kmax, nullptr);
+    const size_t need = workspace_bytes(&tmp, kmax, false, nullptr);
     IMI_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= need, IMI_ERR_WORKSPACE,
                 "imi_kmeans_execute: workspace %zu bytes < %zu required", a->workspace_bytes, need);
+    const bool screened = seeds_screened(a) && a->workspace_bytes >= workspace_bytes(&tmp, kmax, true, nullptr);
 
     KmParams p;
-    workspace_bytes(a, kmax, &p);
+    workspace_bytes(a, kmax, screened, &p);
     p.keys = a->keys;
     p.hs = a->head_stride;
     p.ts = a->token_stride;
@@ -2582,7 +2596,7 @@ extern "C" int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream_
         hipLaunchKernelGGL(km_init_first_kernel, dim3(kmax, segs), dim3(64), 0, stream, p);
         IMI_LAUNCH_CHECK("km_init_first_kernel");
     } else if (a->init_mode == 2) {
-        const int groups = pp_screened(a->n_tokens, segs, dp) ? pp_groups(a->n_tokens, segs) : 0;
+        const int groups = screened ? pp_groups(a->n_tokens, segs) : 0;
         rc = dp == 128 ? seed_plusplus<128>(p, a, segs, groups, stream)
                        : (dp == 64 ? seed_plusplus<64>(p, a, segs, groups, stream)
                                    : seed_plusplus<32>(p, a, segs, groups, stream));

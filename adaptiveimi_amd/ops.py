@@ -2,8 +2,8 @@
 
 All tensors must live on a HIP device; every call enqueues on the current
 torch stream and returns without a host synchronisation.  Workspaces come
-from the torch caching allocator and are zero-filled once on allocation (the
-kernels leave them reusable).
+from the torch caching allocator and, where the kernels need it, are
+zero-filled once on allocation (the kernels leave them reusable).
 """
 from __future__ import annotations
 
@@ -39,17 +39,42 @@ def _require_device(*ts: torch.Tensor) -> torch.device:
     return dev
 
 
-def workspace(name: str, nbytes: int, device: torch.device) -> torch.Tensor:
-    """Zero-filled byte buffer reused across calls (grown on demand), one per
-    (name, device, stream): calls on one stream are ordered, calls on two
-    streams (an index build on a side stream) never share a buffer."""
-    key = (name, device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream)
+def _workspace_key(name: str, device: torch.device, stream: Optional[torch.cuda.Stream] = None):
+    stream = torch.cuda.current_stream(device) if stream is None else stream
+    return name, device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream
+
+
+def workspace(name: str, nbytes: int, device: torch.device, zero: bool = True) -> torch.Tensor:
+    """Byte buffer reused across calls (grown on demand, zero-filled unless
+    ``zero=False``), one per (name, device, stream): calls on one stream are
+    ordered, calls on two streams (an index build on a side stream) never
+    share a buffer.  ``release_build_workspaces`` gives the build's back."""
+    key = _workspace_key(name, device)
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
-        buf = torch.zeros(max(int(nbytes), 256), dtype=torch.uint8, device=device)
+        del buf
+        _WS.pop(key, None)   # before its successor is allocated
+        make = torch.zeros if zero else torch.empty
+        buf = make(max(int(nbytes), 256), dtype=torch.uint8, device=device)
         _WS[key] = buf
     return buf
+
+
+# Build workspaces up to this size are kept (short prompts would pay for the
+# allocation with every cache, 1 % of a 2-layer 8k prefill).
+_KEEP_BYTES = 16 << 20
+
+
+def release_build_workspaces(device: torch.device, stream: Optional[torch.cuda.Stream] = None) -> None:
+    """Give the index build's large workspaces of a stream (the current one)
+    back to torch's allocator: after a prefill nothing reads them, and kmeans++
+    keeps an 8-bit copy of one layer's keys in them (8 x 128k tokens: 0.17 GB
+    in all).  Work enqueued on that stream still uses them safely."""
+    for name in ("kmeans", "index"):
+        key = _workspace_key(name, device, stream)
+        buf = _WS.get(key)
+        if buf is not None and buf.numel() > _KEEP_BYTES:
+            _WS.pop(key, None)
 
 
 def _ks(ks: Sequence[int]):
@@ -107,7 +132,15 @@ def kmeans(keys: torch.Tensor, ks: Sequence[int], max_iters: int, tol: float = 5
                    centroids=cent.data_ptr(), labels=labels.data_ptr(), iters_run=iters.data_ptr())
     need = ctypes.c_size_t()
     check(_lib.lib().imi_kmeans_workspace_size(ctypes.byref(a), ctypes.byref(need)), "imi_kmeans_workspace_size")
-    ws = workspace("kmeans", need.value, dev)
+    try:
+        ws = workspace("kmeans", need.value, dev, zero=False)
+    except torch.OutOfMemoryError:   # kmeans++ without its 8-bit copy: slower, the same picks
+        least = ctypes.c_size_t()
+        check(_lib.lib().imi_kmeans_min_workspace_size(ctypes.byref(a), ctypes.byref(least)),
+              "imi_kmeans_min_workspace_size")
+        if least.value >= need.value:
+            raise
+        ws = workspace("kmeans", least.value, dev, zero=False)
     a.workspace = ws.data_ptr()
     a.workspace_bytes = ws.numel()
     check(_lib.lib().imi_kmeans_execute(ctypes.byref(a), _stream(dev)), "imi_kmeans_execute")
@@ -207,7 +240,7 @@ def build_index(keys: torch.Tensor, values: torch.Tensor, centroids: torch.Tenso
             a.compact_mask = out["compact_mask"].data_ptr()
     need = ctypes.c_size_t()
     check(_lib.lib().imi_index_workspace_size(ctypes.byref(a), ctypes.byref(need)), "imi_index_workspace_size")
-    ws = workspace("index", need.value, dev)
+    ws = workspace("index", need.value, dev, zero=False)
     a.workspace = ws.data_ptr()
     a.workspace_bytes = ws.numel()
     check(_lib.lib().imi_build_index(ctypes.byref(a), _stream(dev)), "imi_build_index")

@@ -81,11 +81,16 @@ typedef struct {
     float* centroids;         /* device [H][P][kmax][Dp] in/out */
     int32_t* labels;          /* device [H][P][T] out (last E-step) */
     int32_t* iters_run;       /* device [H][P] out (E-steps executed), may be NULL */
-    void* workspace;          /* device, >= imi_kmeans_workspace_size() bytes */
+    void* workspace;          /* device, >= imi_kmeans_min_workspace_size() bytes */
     size_t workspace_bytes;
 } imi_kmeans_args;
 
+/* The size to allocate, and the least that imi_kmeans_execute takes.  They
+ * differ for kmeans++ from 16 MB of keys on, where the seeding screens the
+ * rows over an 8-bit copy (half of the keys and 8 bytes per row and subspace
+ * more); with less it reads the keys in every pick, for the same picks. */
 int imi_kmeans_workspace_size(const imi_kmeans_args* a, size_t* bytes);
+int imi_kmeans_min_workspace_size(const imi_kmeans_args* a, size_t* bytes);
 int imi_kmeans_execute(const imi_kmeans_args* a, imi_stream_t stream);
 
 /* One assignment pass with given centroids (the E-step of

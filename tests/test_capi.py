@@ -80,6 +80,19 @@ def test_kmeans_workspace_and_too_small_workspace(L):
     assert "workspace" in L.imi_last_error().decode()
 
 
+def test_kmeans_least_workspace(L):
+    size, least = ctypes.c_size_t(), ctypes.c_size_t()
+    for over, copied in ((dict(), 0), (dict(init_mode=2), 0), (dict(n_tokens=131072), 0),
+                         (dict(n_tokens=131072, init_mode=2), 8 * 131072 * (128 + 2 * 8))):
+        a = _kmeans_args(**over)
+        assert L.imi_kmeans_workspace_size(ctypes.byref(a), ctypes.byref(size)) == 0
+        assert L.imi_kmeans_min_workspace_size(ctypes.byref(a), ctypes.byref(least)) == 0
+        assert copied * 0.95 <= size.value - least.value <= copied * 1.05   # the 8-bit copy and two norms per row
+        a.workspace, a.workspace_bytes = 256, least.value - 1
+        assert L.imi_kmeans_execute(ctypes.byref(a), None) == 4
+        assert "workspace" in L.imi_last_error().decode()
+
+
 def test_select_and_decode_argument_checks(L):
     from adaptiveimi_amd._lib import AttentionArgs, DecodeArgs, SelectArgs
 
