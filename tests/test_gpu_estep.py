@@ -2,8 +2,9 @@
 can go wrong: centroid counts around a 16-centroid tile, a streamed chunk and
 the largest k of each width; tokens with exactly two candidates, with more (a
 few per wave and whole waves), and token counts around a wave, a workgroup
-and a superblock.  Labels, distances and centroids equal the oracle's bit for
-bit (the results are defined exactly, so there is no tolerance)."""
+and a superblock.  kmeans++ with its rows screened, the M-step's forms and the
+re-seeding.  Labels, distances and centroids equal the oracle's bit for bit
+(the results are defined exactly, so there is no tolerance)."""
 import numpy as np
 import pytest
 import torch
@@ -70,6 +71,30 @@ def test_estep_edges(oracle, T, k, parts, form):
             assert np.array_equal(mind[h, p].cpu().numpy(), rmind), (h, p)
 
 
+@pytest.mark.parametrize("H,T,k", [(16, 9001, 130), (16, 8449, 64), (4, 66000, 33)])
+def test_estep_ivf_several_blocks_per_workgroup(oracle, H, T, k):
+    """128 dims over more token blocks than the device holds at once: each
+    workgroup streams the centroids again for its next block (the last one
+    ragged, with waves past the last token that keep to the barriers)."""
+    from adaptiveimi_amd import ops, synthetic
+
+    print(f"[ivf blocks] H={H} T={T} k={k}", flush=True)
+    assert -(-T // 256) * H > 512   # two workgroups on each of 256 CUs
+    keys, _ = synthetic.make_kv(H, T, seed=T + k)
+    kf = oracle.bf16_to_f32(_bits(keys))
+    rng = np.random.default_rng(T + k)
+    cent = np.stack([kf[h][rng.integers(0, T, (k, 3))].mean(1) for h in range(H)])[:, None].astype(np.float32)
+    cent[:, :, 7 % k] = cent[:, :, 2]
+    kd, cd = keys.to(DEV), torch.from_numpy(cent).to(DEV)
+    plain, _ = ops.kmeans_assign(kd, cd, [k], with_distance=False)
+    labels, mind = ops.kmeans_assign(kd, cd, [k])
+    for h in range(H):
+        ref, rmind, _ = oracle.estep(kf[h], cent[h, 0])
+        assert np.array_equal(plain[h, 0].cpu().numpy(), ref), h
+        assert np.array_equal(labels[h, 0].cpu().numpy(), ref), h
+        assert np.array_equal(mind[h, 0].cpu().numpy(), rmind), h
+
+
 @pytest.mark.parametrize("form", ["means 10", "means 100", "channels 30", "channels 300", "ball", "lengths", "huge rows"])
 @pytest.mark.parametrize("T,k,parts", [(1030, 64, 2), (700, 181, 2), (515, 512, 2), (1000, 32, 4), (600, 250, 4),
                                        (600, 130, 1)])
@@ -122,7 +147,7 @@ def test_estep_undecided_tokens(oracle, T, k, parts, form):
     (1, 4097, (8, 8, 5, 3), True), (8, 36000, (64, 64), False), (8, 70001, (45, 20), True), (1, 2050, (300,), False),
     (2, 1030, (700,), True), (1, 530000, (4, 3), False), (2, 16384, (32, 5), True), (2, 16385, (32, 5), True),
     (2, 4096, (128, 60), False), (2, 4097, (128, 60), False), (1, 300, (200, 256), True), (2, 8000, (125,), True),
-    (2, 8001, (125,), False)])
+    (2, 8001, (125,), False), (1, 40001, (300,), False), (1, 40001, (640,), True)])
 def test_lloyd_over_superblock_edges(oracle, H, T, ks, stop):
     """Two Lloyd iterations (labels, member order and sums) around the
     superblocks' sizes (one of 1024 tokens, several, 8192 tokens each, more of
@@ -221,6 +246,10 @@ def _awkward(keys, form):
     (8, 9001, (37, 20), ""), (8, 8193, (9, 9), "outliers"), (8, 9000, (45, 45), "duplicates"), (8, 8999, (12, 5), "huge"),
     (8, 9000, (6, 6), "tiny"), (8, 10240, (8, 30), "zero"), (1, 70001, (16, 3), ""), (8, 9000, (17, 2, 30, 1), ""),
     (8, 9007, (11, 11, 11, 11), "outliers"), (8, 8300, (70,), ""), (8, 9000, (20,), "outliers"), (1, 300100, (9, 4), ""),
+    # several blocks per workgroup, four groups of 256 rows each (64, 32 and 128 dims)
+    (8, 131100, (5, 4), ""), (8, 131100, (4, 5), "flat"), (8, 131100, (4, 4), "outliers"),
+    (8, 70001, (4, 5, 3, 4), ""), (8, 70001, (3, 4, 4, 3), "flat"), (8, 70001, (4, 3, 3, 4), "outliers"),
+    (16, 60001, (5,), ""), (16, 60001, (5,), "flat"), (16, 60001, (4,), "outliers"),
     (8, 9001, (23, 40), "flat"), (8, 8300, (9, 12, 4, 17), "flat"), (8, 9003, (30,), "flat"), (1, 70001, (12, 40), "flat"),
     (2, 4100, (33, 64), ""), (2, 257, (20, 1), ""), (1, 255, (64,), "duplicates"),
     (8, 9001, (9, 12), "lengths"), (8, 9000, (11,), "steps"), (8, 8200, (5, 9, 3, 8), "lengths"), (2, 4095, (20, 9), "lengths"),
