@@ -529,8 +529,7 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
     __shared__ unsigned long long s_won[STREAM ? 1 : NW][64];
     __shared__ uint16_t s_pairs[STREAM ? 1 : NW][128];
     if constexpr (!STREAM) {
-        float4 v[2 * KH], org[2 * KH], far[2 * KH];
-        load_tile(wave, v);
+        float4 org[2 * KH], far[2 * KH];
         const float4* row0 = reinterpret_cast<const float4*>(cg);
         const float4* row1 = reinterpret_cast<const float4*>(cg + static_cast<int64_t>(k / 2) * DP);
 #pragma unroll
@@ -541,13 +540,10 @@ __global__ __launch_bounds__(64 * NW, (STREAM || EXACT == kExactGlobal ? 2 : EXA
 #pragma unroll
         for (int i = 0; i < 2 * KH; ++i)
             org[i] = make_float4(org[i].x + far[i].x, org[i].y + far[i].y, org[i].z + far[i].z, org[i].w + far[i].w);
-        // (the tile's loads stay above, beside the origin's)
-#pragma unroll
-        for (int i = 0; i < 2 * KH; ++i) asm volatile("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));
-#pragma unroll 1
         for (int ct = wave; ct < nct; ct += NW) {
+            float4 v[2 * KH];
+            load_tile(ct, v);
             store_tile(ct, ct, v, org);
-            if (ct + NW < nct) load_tile(ct + NW, v);
         }
 #pragma unroll
         for (int i = 0; i < 2 * KH; ++i) {
@@ -1086,46 +1082,41 @@ __device__ __forceinline__ int pp_first_reaching(const double (&v)[PER], double 
 // load, four loads ahead, each row added from its lane.  Both loops have the
 // same running sums, so the second starts at the 64th part of the rows that
 // the target lies in (their sums before are kept, one per lane).
-// Bound by the chain of double additions: 21 ns per row, 2.8 ms per pick at
+// Bound by the chain of double additions: 23 ns per row, 3 ms per pick at
 // 128k tokens, 16 segments (one lane with a load per addition: 20 ms; the same
 // in a workgroup of 256 threads: 11 ms).
 __device__ __forceinline__ int pp_sequential_row(const float* md, int T, double canon) {
-    constexpr int AHEAD = 4;
+    constexpr int AHEAD = 4, STEP = 16;
     const int lane = lane_id();
-    const int part = (T + 64 * 64 * AHEAD - 1) / (64 * 64 * AHEAD) * 64 * AHEAD;   // rows per lane's part
+    const int part = (T + 4095) / 4096 * 64;   // rows per lane's part
     double sum = 0.0, before = 0.0, target = INFINITY;
     int first = 0, last = T;
-    float next[AHEAD];
-    const auto load = [&](int i) {   // (a zero changes no sum)
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u) next[u] = i + 64 * u + lane < T ? md[i + 64 * u + lane] : 0.0f;
-    };
+    const auto load = [&](int i) { return i + lane < T ? md[i + lane] : 0.0f; };   // (a zero changes no sum)
 #pragma unroll 1
     for (int pass = 0; pass < 2; ++pass) {
-        load(first);
-#pragma unroll 1
-        for (int i = first; i < last; i += 64 * AHEAD) {
-            float v[AHEAD];
+        float next[AHEAD];
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) v[u] = next[u];
-            load(i + 64 * AHEAD);
+        for (int u = 0; u < AHEAD; ++u) next[u] = load(first + 64 * u);
+#pragma unroll 1
+        for (int i = first; i < last; i += 64) {
+            const float v = next[0];
+#pragma unroll
+            for (int u = 0; u + 1 < AHEAD; ++u) next[u] = next[u + 1];
+            next[AHEAD - 1] = load(i + 64 * AHEAD);
             if (i % part == 0 && lane == i / part) before = sum;
-#pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {
-                const auto row = [&](int j) {
-                    return static_cast<double>(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[u]), j)));
-                };
+            const auto row = [&](int j) {
+                return static_cast<double>(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)));
+            };
 #pragma unroll 1
-                for (int j0 = 0; j0 < 64; j0 += 16) {
-                    double s = sum;
+            for (int j0 = 0; j0 < 64; j0 += STEP) {
+                double s = sum;
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) sum += row(j0 + j);
-                    if (sum < target) continue;
+                for (int j = 0; j < STEP; ++j) sum += row(j0 + j);
+                if (sum < target) continue;
 #pragma unroll 1
-                    for (int j = 0; j < 16; ++j) {
-                        s += row(j0 + j);
-                        if (s >= target) return i + 64 * u + j0 + j;
-                    }
+                for (int j = 0; j < STEP; ++j) {
+                    s += row(j0 + j);
+                    if (s >= target) return i + j0 + j;
                 }
             }
         }
@@ -1138,6 +1129,14 @@ __device__ __forceinline__ int pp_sequential_row(const float* md, int T, double 
         sum = at > 0 ? readlane_f64(before, at) : 0.0;
     }
     return 0;
+}
+
+// As a call, where the code in line made every pick longer (it is seldom
+// run, but a pick is short: 6.24 against 6.55 us at 8k tokens, 6.8 against 7.0
+// over 128 dims at 16k); with blocks of four groups the call's scratch would
+// cost more (29.8 against 29.3 us at 128k).
+__device__ __attribute__((noinline)) int pp_sequential_row_call(const float* md, int T, double canon) {
+    return pp_sequential_row(md, T, canon);
 }
 
 // Row of pick c >= 1 of one segment (one wave; the row to every lane) from the
@@ -1176,7 +1175,8 @@ __device__ int pp_pick_row(const float* md, const PpBlock* st, int nb, int T, do
     emax = wave_emax(emax);
     int logT = 0;
     while ((1ll << logT) < static_cast<long long>(T)) ++logT;
-    if (__builtin_expect(emin != 0x7FFFFFFF && (emax - emin) + 24 + logT > 53, 0)) return pp_sequential_row(md, T, canon);
+    if (__builtin_expect(emin != 0x7FFFFFFF && (emax - emin) + 24 + logT > 53, 0))
+        return RPL == 16 ? pp_sequential_row(md, T, canon) : pp_sequential_row_call(md, T, canon);
     const double total = readlane_f64(wave_incl_scan_f64((sums[0] + sums[1]) + (sums[2] + sums[3])), 63);
     const double target = canon * total + 0.0;
     double base;
