@@ -111,8 +111,9 @@ inline int device_cus() {
     return cached[dev];
 }
 
-// Centroids per subspace of a 2-way or 4-way IMI: the k-means E-step holds
-// k x 64 fp32 rows in LDS (132 KB at 512), the 2-way ranking pipeline scores
+// Centroids per subspace of a 2-way or 4-way IMI: the k-means E-step holds all
+// of a subspace's packed centroids in LDS (4 bytes per dim and 4 each: 130 KB
+// at 512 of 64 dims) and numbers them in 9 bits, the 2-way ranking pipeline scores
 // k * k <= 1024 x 256 cells per head.  512 covers the reference's adaptive k
 // (layer_pipeline.cpp:177-228) up to 4M tokens.
 constexpr int kImiMaxK = 512;

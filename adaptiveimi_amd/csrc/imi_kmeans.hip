@@ -46,7 +46,9 @@ struct KmParams {
     // [seg][nsb][kmax + 1] each superblock's first place of every label, then
     // its token count
     int32_t* loff;
-    int32_t* empties;  // [seg][kmax] ordinal of an empty cluster, -1 otherwise
+    // [seg][kmax] ordinal of an empty cluster, otherwise -1, or -1 minus the size
+    // of a cluster left to a workgroup (kWaveMost)
+    int32_t* empties;
     float* prev;       // [seg][2] inertia of the last tested iteration
     int32_t* done;     // [seg] or null
     int32_t* iters;    // [seg] or null
@@ -195,9 +197,9 @@ __device__ __forceinline__ float l2_lanes8_bf16(const V (&v)[DP / 8], const floa
 // benchmark's keys, since every block of tokens packs the centroids again).
 //
 // Bound by: reading the keys up to k = 64 (64 x 64, 128k tokens, 8 heads: 268
-// MB in 59 us, 4.5 TB/s; a barrier-synchronised form with the label ranks in
+// MB in 60 us, 4.5 TB/s; a barrier-synchronised form with the label ranks in
 // it took 85 us), the three VALU operations and the and-or per value beside
-// the matrix work beyond (k = 181, 512k tokens: 485 us; 4.65 ms as fp32
+// the matrix work beyond (k = 181, 512k tokens: 490 us; 4.65 ms as fp32
 // distances to every centroid; IVF, k = 1018, 16k tokens, 8 heads: 104 us,
 // 1.02 ms as such).
 typedef __attribute__((ext_vector_type(8))) __bf16 km_bf16x8_t;
@@ -1435,10 +1437,10 @@ __global__ __launch_bounds__(256) void km_pp_exact_kernel(KmParams a, PpStep ps)
 // row (lane part j sums dims j, j + 8, .., the reference's lane j; row shifts
 // add the eight sums left to right).  Only the block statistics cross waves.
 //
-// Bound by the copy's bytes (44 per 64-dim row with norm and minima, 76 when
+// Bound by the copy's bytes (44 per 64-dim row with norm and minima, 80 when
 // both halves are read) and the queue's dependent loads for large inputs, by
 // the pick's dependent loads for small ones.  Per pick, 64 dims, 16 segments:
-// 29.5 us at 128k tokens (22 us for the late picks; 33 us with the whole copy
+// 29.6 us at 128k tokens (22 us for the late picks; 33 us with the whole copy
 // read, 55 us reading the keys), 106 us at 512k (146 and 250 us); keys without
 // dominant channels read both halves one after the other, 7 % slower than the
 // whole copy at once.  The next block's loads are issued before the queue (8
@@ -1715,8 +1717,8 @@ __global__ __launch_bounds__(1024) void km_stop_kernel(KmParams a, int it) {
 // first place of each label, then the token count).  The ordered slice goes
 // through LDS (coalesced stores) up to kStagedItems tokens.  11.6 us at 128k
 // tokens, 16 segments; superblocks of thousands of tokens keep the M-step's
-// member search and its column of label offsets short (62 us per M-step, 68 us
-// with one row of offsets per 256 tokens), and serve any T (a scan over
+// member search and its column of label offsets short (58 us per M-step; 62
+// against 68 us with one row of offsets per 256 tokens in an earlier form), and serve any T (a scan over
 // per-block histograms and a scatter took 340 us at 512k tokens, k = 181; this
 // kernel 34 us).
 __host__ __device__ inline size_t members_lds_bytes(int waves, int kmax, int sbt) {
@@ -1822,7 +1824,7 @@ __device__ __forceinline__ int nth_large(const KmParams& a, int seg, int n) {
 // contexts the two launches this saves cost more than the scan: at 11k
 // tokens, k = 32, 4 heads, 11.8 us against 8.3 + 4.8 us (and 3.1 us for a stop
 // test) plus the launches between.
-// Draw = MoreDraws: what km_update_wave_kernel leaves, the n_th cluster of
+// Draw = MoreDraws: what km_update_wave_kernel leaves, the n-th cluster of
 // more than kWaveMost members for workgroup n of the first a.T / (kWaveMost +
 // 1), and behind them the empty clusters past its draws (it: their first
 // ordinal).
