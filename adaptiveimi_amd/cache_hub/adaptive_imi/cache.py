@@ -147,6 +147,7 @@ class adpimi_cache:  # noqa: N801  (reference class name)
         # device (no host synchronisation).
         self.async_build = bool(self.runtime_config["pipeline"].get("async_build", True))
         self._build_stream: Optional[torch.cuda.Stream] = None
+        self._built_on: Dict[torch.device, set] = {}   # streams that hold the builds' workspaces
         self._build_events: List[Optional[torch.cuda.Event]] = [None] * layer_num
         # online index maintenance (cache.py:305-311 defaults)
         acfg = self.runtime_config["async_update"]
@@ -341,6 +342,9 @@ class adpimi_cache:  # noqa: N801  (reference class name)
                     self._build_events[layer_idx] = ev
                 else:
                     self._build_layer_index(layer_idx, mk, mv)
+                if key_states.is_cuda:
+                    self._built_on.setdefault(key_states.device, set()).add(
+                        self._build_stream if self.async_build else torch.cuda.current_stream(key_states.device))
                 self.layer_started[layer_idx] = True
             ss, se = self.static_pattern_start, self.static_pattern_end
             self.steady_zone_keys[layer_idx][start_bdx:end_bdx, :, :ss, :] = (
@@ -408,8 +412,10 @@ class adpimi_cache:  # noqa: N801  (reference class name)
         self.buffer_size = sz["buffer_pages"]
         self.buffer_budget_pages = self.buffer_size
         self.execution_stride = self.buffer_size * self.page_size + self.static_capacity   # runtime.py:62
-        for dev in {c.device for c in self.centroids if c is not None}:
-            ops.release_build_workspaces(dev, self._build_stream)   # every layer's build is enqueued
+        for dev, streams in self._built_on.items():   # every layer's build is enqueued
+            for stream in streams:
+                ops.release_build_workspaces(dev, stream)
+        self._built_on.clear()
         self.cache_prepared = True
 
     def _update_state(self, layer_idx: int) -> Optional[ops.OnlineUpdate]:

@@ -39,13 +39,15 @@ def test_kmeans_with_the_least_workspace(H, T, ks):
         assert all(torch.equal(cent[:, p, :k], ref[0][:, p, :k]) for p, k in enumerate(ks))
 
 
-@pytest.mark.parametrize("side", [True, False])
-def test_cache_gives_the_build_workspaces_back(monkeypatch, side):
-    """Large ones, of the stream that built; the next prefill makes them anew."""
+@pytest.mark.parametrize("side,other", [(True, False), (False, False), (False, True)])
+def test_cache_gives_the_build_workspaces_back(monkeypatch, side, other):
+    """Large ones, of the stream that built (the cache's own, the caller's, or
+    one that the caller left before it prepares the cache); the next prefill
+    makes them anew."""
     from adaptiveimi_amd import ops, synthetic
     from adaptiveimi_amd.cache_hub.adaptive_imi import adpimi_cache
 
-    print(f"[workspaces] side={side}", flush=True)
+    print(f"[workspaces] side={side} other={other}", flush=True)
     H, S, L = 2, 1500, 2
     layers = [[x.transpose(0, 1).unsqueeze(0).contiguous().to(DEV) for x in synthetic.make_kv(H, S, seed=i)] for i in range(L)]
     results = []
@@ -55,9 +57,14 @@ def test_cache_gives_the_build_workspaces_back(monkeypatch, side):
                              2, 0.1, 0.05, 32, 1, 1, 8, subspace_parts=2,
                              runtime_config=dict(pipeline=dict(async_build=side)))
         ops.workspace("attention", 256, torch.device(DEV))
-        for i, (k, v) in enumerate(layers):
-            cache.prefill_update_kv_cache(None, k, v, i, 0)
-        stream = cache._build_stream if side else torch.cuda.current_stream()
+        main = torch.cuda.current_stream()
+        caller = torch.cuda.Stream() if other else main
+        caller.wait_stream(main)
+        with torch.cuda.stream(caller):
+            for i, (k, v) in enumerate(layers):
+                cache.prefill_update_kv_cache(None, k, v, i, 0)
+        main.wait_stream(caller)
+        stream = cache._build_stream if side else caller
         mine = {(n, stream.cuda_stream) for n in ("kmeans", "index")}
         others = {k for k in ops._WS if (k[0], k[2]) not in mine}
         assert mine <= {(n, s) for n, _, s in ops._WS}
