@@ -403,7 +403,7 @@ __device__ __forceinline__ void nearest_of_all(const uint16_t* row, const float*
         load_spread<DP>(cg + static_cast<int64_t>(min(c + 1, k - 1)) * DP, q, next);
         __builtin_amdgcn_sched_barrier(0);   // above the chains, its wait below them
         const float d = l2_lanes8_spread<DP>(x, cv, std::make_integer_sequence<int, DP>{});
-        // (a load of this round, not of the next one's values)
+        // (loaded here, not where the next step uses the values)
 #pragma unroll
         for (int e = 0; e < DP / 16; ++e) asm volatile("" : "+v"(next[e]));
         if (d < best) {
